@@ -84,6 +84,8 @@ struct bromoc_ctx {
     double4 *spos[2] = {nullptr, nullptr};  // the same, in spatial order
     SortBufs sb{};
     bool sort_dirty = true;
+    int sort_tile = 0;                      // spos is in tile order, targets per lane (0: not)
+    int truns = 1;                          // classes and ion types that begin a tile
     int since_sort = 0;
     double r2near = 0.0;
     int cur = 0;
@@ -456,15 +458,15 @@ StepParams params_for(bromoc_ctx *c) {
     p.sposo = c->spos[c->cur ^ 1];
     p.tpb = c->tpb > 0 ? c->tpb : 4;
     if (tile_mode(p.tpb)) {
-        const int tt = 64 * (p.tpb - TPB_TILE);
         p.ttpl = p.tpb - TPB_TILE;
-        p.ntile = (p.ntot + tt - 1) / tt;
-        p.titems = p.ntile * (p.ntile + 1) / 2;
-        p.tnc = p.rfon ? 5 : 3;
+        p.ntile = tile_count(p.ntot, p.ttpl, c->truns);
+        p.trun = tile_run(p.ntile);
+        p.titems = tile_items(p.ntile);
         p.tpart = c->tpart;
         p.tener = c->tener;
-        // one word per tile pair after the energies: its reaction-field sums were written
+        // one word per 64 slots of a row after the energies: its A and B were written
         p.tflag = reinterpret_cast<int32_t *>(c->tener + (size_t)NTE * p.titems);
+        p.rank = c->sb.trank;
     }
     return p;
 }
@@ -474,8 +476,8 @@ StepParams params_for(bromoc_ctx *c) {
 // TILE_MAX_BYTES.
 constexpr size_t TILE_MAX_BYTES = size_t(3) << 30;
 int ensure_tiles(bromoc_ctx *c, int ttpl) {
-    const size_t np = tile_part_doubles(c->cap, ttpl, c->base.rfon);
-    const size_t ne = tile_ener_doubles(c->cap, ttpl);
+    const size_t np = tile_part_doubles(c->cap, ttpl, c->truns, c->base.rfon);
+    const size_t ne = tile_ener_doubles(c->cap, ttpl, c->truns);
     if (8 * (np + ne) > TILE_MAX_BYTES)
         return fail(c, BROMOC_E_CAPACITY, "tile buffers beyond their limit");
     if (np > c->tpart_n) {
@@ -501,14 +503,24 @@ bool tiles_allowed(const bromoc_ctx *c) {
     return !(c->base.dmode == 3 && c->ns > 0);
 }
 
-// Re-sort the partner array when positions were replaced or after GRAPH_K steps.
-int ensure_sorted(bromoc_ctx *c, bool force = false) {
-    if (!force && !c->sort_dirty && c->since_sort < GRAPH_K) return BROMOC_OK;
+// Re-sort the partner array when positions were replaced, after GRAPH_K steps, or when it
+// is in another order: the spatial order (tiles 0), or tile mode's for tiles of 64 * tiles.
+int ensure_sorted(bromoc_ctx *c, bool force, int tiles) {
+    if (!force && !c->sort_dirty && c->since_sort < GRAPH_K && c->sort_tile == tiles) return BROMOC_OK;
     HIPCHK(c, sort_partners(c->sb, c->pos[c->cur], c->ntot, c->spos[c->cur], c->spos[c->cur ^ 1],
                             c->stream));
+    if (tiles > 0)
+        HIPCHK(c, sort_tiles(c->sb, c->pos[c->cur], c->ntot, 64 * tiles,
+                             64 * tiles * tile_count(c->ntot, tiles, c->truns), c->spos[c->cur],
+                             c->spos[c->cur ^ 1], c->stream));
+    c->sort_tile = tiles;
     c->sort_dirty = false;
     c->since_sort = 0;
     return BROMOC_OK;
+}
+
+int ensure_sorted(bromoc_ctx *c, bool force = false) {
+    return ensure_sorted(c, force, tile_mode(c->tpb) ? c->tpb - TPB_TILE : 0);
 }
 
 // Pinned host staging for a call's small copies (the step loop's control words, GRAND's
@@ -631,7 +643,20 @@ int bromoc_create(const bromoc_system *s, int device, bromoc_ctx **out) {
         for (int i = 0; i < s->ntot; i++) p4[i] = make_double4(s->x[i], s->y[i], s->z[i], pack_type(t2[i], i));
         for (int b = 0; b < 2; b++) ACHK(dupload(c, &c->pos[b], p4.data(), cap));
     }
-    for (int b = 0; b < 2; b++) ACHK(dalloc(c, &c->spos[b], cap));
+    // tile mode's order has empty slots at the end of each run: at most a tile less one each
+    for (int b = 0; b < 2; b++) ACHK(dalloc(c, &c->spos[b], (size_t)cap + TILE_MAX_RUNS * 256));
+    {
+        std::vector<char> seen(MAX_LDS_TYPES + 1, 0);
+        auto run_of = [&](int t2v) {
+            t2v = std::min(std::max(t2v, 0), MAX_LDS_TYPES);
+            c->truns += seen[t2v] ? 0 : 1;
+            seen[t2v] = 1;
+        };
+        c->truns = s->nfix > 0 ? 1 : 0;
+        for (int i = 0; i < ns; i++) run_of(s->typtyp[i]);
+        for (int t = s->nold + 1; t <= s->ntype; t++) run_of(s->nwtype[t]);
+        c->truns = std::max(c->truns, 1);
+    }
     ACHK(dalloc(c, &c->sb.keys, cap));
     ACHK(dalloc(c, &c->sb.keys_out, cap));
     ACHK(dalloc(c, &c->sb.vals, cap));
@@ -641,6 +666,8 @@ int bromoc_create(const bromoc_system *s, int device, bromoc_ctx **out) {
     ACHK(dalloc(c, &c->sb.cflag, cap));
     ACHK(dalloc(c, &c->sb.cell_start, (size_t)cap + 1));
     ACHK(dalloc(c, &c->sb.ncell, 1));
+    ACHK(dalloc(c, &c->sb.torder, cap));
+    ACHK(dalloc(c, &c->sb.trank, cap));
     {
         // Morton cells of 8 A over the box (10 bits per axis)
         SortGeom &g = c->sb.geom;
@@ -669,7 +696,7 @@ int bromoc_create(const bromoc_system *s, int device, bromoc_ctx **out) {
     ACHK(dalloc(c, &c->fz, cap));
     ACHK(dalloc(c, &c->fdna, std::max(ns, 1)));
     ACHK(dalloc(c, &c->epart, (size_t)NE * cap));
-    ACHK(dalloc(c, &c->ered, (size_t)NE * (1 + RED_BLOCKS)));
+    ACHK(dalloc(c, &c->ered, (size_t)NE * (1 + 2 * RED_BLOCKS)));
     ACHK(dupload(c, &c->pairidx, s->pairidx, (size_t)nt1 * nt1));
     c->h_pairs.assign(s->pairs, s->pairs + s->npair + 1);
     c->h_pairidx.assign(s->pairidx, s->pairidx + (size_t)nt1 * nt1);
@@ -1174,8 +1201,8 @@ static int autotune(bromoc_ctx *c) {
     std::vector<int> cand = {1, 2, 4, 8};
     if (tiles_allowed(c)) {
         for (int t : {1, 2, 4}) {
-            const size_t bytes = 8 * (tile_part_doubles(c->cap, t, c->base.rfon) +
-                                      tile_ener_doubles(c->cap, t));
+            const size_t bytes = 8 * (tile_part_doubles(c->cap, t, c->truns, c->base.rfon) +
+                                      tile_ener_doubles(c->cap, t, c->truns));
             // a tile must hold enough slots for the shape to be worth timing, and the
             // partial sums must stay within their limit
             if (bytes <= TILE_MAX_BYTES && c->ntot >= 64 * t * 4 && ensure_tiles(c, t) == BROMOC_OK)
@@ -1192,8 +1219,10 @@ static int autotune(bromoc_ctx *c) {
     for (int round = 0; round < 3; round++) {
         for (int q = 0; q < nc; q++) {
             c->tpb = cand[q];
+            sst = ensure_sorted(c);   // the shape's own partner order
             StepParams p = params_for(c);
             c->tpb = 0;
+            if (sst) return sst;
             p.mode = 0;
             p.write_energy = 0;
             p.write_forces = 0;
@@ -2303,6 +2332,7 @@ struct AdjRun {
         // pick: every pass, and every context of the same system, replays the trajectory
         // bitwise
         p.tpb = 2;
+        p.rank = c->sb.rank;
         p.mode = 1;
         p.write_energy = 0;
         p.write_forces = 0;
@@ -2320,7 +2350,7 @@ struct AdjRun {
         if (s % K == 0) {
             HIPCHK(c, hipMemcpyAsync(ckpt + (size_t)(s / K) * nt, c->pos[c->cur],
                                      sizeof(double4) * (size_t)nt, hipMemcpyDeviceToDevice, c->stream));
-            int sst = ensure_sorted(c, true);
+            int sst = ensure_sorted(c, true, 0);
             if (sst) return sst;
         }
         HIPCHK(c, launch_step(step_params(s), c->stream));
@@ -2430,7 +2460,7 @@ int bromoc_adjoint_rdf(bromoc_ctx *c, int32_t nsteps, int32_t K, const bromoc_rd
         for (int seg = R.nseg - 1; seg >= 0; seg--) {
             const int s0 = seg * K, s1 = std::min(s0 + K, nsteps);
             HIPCHK(c, hipMemcpyAsync(c->pos[c->cur], R.ckpt + (size_t)seg * nt, v4, hipMemcpyDeviceToDevice, c->stream));
-            int sst = ensure_sorted(c, true);
+            int sst = ensure_sorted(c, true, 0);
             if (sst) return sst;
             for (int s = s0; s < s1; s++) {
                 HIPCHK(c, hipMemcpyAsync(traj + (size_t)(s - s0) * nt, c->pos[c->cur], v4, hipMemcpyDeviceToDevice, c->stream));
@@ -2531,7 +2561,7 @@ int bromoc_tangent_rdf(bromoc_ctx *c, int32_t nsteps, int32_t K, const bromoc_rd
     for (int s = 0; s < nsteps; s++) {
         // the tangent of step s at x_s, before the step moves the positions
         if (s % K == 0) {      // the checkpoint's sort, as the forward pass makes it
-            int sst = ensure_sorted(c, true);
+            int sst = ensure_sorted(c, true, 0);
             if (sst) return sst;
         }
         A.x = c->pos[c->cur];

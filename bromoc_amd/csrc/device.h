@@ -38,6 +38,42 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
+// Lane moves within the wavefront by DPP: no LDS crossbar, two moves per double.  A lane
+// without a source keeps `old`.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp(double old, double v) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+constexpr int DPP_SHR1 = 0x111, DPP_SHR2 = 0x112, DPP_SHR4 = 0x114, DPP_SHR8 = 0x118;   // in a row of 16
+constexpr int DPP_BCAST15 = 0x142, DPP_BCAST31 = 0x143;   // a row's last lane to the next row(s)
+constexpr int DPP_WAVE_ROL1 = 0x134;                      // lane l takes lane l + 1's (mod 64)
+__device__ __forceinline__ double wave_next(double v) { return dpp<DPP_WAVE_ROL1>(v, v); }
+__device__ __forceinline__ uint32_t wave_next(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, DPP_WAVE_ROL1, 0xf, 0xf, false);
+}
+// lane 63's value on every lane
+__device__ __forceinline__ double wave_last(double v) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), WAVE - 1),
+                            __builtin_amdgcn_readlane(__double2loint(v), WAVE - 1));
+}
+// a value that is the same on every lane, in scalar registers
+__device__ __forceinline__ double wave_uniform(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+__device__ __forceinline__ double wave_min(double v) {
+    v = fmin(v, dpp<DPP_SHR1>(v, v));
+    v = fmin(v, dpp<DPP_SHR2>(v, v));
+    v = fmin(v, dpp<DPP_SHR4>(v, v));
+    v = fmin(v, dpp<DPP_SHR8>(v, v));
+    v = fmin(v, dpp<DPP_BCAST15, 0xa>(v, v));
+    v = fmin(v, dpp<DPP_BCAST31, 0xc>(v, v));
+    return wave_last(v);
+}
+__device__ __forceinline__ double wave_max(double v) { return -wave_min(-v); }
+
 // Order-independent sums of doubles: a term v is cut at the 2^-32 grid into an integer part
 // floor(v 2^32) and W - 1 further 32-bit digits below it (units 2^-64, 2^-96), each added
 // with an integer atomic; integer addition is associative, so the total is the same
@@ -947,6 +983,45 @@ __device__ __forceinline__ const double *noise_row(const StepParams &P, int i) {
     return P.noise + row * P.noise_stride + 3 * (int64_t)i;
 }
 
+// squared distance, the same bits wherever a pair is met and in whichever order
+__device__ __forceinline__ double pair_d2(double dx, double dy, double dz) {
+    return fma(dz, dz, fma(dy, dy, dx * dx));
+}
+
+// sqrt(d2), correctly rounded, from rinv = 1/sqrt(d2) to a few ulp: the residual of the
+// product, exact by fma, corrects it twice (the first leaves it within an ulp, the second
+// rounds the exact root, to which no double is a tie).  Zero and infinity come out as NaN.
+__device__ __forceinline__ double root_of(double d2, double rinv) {
+    const double h = 0.5 * rinv;
+    double x = d2 * rinv;
+    x = fma(fma(-x, x, d2), h, x);
+    return fma(fma(-x, x, d2), h, x);
+}
+
+// The wall of a table pair, below its table's range.
+__device__ __forceinline__ double pair_wall(const DevPair &pp, double rinv, double &y) {
+    const double ix2 = rinv * rinv;
+    const double cw = pp.sc1 * pow6(ix2);
+    y = cw + pp.sc2;
+    return 12.0 * cw * ix2;
+}
+
+// The wall or tabulated quadratic of a table pair within its range (getyd,
+// polynom.f90:197-230), given rinv = 1/sqrt(d2): energy y, returns the force factor.
+__device__ __forceinline__ double pair_table(const DevPair &pp, const double4 *__restrict__ ep,
+                                             double ires, double d2, double rinv, double &y) {
+    if (d2 < pp.dm2lo) return pair_wall(pp, rinv, y);
+    // the knot index from the correctly rounded root, as getyd forms it
+    // (polynom.f90:225-226): 1/sqrt is within an ulp only, and one ulp at a knot
+    // selects the neighbouring segment, where the table jumps by ~1e-9
+    const double x = sqrt(d2);
+    int k = (int)((x - pp.dmi) * ires) + pp.nxi;
+    k = min(max(k, pp.nxi), pp.nlast);
+    const double4 e = ep[k];
+    y = e.x + x * (e.y + x * e.z);
+    return -e.y * rinv - 2.0 * e.z;
+}
+
 // Table pair (getyd, polynom.f90:197-230) in tail-first form: every lane forms the
 // analytic tail sc3/r^6 + fct/r from rinv = 1/sqrt(d2); only lanes inside the table range
 // (d2 <= dm2hi) enter the branch that replaces it with the wall or the tabulated quadratic,
@@ -962,23 +1037,7 @@ __device__ __forceinline__ double pair_near_far(const DevPair &pp, const double4
     const double f = tl.y * rinv;
     y = c + f;
     double de = (6.0 * c + f) * ix2;
-    if (d2 <= tl.z) {
-        if (d2 < pp.dm2lo) {
-            const double cw = pp.sc1 * pow6(ix2);
-            y = cw + pp.sc2;
-            de = 12.0 * cw * ix2;
-        } else {
-            // the knot index from the correctly rounded root, as getyd forms it
-            // (polynom.f90:225-226): 1/sqrt is within an ulp only, and one ulp at a knot
-            // selects the neighbouring segment, where the table jumps by ~1e-9
-            const double x = sqrt(d2);
-            int k = (int)((x - pp.dmi) * ires) + pp.nxi;
-            k = min(max(k, pp.nxi), pp.nlast);
-            const double4 e = ep[k];
-            y = e.x + x * (e.y + x * e.z);
-            de = -e.y * rinv - 2.0 * e.z;
-        }
-    }
+    if (d2 <= tl.z) de = pair_table(pp, ep, ires, d2, rinv, y);
     return de;
 }
 

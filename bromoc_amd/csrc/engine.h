@@ -248,18 +248,31 @@ struct StepParams {
     double *mleg;            // [cap+1][npl] P_0.. of x, y, z scaled (zeros outside the region)
     double *mchg;            // [cap+1] charge of each moving ion inside the region, else 0
     double *mcoef, *mq, *mer;   // [ntpol] coefficients, M q rfscal, per-row energy terms
-    // tile mode (tiles.hip): tiles of 64 * ttpl consecutive slots of the spatial order;
-    // tpart[((K * ntile + I) * tnc + c) * TT + t]: component c (fx, fy, fz, and with the
-    // fused reaction field A, B) of slot t of tile I from the tile pair of I and K, each
-    // entry written once per step; tener[cat][item]: pair energies of each tile pair
+    // tile mode (tiles.hip): tiles of TT = 64 * ttpl consecutive slots of the tile order, in
+    // column groups of trun tiles; tile I's rows of partial sums are rows tile_row(I).. of
+    // tpart[(row * tnc + c) * TT + t]: component c (fx, fy, fz, and with the fused reaction
+    // field A, B) of slot t, first one row per lower tile, then one per group from I's own;
+    // tener[cat][item]: pair energies of each item (a tile and a group)
     double *tpart, *tener;
-    int32_t *tflag;          // [titems] 1 where a tile pair wrote its reaction-field rows
-    int32_t ntile, ttpl, tnc, titems;
+    int32_t *tflag;          // [row][ttpl] 1 where a row's 64 slots hold A and B too
+    int32_t ntile, ttpl, trun, titems;
 };
 
 // tpb values of tile mode: TPB_TILE + targets per lane (1, 2 or 4)
 constexpr int TPB_TILE = 16;
-constexpr int TILE_WAVES = 2;      // wavefronts of a k_tiles block (tile pairs sharing tile J)
+// items wanted of a grouping (tile_run): four rounds of the chip's 4,096 resident wavefronts
+constexpr int TILE_MIN_ITEMS = 16384;
+int tile_run(int n);               // tiles per column group of n tiles
+// tiles that hold n particles in `runs` runs (fixed ions, each type), each beginning a tile (an
+// upper bound: the runs' sizes are known on the device only)
+int tile_count(int n, int ttpl, int runs);
+int tile_items(int n);
+// rows of partial sums of the tiles before T, of n tiles in groups of R: t + (groups from
+// t's own) for each tile t
+__host__ __device__ inline int64_t tile_row(int64_t T, int64_t n, int64_t R) {
+    const int64_t q = T / R, r = T - q * R;
+    return T * (T - 1) / 2 + T * ((n + R - 1) / R) - (R * (q * (q - 1) / 2) + r * q);
+}
 __host__ __device__ inline bool tile_mode(int tpb) { return tpb > TPB_TILE; }
 
 // pair-energy categories of the tile kernel (tener rows) and the ECat each one feeds
@@ -282,10 +295,15 @@ struct SortBufs {
     int32_t *cflag;                // [cap] cell numbers (exclusive scan of the key changes)
     int32_t *cell_start;           // [cap+1] first slot of each occupied cell, then n
     int32_t *ncell;                // [1] occupied cells
+    int32_t *trank, *torder;       // [cap] the tile order and its inverse (tile mode)
 };
 size_t sort_hist_ints(int n);
 hipError_t sort_partners(const SortBufs &b, const double4 *pos, int n, double4 *spos0,
                          double4 *spos1, hipStream_t s);
+// tile mode: after sort_partners, spos regrouped stably (fixed ions, then by type), each run
+// from a multiple of tt slots on, over nslot slots (torder, trank)
+hipError_t sort_tiles(const SortBufs &b, const double4 *pos, int n, int tt, int nslot,
+                      double4 *spos0, double4 *spos1, hipStream_t s);
 
 // launchers (kernels.hip)
 hipError_t launch_step(const StepParams &p, hipStream_t s);   // launch_dna + launch_pairs
@@ -303,16 +321,17 @@ hipError_t launch_mmij_interact(const StepParams &p, double xj, double yj, doubl
                                 int j, double *out, hipStream_t s);
 // out[cat] = sum over particles of epart[cat], plus for the pair categories the sum over
 // the tile pairs of tener (tile mode), both in a fixed order; out holds NE * (1 +
-// RED_BLOCKS) doubles (the range sums follow the NE results)
+// 2 * RED_BLOCKS) doubles (the range sums and their errors follow the NE results)
 hipError_t launch_reduce_energy(const double *epart, int ecap, int n, double *out,
                                 hipStream_t s, const double *tener = nullptr, int titems = 0);
 // tile mode (tiles.hip): k_tiles over every tile pair (which & 1), then k_tfin over every
 // slot (which & 2)
 hipError_t launch_tiles(const StepParams &p, hipStream_t s, int which = 3);
-// device bytes of the tile buffers for `cap` particles at ttpl targets per lane (fused
+// doubles of the tile buffers for up to `cap` particles at ttpl targets per lane (fused
 // reaction field: rf != 0)
-size_t tile_part_doubles(int cap, int ttpl, int rf);
-size_t tile_ener_doubles(int cap, int ttpl);
+size_t tile_part_doubles(int cap, int ttpl, int runs, int rf);
+size_t tile_ener_doubles(int cap, int ttpl, int runs);
+constexpr int TILE_MAX_RUNS = MAX_LDS_TYPES;   // fixed ions (0), then the atnam2 types
 hipError_t launch_advance(int64_t *ctr, int64_t by, hipStream_t s);
 hipError_t launch_philox_fill(const int64_t *ctl, uint64_t stream, int nrows, int ntot,
                               int64_t stride, double *out, hipStream_t s);

@@ -1162,11 +1162,24 @@ __device__ __forceinline__ int tile_cat_of(int cat) {
 // energies (tile mode), as one sequence cut into RED_BLOCKS contiguous ranges; block b
 // sums range b (four interleaved accumulators per thread, so loads overlap, then a tree),
 // and k_reduce_finish adds the RED_BLOCKS range sums in order.  Fixed shapes throughout:
-// the same inputs give the same bits.
+// the same inputs give the same bits.  The sums carry their rounding errors along (two_sum):
+// tile mode's items hold pairs of one type pair, so their energies are large and of both
+// signs (10^6 against a total of 3 10^3 kcal/mol at 6000 ions), and plain sums lost a digit.
+struct Sum2 { double s, c; };   // sum and its accumulated error
+__device__ __forceinline__ void sum2_add(Sum2 &a, double v) {
+    const double t = a.s + v, b = t - a.s;
+    a.c += (a.s - (t - b)) + (v - b);
+    a.s = t;
+}
+__device__ __forceinline__ void sum2_add(Sum2 &a, const Sum2 &b) {
+    sum2_add(a, b.s);
+    a.c += b.c;
+}
+
 __global__ __launch_bounds__(BLOCK) void k_reduce_energy(const double *epart, int ecap, int n,
-                                                         double *part, const double *tener,
+                                                         Sum2 *part, const double *tener,
                                                          int titems) {
-    __shared__ double s[BLOCK];
+    __shared__ Sum2 s[BLOCK];
     const int cat = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     const double *src = epart + (size_t)cat * ecap;
     const int tc = tener ? tile_cat_of(cat) : -1;
@@ -1175,38 +1188,46 @@ __global__ __launch_bounds__(BLOCK) void k_reduce_energy(const double *epart, in
     const int chunk = (m + RED_BLOCKS - 1) / RED_BLOCKS;
     const int lo = b * chunk, hi = min(lo + chunk, m);
     auto val = [&](int k) { return k < n ? src[k] : tsrc[k - n]; };
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+    Sum2 a[4] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
     int k = lo + tid;
     for (; k + 3 * BLOCK < hi; k += 4 * BLOCK) {
-        a0 += val(k);
-        a1 += val(k + BLOCK);
-        a2 += val(k + 2 * BLOCK);
-        a3 += val(k + 3 * BLOCK);
+        double v[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = val(k + q * BLOCK);
+#pragma unroll
+        for (int q = 0; q < 4; q++) sum2_add(a[q], v[q]);
     }
-    for (; k < hi; k += BLOCK) a0 += val(k);
-    s[tid] = (a0 + a1) + (a2 + a3);
+    for (; k < hi; k += BLOCK) sum2_add(a[0], val(k));
+#pragma unroll
+    for (int q = 1; q < 4; q++) sum2_add(a[0], a[q]);
+    s[tid] = a[0];
     __syncthreads();
     for (int h = BLOCK / 2; h > 0; h >>= 1) {
-        if (tid < h) s[tid] += s[tid + h];
+        if (tid < h) {
+            Sum2 x = s[tid];
+            sum2_add(x, s[tid + h]);
+            s[tid] = x;
+        }
         __syncthreads();
     }
     if (tid == 0) part[(size_t)cat * RED_BLOCKS + b] = s[0];
 }
 
-__global__ void k_reduce_finish(const double *part, double *out) {
+__global__ void k_reduce_finish(const Sum2 *part, double *out) {
     const int cat = threadIdx.x;
     if (cat >= NE) return;
-    double acc = 0.0;
-    for (int b = 0; b < RED_BLOCKS; b++) acc += part[(size_t)cat * RED_BLOCKS + b];
-    out[cat] = acc;
+    Sum2 acc = {0.0, 0.0};
+    for (int b = 0; b < RED_BLOCKS; b++) sum2_add(acc, part[(size_t)cat * RED_BLOCKS + b]);
+    out[cat] = isfinite(acc.s) ? acc.s + acc.c : acc.s;   // the error of an infinite sum is not a number
 }
 
 hipError_t launch_reduce_energy(const double *epart, int ecap, int n, double *out,
                                 hipStream_t s, const double *tener, int titems) {
-    double *part = out + NE;   // the caller's buffer holds NE * (1 + RED_BLOCKS) doubles
+    // the caller's buffer holds NE * (1 + 2 * RED_BLOCKS) doubles
+    Sum2 *part = reinterpret_cast<Sum2 *>(out + NE);
     hipLaunchKernelGGL(k_reduce_energy, dim3(NE, RED_BLOCKS), dim3(BLOCK), 0, s, epart, ecap, n,
                        part, tener, titems);
-    hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(64), 0, s, (const double *)part, out);
+    hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(64), 0, s, (const Sum2 *)part, out);
     return hipGetLastError();
 }
 

@@ -410,4 +410,63 @@ hipError_t sort_partners(const SortBufs &b, const double4 *pos, int n, double4 *
     return hipGetLastError();
 }
 
+// key of slot k of the spatial order in the tile order: fixed ion 0, else the atnam2 type (sites
+// and ions have types of their own, sites the lower ones)
+__global__ void k_type_keys(const double4 *__restrict__ spos, int n, SortGeom g, uint32_t *keys) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const double w = spos[k].w;
+    const int i = __double2hiint(w), t = __double2loint(w);
+    keys[k] = i >= g.nsites && i < g.nsites + g.nfix ? 0u : (uint32_t)t;
+}
+
+// spos over the padded slots: run t of the tile order (its first particle at hist[t * nb],
+// the scanned histogram) begins at the next multiple of tt after the run before it; slots
+// past a run's last particle are empty (index -1, at the middle of the box)
+__global__ void k_tile_gather(const double4 *__restrict__ pos, const int32_t *__restrict__ order,
+                              const int32_t *__restrict__ hist, int nb, int n, int tt, int nslot,
+                              SortGeom g, double4 *spos0, double4 *spos1, int32_t *rank) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nslot) return;
+    int at = 0, src = -1;   // first slot of the run; the slot's place in the tile order
+    for (int t = 0; t < TILE_MAX_RUNS; t++) {
+        const int lo = hist[t * nb], hi = hist[(t + 1) * nb], c = hi - lo;
+        if (s >= at && s < at + c) src = lo + (s - at);
+        at += (c + tt - 1) / tt * tt;
+    }
+    double4 p;
+    if (src >= 0) {
+        const int j = order[src];
+        p = pos[j];
+        rank[j] = s;
+    } else {
+        p = make_double4(g.lo[0] + 0.5 * g.n[0] / g.inv, g.lo[1] + 0.5 * g.n[1] / g.inv,
+                         g.lo[2] + 0.5 * g.n[2] / g.inv, __hiloint2double(-1, 0));
+    }
+    spos0[s] = p;
+    spos1[s] = p;
+}
+
+// The tile order: the spatial order regrouped by type (less than MAX_LDS_TYPES of them),
+// the fixed ions first, stably, so that a tile's particles are of one type and near each
+// other.  One more radix pass over the sorted slots; order, rank and cell_start stay those of the
+// spatial order.
+hipError_t sort_tiles(const SortBufs &b, const double4 *pos, int n, int tt, int nslot,
+                      double4 *spos0, double4 *spos1, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    const int blk = 256, grid = (n + blk - 1) / blk;
+    const int nb = sort_blocks(n), chunk = (n + nb - 1) / nb;
+    // keys and vals are free once the spatial order is in keys_out and order
+    uint32_t *unused = reinterpret_cast<uint32_t *>(b.vals);
+    hipLaunchKernelGGL(k_type_keys, dim3(grid), dim3(blk), 0, s, (const double4 *)spos0, n, b.geom, b.keys);
+    hipLaunchKernelGGL(k_digit_hist, dim3(nb), dim3(SORT_BLOCK), 0, s, b.keys, n, chunk, 0, b.hist);
+    hipLaunchKernelGGL(k_scan_excl, dim3(1), dim3(SCAN_BLOCK), 0, s, b.hist, SORT_RADIX * nb,
+                       (int32_t *)nullptr);
+    hipLaunchKernelGGL(k_digit_scatter, dim3(nb), dim3(SORT_BLOCK), 0, s, b.keys, b.order, unused,
+                       b.torder, n, chunk, 0, b.hist);
+    hipLaunchKernelGGL(k_tile_gather, dim3((nslot + blk - 1) / blk), dim3(blk), 0, s, pos, b.torder,
+                       b.hist, nb, n, tt, nslot, b.geom, spos0, spos1, b.trank);
+    return hipGetLastError();
+}
+
 }  // namespace bromoc

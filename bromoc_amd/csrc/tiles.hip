@@ -6,28 +6,41 @@
 // gathers instead, every target over all partners, which costs every pair twice.  Tile
 // mode keeps the reference's once-per-pair work and stays deterministic:
 //
-//  * the particles in spatial order (spos) are cut into tiles of TT = 64 * TPL slots;
-//  * k_tiles: one wavefront per tile pair (I, J), I <= J, two per workgroup on the same
-//    column J, which share tile J's partner data in LDS.  Lane l holds the TPL targets
-//    l, l + 64, .. of tile I in registers; tile J's partners sit in LDS.  At step k every
-//    lane takes a different partner (a rotation, so no two lanes touch one partner at
-//    once), evaluates it against its TPL targets, adds the targets' shares in registers
-//    and the partner's share into the partner's LDS accumulator.  Each pair's reaction-
-//    field cross term (when the system has one) is evaluated in the same sweep.  At the
-//    end the wavefront writes tile I's sums to tpart[J][I] and tile J's to tpart[I][J]
-//    (a diagonal tile pair writes their sum once): every entry of tpart is written exactly
-//    once per step, and the pair energies go to tener[cat][item];
-//  * the sweep a wavefront runs depends on what its two tiles hold (the sort puts CG-DNA
-//    sites, fixed ions and moving ions in separate runs, so most tiles hold one class):
-//    two tiles of moving ions off the diagonal need no per-pair masks, and their
-//    reaction-field term, when every ion of both tiles is either inside the grid with a
-//    nonzero srfe or outside it with none, reduces to per-ion weights folded into the
-//    charges (or vanishes, when one tile has no ion inside); a tile of sites against a tile
-//    of moving ions is all site-ion pairs with no reaction field; tiles of sites and fixed
-//    ions only have no pair to evaluate.  Everything else takes the masked sweep;
-//  * k_tfin: eight lanes per slot sum the slot's ntile partial rows in a fixed order,
+//  * the particles in tile order (sort.hip: fixed ions, then by atnam2 type, then space) are
+//    cut into tiles of TT = 64 * TPL slots; each type begins a new tile, so a tile holds
+//    fixed ions, sites of one type or moving ions of one type, and empty slots at the end
+//    of a run;
+//  * k_tiles: one wavefront per item (I, g): tile I's particles are its targets, TPL per
+//    lane in registers, and the tiles J >= I of column group g (R consecutive tiles) pass by
+//    in chunks of 64 partners.  A chunk's positions are staged in LDS, twice in a row, so
+//    that at step k lane l reads partner l + k without wrapping; every lane takes another
+//    partner, evaluates it against its TPL targets and adds the targets' shares in
+//    registers.  The partners' shares travel: each lane holds the sums of the partner it is
+//    evaluating and hands them to its lower neighbour after the step (DPP wavefront
+//    rotation), so after 64 steps lane l holds partner l's sums -- no LDS accumulators, whose
+//    read-modify-write took as long as the arithmetic.  Each pair's reaction-field cross
+//    term (when the system has one) is evaluated in the same sweep;
+//  * the targets' sums are written once per item, a chunk's partner sums once per (I, J): a
+//    tile's rows of tpart, one per lower tile and one per group of higher ones, each written
+//    once per step; pair energies go to tener[cat][item];
+//  * the sweep a chunk takes depends on what it and the target tile hold.  Against a chunk
+//    of moving ions there is one pair type, its parameters in scalar registers.  When no
+//    partner of the chunk is within table range of the targets' bounding box (97 % of the
+//    chunks at 56,000 particles) the sweep is straight-line code: the analytic tail alone,
+//    no comparison, no table.  In near chunks the
+//    sweep leaves the pairs in range out and notes them, a bit per pair for the target and one
+//    that travels with the partner; then each lane works off its targets' bits and its
+//    partner's, so the table's root, index and gather (three times the tail's arithmetic and a
+//    memory round trip) are paid per pair in range and not per step that has one.  Masks
+//    (the diagonal, empty slots) are a variant of their own.  The reaction-field term, when
+//    every ion of both sides is either inside the grid with a nonzero srfe or outside it
+//    with none, reduces to per-ion weights folded into the charges (or vanishes, when one
+//    side has no ion inside); sites against moving ions have none.  Fixed ions, and ions at
+//    the edge of the reaction-field grid, take the general masked sweep;
+//  * k_tfin: eight lanes per slot sum the slot's partial rows in a fixed order,
 //    gather the grid corners and finish the particle as k_step does (CG-DNA list forces,
 //    reaction-field gradients and self term, MEMBRANE, energies, BD update).
+#include <algorithm>
 #include <type_traits>
 
 #include "device.h"
@@ -42,16 +55,41 @@ constexpr int F_RFT = 64;   // reaction-field cross term fused into the pair swe
 constexpr int SL_VALID = 1, SL_SITE = 2, SL_FIXED = 4, SL_RECV = 8, SL_HI = 16, SL_ION = 32,
               SL_RFON = 64, SL_RFODD = 128;
 
-size_t tile_part_doubles(int cap, int ttpl, int rf) {
-    const size_t tt = 64 * (size_t)ttpl, n = (cap + tt - 1) / tt;
-    return n * n * (rf ? 5 : 3) * tt;
+// Column groups of n tiles: R tiles per group, so that an item's targets (their sums, and
+// the row they write) serve R tiles.  The largest R that still gives the chip several
+// rounds of wavefronts, since the items' lengths differ.
+int tile_run(int n) {
+    for (int r = 8; r > 1; r >>= 1) {
+        const int64_t g = (n + r - 1) / r;
+        if (r * g * (g + 1) / 2 >= TILE_MIN_ITEMS) return r;
+    }
+    return 1;
 }
-size_t tile_ener_doubles(int cap, int ttpl) {
-    const size_t tt = 64 * (size_t)ttpl, n = (cap + tt - 1) / tt;
-    return (size_t)(NTE + 1) * (n * (n + 1) / 2);   // energies, then the tflag words
+int tile_items(int n) {
+    const int r = tile_run(n), g = (n + r - 1) / r;
+    return r * (g * (g + 1) / 2);
 }
 
-// The particle in slot s of the spatial order: position, and a word of atnam2 type and
+int tile_count(int n, int ttpl, int runs) {
+    const int tt = 64 * ttpl;
+    return (int)((n + (int64_t)runs * (tt - 1)) / tt);
+}
+size_t tile_part_doubles(int cap, int ttpl, int runs, int rf) {
+    const size_t tt = 64 * (size_t)ttpl, nc = tile_count(cap, ttpl, runs);
+    size_t rows = 0;   // the run length, and so the rows, follow the tiles now in use
+    for (size_t n = 1; n <= nc; n++) rows = std::max(rows, (size_t)tile_row(n, n, tile_run((int)n)));
+    return rows * (rf ? 5 : 3) * tt;
+}
+size_t tile_ener_doubles(int cap, int ttpl, int runs) {
+    const size_t nc = tile_count(cap, ttpl, runs);
+    size_t m = 0;
+    for (size_t n = 1; n <= nc; n++)   // energies, then the tflag words
+        m = std::max(m, (size_t)NTE * tile_items((int)n) +
+                            ((size_t)tile_row(n, n, tile_run((int)n)) * ttpl + 1) / 2);
+    return m;
+}
+
+// The particle in slot s of the tile order: position, and a word of atnam2 type and
 // flags (the pair kernels' masks); with the reaction field, srfe, reff and the charge.
 struct SlotInfo {
     double x, y, z, sr, rr, q;
@@ -61,11 +99,11 @@ struct SlotInfo {
 template <int FEAT>
 __device__ __forceinline__ SlotInfo slot_info(const StepParams &P, int s) {
     SlotInfo o;
-    const bool ok = s < P.ntot;
-    const double4 pa = P.spos[ok ? s : 0];
-    const int idx = __double2hiint(pa.w), t2 = __double2loint(pa.w);
-    const bool site = idx < P.nsites, fixed = !site && idx < P.nsites + P.nfix;
-    bool recv = !site && !fixed;
+    const double4 pa = P.spos[s];   // an empty slot: index -1, at the box's centre
+    const bool ok = __double2hiint(pa.w) >= 0;
+    const int idx = ok ? __double2hiint(pa.w) : 0, t2 = __double2loint(pa.w);
+    const bool site = ok && idx < P.nsites, fixed = ok && !site && idx < P.nsites + P.nfix;
+    bool recv = ok && !site && !fixed;
     if constexpr ((FEAT & F_DNA) != 0) {
         if (site) recv = P.stfree[idx] != 0;
     }
@@ -75,7 +113,7 @@ __device__ __forceinline__ SlotInfo slot_info(const StepParams &P, int s) {
     o.x = pa.x; o.y = pa.y; o.z = pa.z;
     o.sr = 0.0; o.rr = 0.0; o.q = 0.0;
     if constexpr ((FEAT & F_RFT) != 0) {
-        if (!site) {
+        if (ok && !site) {
             // (srfe, reff, inside the grid box, moving) from k_rfpar; charge in rfq.w
             const double4 ra = P.rfa[idx];
             o.sr = ra.x; o.rr = ra.y;
@@ -107,340 +145,487 @@ __device__ __forceinline__ int wave_or8(int v) {
     return r;
 }
 
-// Blocks of k_tiles: column J of the tile pairs (I, J), I <= J, in pairs of rows -- block
-// c of column J holds the items (2c, J) and (2c + 1, J), one per wavefront, so the two
-// wavefronts share tile J's partner data in LDS.  Column j has j / 2 + 1 blocks; the
-// columns before J have tile_blocks(J) = m (m + 1) for J = 2m and (m + 1)^2 for J = 2m + 1.
-__host__ __device__ __forceinline__ int tile_blocks(int J) {
-    const int m = J >> 1;
-    return (J & 1) ? (m + 1) * (m + 1) : m * (m + 1);
+// item -> (row I, group g): group g holds the rows 0 .. (g + 1) R - 1, groups in order
+__device__ __forceinline__ void item_tiles(int item, int R, int &I, int &g) {
+    const int h = item / R;   // g (g + 1) / 2 <= h
+    int k = (int)((sqrt(8.0 * (double)h + 1.0) - 1.0) * 0.5);
+    while (k > 0 && k * (k + 1) / 2 > h) k--;
+    while ((k + 1) * (k + 2) / 2 <= h) k++;
+    g = k;
+    I = item - R * (k * (k + 1) / 2);
 }
-__device__ __forceinline__ void block_tiles(int b, int &J, int &c) {
-    int j = (int)(2.0 * sqrt((double)b));
-    while (j > 0 && tile_blocks(j) > b) j--;
-    while (tile_blocks(j + 1) <= b) j++;
-    J = j;
-    c = b - tile_blocks(j);
-}
-// LDS row stride of the type-pair tables: even, so that the rows (t, p) and (p, t), which a
-// wavefront reads at once, fall in different banks
-__host__ __device__ __forceinline__ int tail_stride(int nt1) { return nt1 + (nt1 & 1); }
 
-template <int FEAT, int TPL>
-__global__ __launch_bounds__(TILE_WAVES * WAVE) void k_tiles(StepParams P) {
+// a chunk of 64 partners staged by the wavefront, each entry twice (at p and p + 64)
+template <bool RF, int TT>
+struct Chunk {
+    double x[2 * WAVE], y[2 * WAVE], z[2 * WAVE];
+    double tx[TT], ty[TT], tz[TT];   // the targets, for the partners' pairs in range
+    union {
+        struct { double rr[RF ? 2 * WAVE : 1], qs[RF ? 2 * WAVE : 1]; };   // reff; weight * charge * srfe
+        struct {   // the general sweep's: srfe, reff, charge, index
+            double sr[RF ? 2 * WAVE : 1], rg[RF ? 2 * WAVE : 1], q[RF ? 2 * WAVE : 1];
+            int ix[RF ? 2 * WAVE : 1];
+        };
+    };
+    int tf[2 * WAVE];   // type and flags
+};
+
+// wavefronts per SIMD the registers are held to
+constexpr int tile_occ(int feat, int tpl) {
+    return tpl == 4 ? 2 : (feat & F_TAB) == 0 ? 2 : tpl == 1 ? ((feat & F_RFT) ? 4 : 5) : (feat & F_RFT) ? 3 : 4;
+}
+
+// k_tiles: see the file comment.  One wavefront per block: its item ends on its own.  Bound by
+// FP64 issue where the system is large: 27 issue slots a far pair (four of them the reciprocal
+// root's), 24 more with the reaction field, and the rotation's ten moves a step.  Measured, one
+// launch (before, with LDS accumulators, per-pair table parameters and a branch per pair;
+// after): 56,000 particles with the reaction field on every ion pair 3.34 -> 2.56 ms, 12,457
+// particles 237 -> 177 us, 6,001 particles 55 -> 47 us.
+template <int FEAT, int TPL, bool EN>
+__global__ __launch_bounds__(WAVE)
+__attribute__((amdgpu_waves_per_eu(tile_occ(FEAT, TPL))))
+void k_tiles(StepParams P) {
     constexpr int TT = WAVE * TPL;
-    constexpr bool RF = (FEAT & F_RFT) != 0;
-    constexpr int NR = RF ? TT : 1;
-    // tile J's partner data, shared by the block's wavefronts
-    __shared__ double s_x[TT], s_y[TT], s_z[TT];
-    __shared__ int s_tf[TT], s_ix[RF ? TT : 1];
-    __shared__ double s_sr[NR], s_rr[NR], s_q[NR];
-    // each wavefront's partner sums
-    __shared__ double s_afx[TILE_WAVES][TT], s_afy[TILE_WAVES][TT], s_afz[TILE_WAVES][TT];
-    __shared__ double s_afa[TILE_WAVES][NR], s_afb[TILE_WAVES][NR];
-    // by type pair (row stride tail_stride): (sc3, tail fct, dm2hi, flags); the near branch
-    // reads the rest of the pair row from global memory
-    extern __shared__ double4 s_tail[];
+    constexpr bool RF = (FEAT & F_RFT) != 0, TAB = (FEAT & F_TAB) != 0;
+    __shared__ Chunk<RF, TT> C;
 
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid >> 6;
-    const int b = blockIdx.x;
-    const int n = P.ntile, nt1 = P.nttyp + 1, S = tail_stride(nt1);
-    if (b >= tile_blocks(n)) return;
-    int J, cp;
-    block_tiles(b, J, cp);
-    const int I = TILE_WAVES * cp + wv;
-    const bool active = I <= J;
-    const bool diag = I == J;
-    const int item = J * (J + 1) / 2 + I;   // the tile pair's index: (I, J) by columns
-    for (int k = tid; k < nt1 * nt1; k += TILE_WAVES * WAVE) {
-        const DevPair &d = P.rows[k];
-        const int l = (k / nt1) * S + k % nt1;
-        s_tail[l] = make_double4(d.sc3, d.fct, d.dm2hi, (double)d.flags);
-    }
-    double *const s_fx = s_afx[wv], *const s_fy = s_afy[wv], *const s_fz = s_afz[wv];
-    double *const s_fa = s_afa[wv], *const s_fb = s_afb[wv];
-    // partners: tile J into LDS; this wavefront's sums cleared
-    for (int p = tid; p < TT; p += TILE_WAVES * WAVE) {
-        const SlotInfo o = slot_info<FEAT>(P, J * TT + p);
-        s_x[p] = o.x; s_y[p] = o.y; s_z[p] = o.z; s_tf[p] = o.tf;
-        if constexpr (RF) { s_ix[p] = o.idx; s_sr[p] = o.sr; s_rr[p] = o.rr; s_q[p] = o.q; }
-    }
+    const int lane = threadIdx.x, item = blockIdx.x;
+    const int n = P.ntile, nt1 = P.nttyp + 1, R = P.trun;
+    int I, g;
+    item_tiles(item, R, I, g);
+    double en[EN ? NTE : 1];
 #pragma unroll
-    for (int u = 0; u < TPL; u++) {
-        const int p = lane + WAVE * u;
-        s_fx[p] = 0.0; s_fy[p] = 0.0; s_fz[p] = 0.0;
-        if constexpr (RF) { s_fa[p] = 0.0; s_fb[p] = 0.0; }
+    for (int c = 0; c < (EN ? NTE : 1); c++) en[c] = 0.0;
+    if (I >= n) {   // past the last tile of a partial last group
+        if (EN && lane < NTE) P.tener[(size_t)lane * P.titems + item] = 0.0;
+        return;
     }
+    const int NC = RF ? 5 : 3;
+    const int J0 = max(I, g * R), J1 = min((g + 1) * R, n);
     // targets: tile I in registers
     double tx[TPL], ty[TPL], tz[TPL], tsr[TPL], trr[TPL], tq[TPL];
     int ttf[TPL], tix[TPL];
-    double ax_[TPL], ay_[TPL], az_[TPL], aa_[TPL], ab_[TPL];
+    double ax_[TPL], ay_[TPL], az_[TPL], aa_[TPL], ab_[TPL];   // aa_, ab_: general sweep
+    double wa[TPL], wb[TPL], tqs[TPL];   // the weighted sweeps' A and B over their factors
+    int andI = ~0, orI = 0;
 #pragma unroll
     for (int u = 0; u < TPL; u++) {
-        const SlotInfo o = slot_info<FEAT>(P, (active ? I : J) * TT + lane + WAVE * u);
+        const SlotInfo o = slot_info<FEAT>(P, I * TT + lane + WAVE * u);
         tx[u] = o.x; ty[u] = o.y; tz[u] = o.z; ttf[u] = o.tf; tix[u] = o.idx;
         tsr[u] = o.sr; trr[u] = o.rr; tq[u] = o.q;
-        ax_[u] = ay_[u] = az_[u] = aa_[u] = ab_[u] = 0.0;
+        ax_[u] = ay_[u] = az_[u] = aa_[u] = ab_[u] = wa[u] = wb[u] = 0.0;
+        C.tx[lane + WAVE * u] = o.x; C.ty[lane + WAVE * u] = o.y; C.tz[lane + WAVE * u] = o.z;
+        const int f = o.tf >> 16;
+        tqs[u] = (f & SL_RFON) ? P.celec * o.q * o.sr : 0.0;
+        andI &= (f & SL_VALID) ? f : ~SL_VALID;
+        orI |= f;
     }
-    __syncthreads();
-    // the block's last barrier: a wavefront past the column's diagonal has no tile pair
-    if (!active) return;
-
-    double en[NTE];
+    const int t2I = __builtin_amdgcn_readfirstlane(ttf[0] & 0xFFFF);   // a run begins with a particle
+    andI = wave_and8(andI); orI = wave_or8(orI);
+    // the tile's class (every particle's: an empty slot has no say)
+    const bool ionI = (orI & SL_ION) && (andI & SL_ION), siteI = (orI & SL_SITE) && (andI & SL_SITE);
+    // the targets' bounding box
+    double bx0 = tx[0], bx1 = tx[0], by0 = ty[0], by1 = ty[0], bz0 = tz[0], bz1 = tz[0];
 #pragma unroll
-    for (int c = 0; c < NTE; c++) en[c] = 0.0;
+    for (int u = 1; u < TPL; u++) {
+        bx0 = fmin(bx0, tx[u]); bx1 = fmax(bx1, tx[u]);
+        by0 = fmin(by0, ty[u]); by1 = fmax(by1, ty[u]);
+        bz0 = fmin(bz0, tz[u]); bz1 = fmax(bz1, tz[u]);
+    }
+    bx0 = wave_min(bx0); bx1 = wave_max(bx1);
+    by0 = wave_min(by0); by1 = wave_max(by1);
+    bz0 = wave_min(bz0); bz1 = wave_max(bz1);
+    bool rfany = false;   // the targets' reaction-field sums (A, B) may be nonzero
 
-    auto sweep = [&](auto en_on) {
-        constexpr bool EN = decltype(en_on)::value;
-        for (int k = 0; k < TT; k++) {
-            // rotation: at step k the lanes hold 64 different partners, and over the TT
-            // steps every lane meets every partner once
-            const int p = ((lane + k / TPL) & (WAVE - 1)) + WAVE * (k % TPL);
-            const double px = s_x[p], py = s_y[p], pz = s_z[p];
-            const int ptf = s_tf[p];
-            const int t2p = ptf & 0xFFFF, pfl = ptf >> 16;
-            double psr = 0.0, prr = 0.0, pq = 0.0;
-            int pix = 0;
-            if constexpr (RF) { psr = s_sr[p]; prr = s_rr[p]; pq = s_q[p]; pix = s_ix[p]; }
-            double gx = 0.0, gy = 0.0, gz = 0.0;    // pair force on the partner (negated)
-            double rx = 0.0, ry = 0.0, rz = 0.0, ga = 0.0, gb = 0.0;   // reaction field
-#pragma unroll
-            for (int u = 0; u < TPL; u++) {
-                const int tfl = ttf[u] >> 16, t2t = ttf[u] & 0xFFFF;
-                const int both = tfl & pfl;
-                bool skip = !(both & SL_VALID) || (both & (SL_SITE | SL_FIXED)) ||
-                            (diag && p <= lane + WAVE * u);
-                const double dx = tx[u] - px, dy = ty[u] - py, dz = tz[u] - pz;
-                double d2 = dx * dx + dy * dy + dz * dz;
-                d2 = skip ? 1e30 : d2;
-                const int row = t2t * nt1 + t2p, lrow = t2t * S + t2p;
-                const double4 tl = s_tail[lrow];
-                const bool mx = ((tfl | pfl) & SL_SITE) != 0;
-                double y, de;
-                if constexpr ((FEAT & F_TAB) != 0) {
-                    de = pair_near_far<false>(P.rows[row], tl, P.ep, P.ires, d2, y);
-                    if constexpr (EN) {
-                        if (!skip) { if (mx) en[TE_EFPOTMX] += y; else en[TE_EFPOT] += y; }
-                    }
-                } else if ((int)tl.w & PF_EFPOT) {
-                    de = pair_near_far<false>(P.rows[row], tl, P.ep, P.ires, d2, y);
-                    if constexpr (EN) {
-                        if (!skip) { if (mx) en[TE_EFPOTMX] += y; else en[TE_EFPOT] += y; }
-                    }
-                } else {
-                    double q0 = 0.0, q1 = 0.0, q2 = 0.0;
-                    de = pair_analytic(P.rows[row], P, d2, q0, q1, q2);
-                    if constexpr (EN) {
-                        if (!skip) {
-                            en[mx ? TE_QQMX : TE_ELEC] += q0;
-                            en[mx ? TE_VDWMX : TE_VDW] += q1;
-                            en[mx ? TE_SRPMFMX : TE_SRPMF] += q2;
+    for (int J = J0; J < J1; J++) {
+        const bool diag = I == J;
+        double *const prow = P.tpart + ((size_t)(tile_row(J, n, R) + I) * NC) * TT;
+        int32_t *const pflag = P.tflag + (size_t)(tile_row(J, n, R) + I) * TPL;
+#pragma unroll 1
+        for (int q = 0; q < TPL; q++) {
+            const SlotInfo o = slot_info<FEAT>(P, J * TT + WAVE * q + lane);
+            const int pf = o.tf >> 16;
+            const int andJ = wave_and8((pf & SL_VALID) ? pf : ~SL_VALID), orJ = wave_or8(pf);
+            const bool ionJ = (orJ & SL_ION) && (andJ & SL_ION);
+            // the sums of the partner this lane holds
+            double gx = 0.0, gy = 0.0, gz = 0.0, ga = 0.0, gb = 0.0;
+            bool rfsums = false;   // the chunk's A and B may be nonzero
+            // sites among themselves and fixed ions among themselves have no pair
+            if ((orI & SL_VALID) && (orJ & SL_VALID) && !(orI & orJ & (SL_SITE | SL_FIXED))) {
+                __builtin_amdgcn_wave_barrier();
+                C.x[lane] = o.x; C.y[lane] = o.y; C.z[lane] = o.z;
+                C.x[lane + WAVE] = o.x; C.y[lane + WAVE] = o.y; C.z[lane + WAVE] = o.z;
+                const bool fast = ionJ && (siteI || (ionI && !(RF && ((orI | orJ) & SL_RFODD))));
+                const bool rfw = RF && ionI && (orI & SL_RFON) && (orJ & SL_RFON);
+                if (fast) {
+                    const bool mask = diag || !(andI & SL_VALID) || !(andJ & SL_VALID);
+                    const uint64_t pval = __ballot(pf & SL_VALID);
+                    // the pair type: a run's slots are filled from its start
+                    const int t2J = __builtin_amdgcn_readfirstlane(o.tf & 0xFFFF);
+                    const DevPair &pr = P.rows[t2I * nt1 + t2J];
+                    const double s3 = wave_uniform(pr.sc3), s6 = wave_uniform(6.0 * pr.sc3);
+                    const double fc = wave_uniform(pr.fct), hi = wave_uniform(pr.dm2hi);
+                    const int fl = __builtin_amdgcn_readfirstlane(pr.flags);
+                    // a partner within table range of the targets' box?
+                    const double ex = fmax(fmax(bx0 - o.x, o.x - bx1), 0.0);
+                    const double ey = fmax(fmax(by0 - o.y, o.y - by1), 0.0);
+                    const double ez = fmax(fmax(bz0 - o.z, o.z - bz1), 0.0);
+                    const bool far = __ballot(!(ex * ex + ey * ey + ez * ez > hi * (1.0 + 1e-9))) == 0ull;
+                    if constexpr (RF) {
+                        if (rfw) {
+                            const double w = (pf & SL_RFON) ? o.q * o.sr : 0.0;
+                            C.rr[lane] = o.rr; C.qs[lane] = w;
+                            C.rr[lane + WAVE] = o.rr; C.qs[lane + WAVE] = w;
                         }
                     }
-                }
-                de = skip ? 0.0 : de;
-                const double fxp = de * dx, fyp = de * dy, fzp = de * dz;
-                if (tfl & SL_RECV) { ax_[u] += fxp; ay_[u] += fyp; az_[u] += fzp; }
-                gx += fxp; gy += fyp; gz += fzp;
-                if constexpr (RF) {
-                    // rfpar.f90:177-223 for the ion pair (lo, hi) by index: counted when
-                    // srfe(lo) is nonzero and hi is moving and inside the grid box
-                    const bool thi = tix[u] > pix;
-                    const bool on = !skip && !mx &&
-                                    (thi ? (psr != 0.0 && (tfl & SL_HI)) : (tsr[u] != 0.0 && (pfl & SL_HI)));
-                    const double m = on ? 1.0 : 0.0;
-                    const double aux0 = P.celec * tq[u] * pq;
-                    const double srfeij = tsr[u] * psr, reffij = trr[u] * prr;
-                    const double rfdn = rsqrt_nr(reffij * reffij + (on ? d2 : 1.0));
-                    const double rfcf = reffij * rfdn;
-                    const double aux1 = aux0 * rfcf;
-                    const double aux2 = aux0 * srfeij * (rfdn * (rfdn * rfdn));
-                    const double aux3 = -aux2 * ((on ? d2 : 1.0) + reffij * 0.5);
-                    const double der = m * (aux2 * reffij);
-                    if constexpr (EN) en[TE_RFPAR] = fma(m, aux1 * srfeij, en[TE_RFPAR]);
-                    aa_[u] = fma(m, -aux1 * psr, aa_[u]);
-                    ab_[u] = fma(m, aux3 * prr, ab_[u]);
-                    ga = fma(m, -aux1 * tsr[u], ga);
-                    gb = fma(m, aux3 * trr[u], gb);
-                    ax_[u] = fma(der, dx, ax_[u]);
-                    ay_[u] = fma(der, dy, ay_[u]);
-                    az_[u] = fma(der, dz, az_[u]);
-                    rx = fma(der, dx, rx);
-                    ry = fma(der, dy, ry);
-                    rz = fma(der, dz, rz);
-                }
-            }
-            const double pw = (pfl & SL_RECV) ? 1.0 : 0.0;
-            s_fx[p] -= pw * gx + rx;
-            s_fy[p] -= pw * gy + ry;
-            s_fz[p] -= pw * gz + rz;
-            if constexpr (RF) {
-                s_fa[p] += ga;
-                s_fb[p] += gb;
-            }
-            // LDS operations of one wavefront complete in issue order; this keeps the
-            // compiler from moving the next step's partner reads above these updates
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        }
-    };
-    // Mask-free sweep over tile pairs of one class each (see the file comment).  RFW: the
-    // reaction-field term with the ion weights in the charges (a pair counts when both
-    // ions are RFON; with no RFODD ion that is the reference's rule, rfpar.f90:177-223, in
-    // either index order); MX: sites against moving ions, all pairs mixed, forces kept
-    // only for receiving particles.  The radial reaction-field force joins the pair force.
-    auto sweep_fast = [&](auto en_on, auto rf_on, auto mx_on) {
-        constexpr bool EN = decltype(en_on)::value;
-        constexpr bool RFW = decltype(rf_on)::value;
-        constexpr bool MX = decltype(mx_on)::value;
-        double tcq[TPL];
+                    // LDS operations of one wavefront complete in order; the fences keep the
+                    // compiler from moving them across
+                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                    __builtin_amdgcn_wave_barrier();
+                    double e0 = 0.0, e1 = 0.0, e2 = 0.0, e3 = 0.0, erf = 0.0;
+                    // The reaction-field term of a pair (rfpar.f90:177-223) with R = reff reff',
+                    // w = 1/sqrt(R^2 + d2), Q = celec q srfe q' srfe' (ions' weights in qs):
+                    // energy Q R w; force factor Q w^3 R; A of a target sums R w (q' srfe') and
+                    // takes its factor celec q at the end, B sums Q w^3 (d2 + R / 2) reff'.
+                    auto rf_pair = [&](int u, double d2, double prr, double pqs, double &f) {
+                        const double rp = trr[u] * prr;
+                        const double w = rsqrt_c3(fma(rp, rp, d2));
+                        const double a = rp * w, Q = tqs[u] * pqs;
+                        const double a2 = Q * w * (w * w);
+                        const double a3 = a2 * fma(rp, 0.5, d2);
+                        if constexpr (EN) erf = fma(Q, a, erf);
+                        wa[u] = fma(a, pqs, wa[u]);
+                        wb[u] = fma(a3, prr, wb[u]);
+                        ga = fma(a, tqs[u], ga);
+                        gb = fma(a3, trr[u], gb);
+                        f = fma(a2, rp, f);
+                    };
+                    auto add = [&](int u, double f, double dx, double dy, double dz) {
+                        ax_[u] = fma(f, dx, ax_[u]);
+                        ay_[u] = fma(f, dy, ay_[u]);
+                        az_[u] = fma(f, dz, az_[u]);
+                        gx = fma(-f, dx, gx);
+                        gy = fma(-f, dy, gy);
+                        gz = fma(-f, dz, gz);
+                    };
+                    // no pair in range: the tail alone
+                    auto sweep_far = [&](auto rf_on) {
+                        constexpr bool RFW = decltype(rf_on)::value;
+#pragma unroll (TPL == 1 ? 4 : TPL == 2 ? 2 : 1)
+                        for (int k = 0; k < WAVE; k++) {
+                            const double px = C.x[lane + k], py = C.y[lane + k], pz = C.z[lane + k];
+                            double prr = 0.0, pqs = 0.0;
+                            if constexpr (RFW) { prr = C.rr[lane + k]; pqs = C.qs[lane + k]; }
 #pragma unroll
-        for (int u = 0; u < TPL; u++)
-            tcq[u] = ((ttf[u] >> 16) & SL_RFON) ? P.celec * tq[u] : 0.0;
-        for (int k = 0; k < TT; k++) {
-            const int p = ((lane + k / TPL) & (WAVE - 1)) + WAVE * (k % TPL);
-            const double px = s_x[p], py = s_y[p], pz = s_z[p];
-            const int ptf = s_tf[p];
-            const int t2p = ptf & 0xFFFF, pfl = ptf >> 16;
-            double psr = 0.0, prr = 0.0, pq = 0.0;
-            if constexpr (RFW) {
-                psr = s_sr[p];
-                prr = s_rr[p];
-                pq = (pfl & SL_RFON) ? s_q[p] : 0.0;
-            }
-            double gx = 0.0, gy = 0.0, gz = 0.0, ga = 0.0, gb = 0.0;
+                            for (int u = 0; u < TPL; u++) {
+                                const double dx = tx[u] - px, dy = ty[u] - py, dz = tz[u] - pz;
+                                const double d2 = pair_d2(dx, dy, dz);
+                                const double r = rsqrt_c3(d2), i2 = r * r, i4 = i2 * i2, fr = fc * r;
+                                double f = fma(s6 * i2, i4, fr) * i2;
+                                if constexpr (EN) e0 += fma(s3 * i2, i4, fr);
+                                if constexpr (RFW) rf_pair(u, d2, prr, pqs, f);
+                                add(u, f, dx, dy, dz);
+                            }
+                            gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
+                            if constexpr (RFW) { ga = wave_next(ga); gb = wave_next(gb); }
+                        }
+                    };
+                    // a step's mask: a pair counts when both slots hold a particle and, on the
+                    // diagonal, once: against its own chunk a lane takes the first half of the
+                    // rotation, against higher chunks all of it, against lower ones none
+                    auto counts = [&](int u, int k) {
+                        const bool pv = (pval >> ((lane + k) & (WAVE - 1))) & 1ull;
+                        bool c = pv && ((ttf[u] >> 16) & SL_VALID);
+                        if (diag) c = c && (u < q || (u == q && k > 0 && (k < 32 || (k == 32 && lane < 32))));
+                        return c;
+                    };
+                    const int kend = diag && q == 0 ? 33 : WAVE;
+                    // some pair may be in range: the tail of the others, and the bits (k: the
+                    // pair met at step k) of those, per target and per partner
+                    auto sweep_near = [&](auto rf_on, auto mask_on) {
+                        constexpr bool RFW = decltype(rf_on)::value;
+                        constexpr bool MASK = decltype(mask_on)::value;
+                        uint32_t tm[2][TPL], pm[2][TPL];
 #pragma unroll
-            for (int u = 0; u < TPL; u++) {
-                const int t2t = ttf[u] & 0xFFFF;
-                const double dx = tx[u] - px, dy = ty[u] - py, dz = tz[u] - pz;
-                const double d2 = dx * dx + dy * dy + dz * dz;
-                const int row = t2t * nt1 + t2p, lrow = t2t * S + t2p;
-                const double4 tl = s_tail[lrow];
-                double y, de;
-                if constexpr ((FEAT & F_TAB) != 0) {
-                    de = pair_near_far<true>(P.rows[row], tl, P.ep, P.ires, d2, y);
-                    if constexpr (EN) en[MX ? TE_EFPOTMX : TE_EFPOT] += y;
-                } else if ((int)tl.w & PF_EFPOT) {
-                    de = pair_near_far<true>(P.rows[row], tl, P.ep, P.ires, d2, y);
-                    if constexpr (EN) en[MX ? TE_EFPOTMX : TE_EFPOT] += y;
-                } else {
-                    double q0 = 0.0, q1 = 0.0, q2 = 0.0;
-                    de = pair_analytic(P.rows[row], P, d2, q0, q1, q2);
+                        for (int w = 0; w < 2; w++) {
+#pragma unroll
+                            for (int u = 0; u < TPL; u++) tm[w][u] = pm[w][u] = 0u;
+                            const int k1 = MASK ? min(kend, 32 * (w + 1)) : 32 * (w + 1);
+#pragma unroll 1
+                            for (int k = 32 * w; k < k1; k++) {
+                                const double px = C.x[lane + k], py = C.y[lane + k], pz = C.z[lane + k];
+                                const uint32_t bit = 1u << (k & 31);
+                                double prr = 0.0, pqs = 0.0;
+                                if constexpr (RFW) { prr = C.rr[lane + k]; pqs = C.qs[lane + k]; }
+#pragma unroll
+                                for (int u = 0; u < TPL; u++) {
+                                    const double dx = tx[u] - px, dy = ty[u] - py, dz = tz[u] - pz;
+                                    double d2 = pair_d2(dx, dy, dz);
+                                    const bool on = !MASK || counts(u, k);
+                                    if constexpr (MASK) d2 = on ? d2 : 1.0;
+                                    const bool near = on && d2 <= hi;
+                                    const double r = rsqrt_c3(d2), i2 = r * r, i4 = i2 * i2, fr = fc * r;
+                                    double f = fma(s6 * i2, i4, fr) * i2;
+                                    f = on && !near ? f : 0.0;
+                                    if constexpr (EN) e0 += on && !near ? fma(s3 * i2, i4, fr) : 0.0;
+                                    const uint32_t nb = near ? bit : 0u;
+                                    tm[w][u] |= nb;
+                                    pm[w][u] |= nb;
+                                    // a masked pair: zero weight and reff, so every term is zero
+                                    if constexpr (RFW) rf_pair(u, d2, on ? prr : 0.0, on ? pqs : 0.0, f);
+                                    add(u, f, dx, dy, dz);
+                                    pm[w][u] = wave_next(pm[w][u]);
+                                }
+                                gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
+                                if constexpr (RFW) { ga = wave_next(ga); gb = wave_next(gb); }
+                            }
+                            if constexpr (MASK) {   // the steps left out of a half rotation
+#pragma unroll 1
+                                for (int k = max(k1, 32 * w); k < 32 * (w + 1); k++) {
+                                    gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
+                                    if constexpr (RFW) { ga = wave_next(ga); gb = wave_next(gb); }
+#pragma unroll
+                                    for (int u = 0; u < TPL; u++) pm[w][u] = wave_next(pm[w][u]);
+                                }
+                            }
+                        }
+                        // after its 32 steps the second word is home (lane l holds partner
+                        // l's), the first half way round
+#pragma unroll
+                        for (int u = 0; u < TPL; u++)
+                            pm[0][u] = __shfl(pm[0][u], (lane + 32) & (WAVE - 1), WAVE);
+                        const double lo = wave_uniform(pr.dm2lo), dmi = wave_uniform(pr.dmi);
+                        const int nxi = __builtin_amdgcn_readfirstlane(pr.nxi);
+                        const int nlast = __builtin_amdgcn_readfirstlane(pr.nlast);
+                        // the lane's pairs in range with the entries (lane + sgn k) of the
+                        // staged positions sx, sy, sz, two at a time; energy when it is the target
+                        auto work_off = [&](uint64_t m, int sgn, double x0, double y0, double z0,
+                                            const double *sx, const double *sy, const double *sz,
+                                            double &fx, double &fy, double &fz, bool head) {
+                            while (m) {
+                                double dx[2], dy[2], dz[2], d2[2], ri[2], k0[2], k1[2], k2[2];
+                                const bool two = (m & (m - 1)) != 0ull;
+#pragma unroll
+                                for (int h = 0; h < 2; h++) {
+                                    const int k = __ffsll((unsigned long long)m) - 1;
+                                    if (h == 0 && two) m &= m - 1;
+                                    const int p = (lane + sgn * k) & (WAVE - 1);
+                                    dx[h] = x0 - sx[p]; dy[h] = y0 - sy[p]; dz[h] = z0 - sz[p];
+                                    d2[h] = pair_d2(dx[h], dy[h], dz[h]);
+                                    ri[h] = rsqrt_c3(d2[h]);
+                                    int kn = (int)((root_of(d2[h], ri[h]) - dmi) * P.ires) + nxi;
+                                    kn = min(max(kn, nxi), nlast);
+                                    const double *kp = reinterpret_cast<const double *>(P.ep + kn);
+                                    if constexpr (EN) k0[h] = kp[0];
+                                    k1[h] = kp[1];
+                                    k2[h] = kp[2];
+                                }
+                                m &= m - 1;
+#pragma unroll
+                                for (int h = 0; h < 2; h++) {
+                                    double f = -k1[h] * ri[h] - 2.0 * k2[h], y = 0.0;
+                                    if constexpr (EN) {
+                                        const double x = root_of(d2[h], ri[h]);
+                                        y = k0[h] + x * (k1[h] + x * k2[h]);
+                                    }
+                                    if (d2[h] < lo) f = pair_wall(pr, ri[h], y);
+                                    if (h == 1 && !two) f = y = 0.0;
+                                    fx = fma(f, dx[h], fx); fy = fma(f, dy[h], fy); fz = fma(f, dz[h], fz);
+                                    if constexpr (EN) { if (head) e0 += y; }
+                                }
+                            }
+                        };
+#pragma unroll
+                        for (int u = 0; u < TPL; u++) {
+                            const uint64_t mt = tm[0][u] | ((uint64_t)tm[1][u] << 32);
+                            const uint64_t mp = pm[0][u] | ((uint64_t)pm[1][u] << 32);
+                            work_off(mt, 1, tx[u], ty[u], tz[u], C.x, C.y, C.z, ax_[u], ay_[u], az_[u], true);
+                            work_off(mp, -1, o.x, o.y, o.z, C.tx + WAVE * u, C.ty + WAVE * u, C.tz + WAVE * u,
+                                     gx, gy, gz, false);
+                        }
+                    };
+                    // analytic pairs
+                    auto sweep_analytic = [&](auto rf_on) {
+                        constexpr bool RFW = decltype(rf_on)::value;
+#pragma unroll 1
+                        for (int k = 0; k < WAVE; k++) {
+                            const double px = C.x[lane + k], py = C.y[lane + k], pz = C.z[lane + k];
+                            double prr = 0.0, pqs = 0.0;
+                            if constexpr (RFW) { prr = C.rr[lane + k]; pqs = C.qs[lane + k]; }
+#pragma unroll
+                            for (int u = 0; u < TPL; u++) {
+                                const double dx = tx[u] - px, dy = ty[u] - py, dz = tz[u] - pz;
+                                const bool on = !mask || counts(u, k);
+                                const double d2 = on ? pair_d2(dx, dy, dz) : 1.0;
+                                double q0 = 0.0, q1 = 0.0, q2 = 0.0;
+                                double f = pair_analytic(pr, P, d2, q0, q1, q2);
+                                f = on ? f : 0.0;
+                                if constexpr (EN) {
+                                    if (on) { e1 += q0; e2 += q1; e3 += q2; }
+                                }
+                                if constexpr (RFW) rf_pair(u, d2, on ? prr : 0.0, on ? pqs : 0.0, f);
+                                add(u, f, dx, dy, dz);
+                            }
+                            gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
+                            if constexpr (RFW) { ga = wave_next(ga); gb = wave_next(gb); }
+                        }
+                    };
+                    auto pick = [&](auto rf_on) {
+                        if constexpr (!TAB) {
+                            if (!(fl & PF_EFPOT)) { sweep_analytic(rf_on); return; }
+                        }
+                        if (mask) sweep_near(rf_on, std::true_type{});
+                        else if (!far) sweep_near(rf_on, std::false_type{});
+                        else sweep_far(rf_on);
+                    };
+                    if (RF && rfw) {
+                        rfsums = true;
+                        pick(std::bool_constant<RF>{});
+                        // the partners' own factors
+                        ga *= (pf & SL_RFON) ? -o.q : 0.0;
+                        gb = -gb;
+                    } else {
+                        pick(std::false_type{});
+                    }
                     if constexpr (EN) {
-                        en[MX ? TE_QQMX : TE_ELEC] += q0;
-                        en[MX ? TE_VDWMX : TE_VDW] += q1;
-                        en[MX ? TE_SRPMFMX : TE_SRPMF] += q2;
+                        en[TE_EFPOTMX] += siteI ? e0 : 0.0; en[TE_EFPOT] += siteI ? 0.0 : e0;
+                        en[TE_QQMX] += siteI ? e1 : 0.0; en[TE_ELEC] += siteI ? 0.0 : e1;
+                        en[TE_VDWMX] += siteI ? e2 : 0.0; en[TE_VDW] += siteI ? 0.0 : e2;
+                        en[TE_SRPMFMX] += siteI ? e3 : 0.0; en[TE_SRPMF] += siteI ? 0.0 : e3;
+                        en[TE_RFPAR] += erf;
+                    }
+                } else {
+                    C.tf[lane] = o.tf; C.tf[lane + WAVE] = o.tf;
+                    if constexpr (RF) {
+                        C.sr[lane] = o.sr; C.rg[lane] = o.rr; C.q[lane] = o.q; C.ix[lane] = o.idx;
+                        C.sr[lane + WAVE] = o.sr; C.rg[lane + WAVE] = o.rr; C.q[lane + WAVE] = o.q;
+                        C.ix[lane + WAVE] = o.idx;
+                    }
+                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                    __builtin_amdgcn_wave_barrier();
+                    rfsums = RF;
+#pragma unroll 1
+                    for (int k = 0; k < WAVE; k++) {
+                        const double px = C.x[lane + k], py = C.y[lane + k], pz = C.z[lane + k];
+                        const int ptf = C.tf[lane + k];
+                        const int t2p = ptf & 0xFFFF, pfl = ptf >> 16;
+                        const int p = ((lane + k) & (WAVE - 1)) + WAVE * q;   // slot in tile J
+                        double psr = 0.0, prr = 0.0, pq = 0.0;
+                        int pix = 0;
+                        if constexpr (RF) {
+                            psr = C.sr[lane + k]; prr = C.rg[lane + k]; pq = C.q[lane + k];
+                            pix = C.ix[lane + k];
+                        }
+                        double hx = 0.0, hy = 0.0, hz = 0.0;    // pair force on the partner (negated)
+#pragma unroll
+                        for (int u = 0; u < TPL; u++) {
+                            const int tfl = ttf[u] >> 16, t2t = ttf[u] & 0xFFFF;
+                            const int both = tfl & pfl;
+                            bool skip = !(both & SL_VALID) || (both & (SL_SITE | SL_FIXED)) ||
+                                        (diag && p <= lane + WAVE * u);
+                            const double dx = tx[u] - px, dy = ty[u] - py, dz = tz[u] - pz;
+                            double d2 = dx * dx + dy * dy + dz * dz;
+                            d2 = skip ? 1e30 : d2;
+                            const DevPair &rw = P.rows[t2t * nt1 + t2p];
+                            const double4 tl = make_double4(rw.sc3, rw.fct, rw.dm2hi, 0.0);
+                            const bool mx = ((tfl | pfl) & SL_SITE) != 0;
+                            double y, de;
+                            if (TAB || (rw.flags & PF_EFPOT)) {
+                                de = pair_near_far<false>(rw, tl, P.ep, P.ires, d2, y);
+                                if constexpr (EN) {
+                                    if (!skip) { if (mx) en[TE_EFPOTMX] += y; else en[TE_EFPOT] += y; }
+                                }
+                            } else {
+                                double q0 = 0.0, q1 = 0.0, q2 = 0.0;
+                                de = pair_analytic(rw, P, d2, q0, q1, q2);
+                                if constexpr (EN) {
+                                    if (!skip) {
+                                        en[mx ? TE_QQMX : TE_ELEC] += q0;
+                                        en[mx ? TE_VDWMX : TE_VDW] += q1;
+                                        en[mx ? TE_SRPMFMX : TE_SRPMF] += q2;
+                                    }
+                                }
+                            }
+                            de = skip ? 0.0 : de;
+                            const double fxp = de * dx, fyp = de * dy, fzp = de * dz;
+                            if (tfl & SL_RECV) { ax_[u] += fxp; ay_[u] += fyp; az_[u] += fzp; }
+                            hx += fxp; hy += fyp; hz += fzp;
+                            if constexpr (RF) {
+                                // rfpar.f90:177-223 for the ion pair (lo, hi) by index: counted when
+                                // srfe(lo) is nonzero and hi is moving and inside the grid box
+                                const bool thi = tix[u] > pix;
+                                const bool on = !skip && !mx &&
+                                                (thi ? (psr != 0.0 && (tfl & SL_HI)) : (tsr[u] != 0.0 && (pfl & SL_HI)));
+                                const double m = on ? 1.0 : 0.0;
+                                const double aux0 = P.celec * tq[u] * pq;
+                                const double srfeij = tsr[u] * psr, reffij = trr[u] * prr;
+                                const double rfdn = rsqrt_nr(reffij * reffij + (on ? d2 : 1.0));
+                                const double rfcf = reffij * rfdn;
+                                const double aux1 = aux0 * rfcf;
+                                const double aux2 = aux0 * srfeij * (rfdn * (rfdn * rfdn));
+                                const double aux3 = -aux2 * ((on ? d2 : 1.0) + reffij * 0.5);
+                                const double der = m * (aux2 * reffij);
+                                if constexpr (EN) en[TE_RFPAR] = fma(m, aux1 * srfeij, en[TE_RFPAR]);
+                                aa_[u] = fma(m, -aux1 * psr, aa_[u]);
+                                ab_[u] = fma(m, aux3 * prr, ab_[u]);
+                                ga = fma(m, -aux1 * tsr[u], ga);
+                                gb = fma(m, aux3 * trr[u], gb);
+                                ax_[u] = fma(der, dx, ax_[u]);
+                                ay_[u] = fma(der, dy, ay_[u]);
+                                az_[u] = fma(der, dz, az_[u]);
+                                gx = fma(-der, dx, gx);
+                                gy = fma(-der, dy, gy);
+                                gz = fma(-der, dz, gz);
+                            }
+                        }
+                        const double pw = (pfl & SL_RECV) ? 1.0 : 0.0;
+                        gx -= pw * hx; gy -= pw * hy; gz -= pw * hz;
+                        gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
+                        if constexpr (RF) { ga = wave_next(ga); gb = wave_next(gb); }
                     }
                 }
-                if constexpr (RFW) {
-                    const double srfeij = tsr[u] * psr, reffij = trr[u] * prr;
-                    const double rfdn = rsqrt_c3(fma(reffij, reffij, d2));
-                    const double aux0 = tcq[u] * pq;
-                    const double aux1 = aux0 * (reffij * rfdn);
-                    const double aux2 = aux0 * srfeij * (rfdn * (rfdn * rfdn));
-                    const double aux3 = -aux2 * (d2 + reffij * 0.5);
-                    if constexpr (EN) en[TE_RFPAR] = fma(aux1, srfeij, en[TE_RFPAR]);
-                    aa_[u] = fma(-aux1, psr, aa_[u]);
-                    ab_[u] = fma(aux3, prr, ab_[u]);
-                    ga = fma(-aux1, tsr[u], ga);
-                    gb = fma(aux3, trr[u], gb);
-                    de = fma(aux2, reffij, de);
+                // the next chunk's staging stays below this chunk's reads
+                __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            }
+            rfany |= rfsums;
+            if (diag) {   // partner sums of the tile's own slots
+#pragma unroll
+                for (int u = 0; u < TPL; u++) {
+                    if (u != q) continue;
+                    ax_[u] += gx; ay_[u] += gy; az_[u] += gz;
+                    if constexpr (RF) { aa_[u] += ga; ab_[u] += gb; }
                 }
-                ax_[u] = fma(de, dx, ax_[u]);
-                ay_[u] = fma(de, dy, ay_[u]);
-                az_[u] = fma(de, dz, az_[u]);
-                gx = fma(de, dx, gx);
-                gy = fma(de, dy, gy);
-                gz = fma(de, dz, gz);
-            }
-            if constexpr (MX) {
-                const double pw = (pfl & SL_RECV) ? 1.0 : 0.0;
-                s_fx[p] -= pw * gx;
-                s_fy[p] -= pw * gy;
-                s_fz[p] -= pw * gz;
             } else {
-                s_fx[p] -= gx;
-                s_fy[p] -= gy;
-                s_fz[p] -= gz;
+                // a chunk without reaction-field sums writes the three force components only
+                // and says so in its flag, which k_tfin reads before it reads the A and B rows
+                double *const dp = prow + WAVE * q + lane;
+                dp[0] = gx; dp[(size_t)TT] = gy; dp[2 * (size_t)TT] = gz;
+                if constexpr (RF) {
+                    if (rfsums) { dp[3 * (size_t)TT] = ga; dp[4 * (size_t)TT] = gb; }
+                    if (lane == 0) pflag[q] = rfsums ? 1 : 0;
+                }
             }
-            if constexpr (RFW) {
-                s_fa[p] += ga;
-                s_fb[p] += gb;
-            }
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
         }
-        if constexpr (MX) {
-#pragma unroll
-            for (int u = 0; u < TPL; u++)
-                if (!((ttf[u] >> 16) & SL_RECV)) ax_[u] = ay_[u] = az_[u] = 0.0;
-        }
-    };
-
-    // the classes of the two tiles, uniform over the wavefront
-    int andI = ~0, orI = 0, andJ = ~0, orJ = 0;
+    }
+    // the item's row of tile I: after its I partner rows, one per group from I's own
+    const size_t trow = (size_t)tile_row(I, n, R) + I + (g - I / R);
+    double *const dst = P.tpart + trow * NC * TT + lane;
 #pragma unroll
     for (int u = 0; u < TPL; u++) {
-        const int fi = ttf[u] >> 16, fj = s_tf[lane + WAVE * u] >> 16;
-        andI &= fi; orI |= fi; andJ &= fj; orJ |= fj;
-    }
-    andI = wave_and8(andI); orI = wave_or8(orI);
-    andJ = wave_and8(andJ); orJ = wave_or8(orJ);
-    const bool ionI = andI & SL_ION, ionJ = andJ & SL_ION;
-    const bool siteI = (andI & (SL_VALID | SL_SITE)) == (SL_VALID | SL_SITE);
-    const bool siteJ = (andJ & (SL_VALID | SL_SITE)) == (SL_VALID | SL_SITE);
-    const bool wr = P.write_energy != 0;
-    bool rfsums = false;   // this tile pair's reaction-field sums (A, B) may be nonzero
-    if (!(orI & SL_ION) && !(orJ & SL_ION)) {
-        // sites, fixed ions and empty slots only: no pair of these is evaluated
-    } else if (!diag && ionI && ionJ && !(RF && ((orI | orJ) & SL_RFODD))) {
-        if (RF && (orI & SL_RFON) && (orJ & SL_RFON)) {
-            rfsums = true;
-            if (wr) sweep_fast(std::true_type{}, std::bool_constant<RF>{}, std::false_type{});
-            else sweep_fast(std::false_type{}, std::bool_constant<RF>{}, std::false_type{});
-        } else {
-            if (wr) sweep_fast(std::true_type{}, std::false_type{}, std::false_type{});
-            else sweep_fast(std::false_type{}, std::false_type{}, std::false_type{});
-        }
-    } else if (!diag && ((ionI && siteJ) || (siteI && ionJ))) {
-        if (wr) sweep_fast(std::true_type{}, std::false_type{}, std::true_type{});
-        else sweep_fast(std::false_type{}, std::false_type{}, std::true_type{});
-    } else {
-        rfsums = RF;
-        if (wr) sweep(std::true_type{});
-        else sweep(std::false_type{});
-    }
-    // the wavefront reads its own sums back: its LDS operations complete in order, and the
-    // fence keeps the compiler from moving the reads above the sweep's last updates
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_wave_barrier();
-
-    // a tile pair without reaction-field sums writes the three force components only and
-    // says so in tflag[item], which k_tfin reads before it reads the A and B rows
-    const int NC = RF ? 5 : 3, nc = rfsums ? NC : 3;
-    double *const part = P.tpart;
-    if constexpr (RF) {
-        if (lane == 0) P.tflag[item] = rfsums ? 1 : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < TPL; u++) {
-        const int t = lane + WAVE * u;
-        double v[5] = {ax_[u], ay_[u], az_[u], aa_[u], ab_[u]};
-        if (diag) {
-            v[0] += s_fx[t]; v[1] += s_fy[t]; v[2] += s_fz[t];
-            if constexpr (RF) { v[3] += s_fa[t]; v[4] += s_fb[t]; }
-        }
-        double *dst = part + ((size_t)(J * n + I) * NC) * TT + t;
-#pragma unroll
-        for (int c = 0; c < NC; c++)
-            if (c < nc) dst[(size_t)c * TT] = v[c];
-        if (!diag) {
-            const double w[5] = {s_fx[t], s_fy[t], s_fz[t], RF ? s_fa[t] : 0.0, RF ? s_fb[t] : 0.0};
-            double *dp = part + ((size_t)(I * n + J) * NC) * TT + t;
-#pragma unroll
-            for (int c = 0; c < NC; c++)
-                if (c < nc) dp[(size_t)c * TT] = w[c];
+        // the fast sweeps add to every target, a site that is not free too
+        const int f = ttf[u] >> 16;
+        const bool keep = (f & (SL_SITE | SL_RECV)) != SL_SITE;
+        double *const d = dst + WAVE * u;
+        d[0] = keep ? ax_[u] : 0.0; d[(size_t)TT] = keep ? ay_[u] : 0.0; d[2 * (size_t)TT] = keep ? az_[u] : 0.0;
+        if constexpr (RF) {
+            if (rfany) {
+                d[3 * (size_t)TT] = (f & SL_RFON) ? fma(-P.celec * tq[u], wa[u], aa_[u]) : aa_[u];
+                d[4 * (size_t)TT] = ab_[u] - wb[u];
+            }
+            if (lane == 0) P.tflag[trow * TPL + u] = rfany ? 1 : 0;
         }
     }
-    if (P.write_energy) {
+    if constexpr (EN) {
 #pragma unroll
         for (int c = 0; c < NTE; c++) {
             const double v = wave_sum(en[c]);
@@ -458,7 +643,7 @@ __device__ __forceinline__ double group8_sum(double v) {
 }
 
 // k_tfin: slot s of the spatial order, eight lanes per slot (32 slots per block).  The
-// lanes split the slot's ntile partial rows, then its grid corners (lane c takes corner c
+// lanes split the slot's partial rows, then its grid corners (lane c takes corner c
 // of the trilinear stencils, c, c + 8, .. of the 27-node B-spline); lane 0 of the group
 // finishes the particle.  Sites and moving ions are finished as by k_step; a fixed ion
 // only receives its reaction-field force (rfpar.f90:177-223 applies it to both ions of a
@@ -468,32 +653,34 @@ __global__ __launch_bounds__(BLOCK) void k_tfin(StepParams P) {
     constexpr bool RF = (FEAT & F_RFT) != 0;
     const int tid = threadIdx.x, sub = tid & 7;
     const int s = blockIdx.x * (BLOCK / 8) + (tid >> 3);
-    const bool sv = s < P.ntot;
-    const int ss = sv ? s : 0;
+    const int nslot = P.ntile * WAVE * P.ttpl, ss = s < nslot ? s : 0;
     const double4 pa = P.spos[ss];
-    const int i = __double2hiint(pa.w), t2 = __double2loint(pa.w);
+    const bool sv = s < nslot && __double2hiint(pa.w) >= 0;   // else an empty slot
+    const int i = sv ? __double2hiint(pa.w) : 0, t2 = __double2loint(pa.w);
     const int ns = P.nsites;
     const bool is_site = i < ns, fixed = !is_site && i < ns + P.nfix;
-    const int TT = WAVE * P.ttpl, n = P.ntile, NC = RF ? 5 : 3;
+    const int TT = WAVE * P.ttpl, n = P.ntile, NC = RF ? 5 : 3, R = P.trun;
     const int I = ss / TT, t = ss - I * TT;
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    // rows K = sub, sub + 8, .. added in that order, KU of them per iteration so that their
+    // the slot's rows: one per lower tile, one per column group from its own; rows K = sub,
+    // sub + 8, .. added in that order, KU of them per iteration so that their
     // loads (the flags, then the rows) are in flight together
     constexpr int KU = 8;
-    for (int K0 = sub; K0 < n; K0 += 8 * KU) {
+    const size_t row0 = (size_t)tile_row(I, n, R);
+    const int nrow = (int)(tile_row(I + 1, n, R) - row0);
+    for (int K0 = sub; K0 < nrow; K0 += 8 * KU) {
         bool ok[KU], ab[KU];
         const double *src[KU];
 #pragma unroll
         for (int u = 0; u < KU; u++) {
             const int K = K0 + 8 * u;
-            ok[u] = K < n;
-            const int Kc = ok[u] ? K : I;
-            src[u] = P.tpart + ((size_t)(Kc * n + I) * NC) * TT + t;
+            ok[u] = K < nrow;
+            const size_t row = row0 + (ok[u] ? K : 0);
+            src[u] = P.tpart + row * NC * TT + t;
             ab[u] = false;
-            // the A and B rows only where the tile pair (min, max) wrote them
+            // the A and B rows only where they were written
             if constexpr (RF) {
-                const int lo = min(I, Kc), hi = max(I, Kc);
-                const int32_t fl = P.tflag[hi * (hi + 1) / 2 + lo];   // a valid item even when !ok
+                const int32_t fl = P.tflag[row * P.ttpl + (t >> 6)];
                 ab[u] = ok[u] & (fl != 0);
             }
         }
@@ -685,16 +872,23 @@ __global__ __launch_bounds__(BLOCK) void k_tfin(StepParams P) {
 
 template <int FEAT>
 static void dispatch_tiles(const StepParams &p, hipStream_t s, int which) {
-    const int nt1 = p.nttyp + 1;
-    const size_t lds = sizeof(double4) * nt1 * tail_stride(nt1);
-    const int nblk = tile_blocks(p.ntile);
-    if (which & 1) switch (p.ttpl) {
-        case 1: hipLaunchKernelGGL((k_tiles<FEAT & (F_DNA | F_TAB | F_RFT), 1>), dim3(nblk), dim3(TILE_WAVES * WAVE), lds, s, p); break;
-        case 2: hipLaunchKernelGGL((k_tiles<FEAT & (F_DNA | F_TAB | F_RFT), 2>), dim3(nblk), dim3(TILE_WAVES * WAVE), lds, s, p); break;
-        default: hipLaunchKernelGGL((k_tiles<FEAT & (F_DNA | F_TAB | F_RFT), 4>), dim3(nblk), dim3(TILE_WAVES * WAVE), lds, s, p); break;
+    constexpr int TF = FEAT & (F_DNA | F_TAB | F_RFT);
+    if (which & 1) {
+        const dim3 grid(p.titems), block(WAVE);
+#define TILES(T)                                                                          \
+    do {                                                                                  \
+        if (p.write_energy) hipLaunchKernelGGL((k_tiles<TF, T, true>), grid, block, 0, s, p); \
+        else hipLaunchKernelGGL((k_tiles<TF, T, false>), grid, block, 0, s, p);           \
+    } while (0)
+        switch (p.ttpl) {
+            case 1: TILES(1); break;
+            case 2: TILES(2); break;
+            default: TILES(4); break;
+        }
+#undef TILES
     }
     if (which & 2)
-        hipLaunchKernelGGL((k_tfin<FEAT & ~F_TAB>), dim3((p.ntot + BLOCK / 8 - 1) / (BLOCK / 8)),
+        hipLaunchKernelGGL((k_tfin<FEAT & ~F_TAB>), dim3((p.ntile * WAVE * p.ttpl + BLOCK / 8 - 1) / (BLOCK / 8)),
                            dim3(BLOCK), 0, s, p);
 }
 

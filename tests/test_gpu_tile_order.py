@@ -1,0 +1,68 @@
+"""Tile mode's order and sweeps at their edges, against the C oracle: runs of one type that
+fill a tile exactly, miss it by one or spill one particle into the next, a type with a single
+ion, fixed ions in tiles of their own against site tiles, near and far chunks (a dense cluster
+and a far one), and enough tiles that an item takes several columns (tile_run > 1).
+
+Bar as the other parity tests: energies and norm-wise forces 1e-10 relative (FP64 sums of
+some 10^3 to 10^4 terms in another order, ~1e-13, and the pair forms to a few ulp).
+"""
+import numpy as np
+import pytest
+
+from bromoc_amd import configs
+from bromoc_amd.engine import Engine
+from oracle.oracle import Oracle
+
+from helpers import energy_errs, force_err, plain, pore_small, with_fixed
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-10
+
+
+def _check(s, tpb, monkeypatch):
+    monkeypatch.setenv("BROMOC_TPB", str(tpb))
+    g, o = Engine(s), Oracle(s)
+    assert g.tuning() == tpb
+    eg, eo = g.energy(), o.energy()
+    bad = {k: v for k, v in energy_errs(eg, eo).items() if v > TOL}
+    assert not bad, bad
+    assert force_err(g.forces(), o.forces()) <= TOL
+
+
+@pytest.mark.parametrize("tpb", [17, 18, 20])
+@pytest.mark.parametrize("counts", [(63, 1), (64, 64), (65, 127), (128, 129), (256, 3), (1, 300)])
+def test_type_runs_at_tile_edges(counts, tpb, monkeypatch):
+    a, b = counts
+    s = plain(seed=a + b, n_per_type=(a + b + 1) // 2).copy()
+    n = a + b
+    s.ntot = s.capacity = n
+    s.x, s.y, s.z = s.x[:n].copy(), s.y[:n].copy(), s.z[:n].copy()
+    s.typei = np.random.default_rng(n).permutation([1] * a + [2] * b).astype(np.int32)
+    _check(s, tpb, monkeypatch)
+
+
+@pytest.mark.parametrize("tpb", [17, 18, 20])
+@pytest.mark.parametrize("rf", [False, True])
+def test_fixed_ions_against_sites(rf, tpb, monkeypatch):
+    """More than a tile of each: the site forces include the fixed ions' (energy.mono.f90:584)."""
+    s = with_fixed(pore_small(seed=9, n_bp=24, n_ions=420), 130, nonfree=(0, 5, 70))
+    if rf:
+        s = configs.with_rfpar(s, seed=3, shape=(37, 37, 55), dcel=1.0, wall_radius=12.0)
+    _check(s, tpb, monkeypatch)
+
+
+@pytest.mark.parametrize("tpb", [17, 18])
+def test_near_and_far_clusters(tpb, monkeypatch):
+    """Two dense clusters further apart than the tables reach: pairs in range at most steps
+    of some chunks, at none of others."""
+    s = plain(seed=5, n_per_type=200).copy()
+    rng = np.random.default_rng(5)
+    g = np.stack(np.meshgrid(*[np.arange(6) * 2.4] * 3, indexing="ij"), -1).reshape(-1, 3)[:200]
+    p = np.concatenate([g, g + [60.0, 5.0, 70.0]]) + rng.uniform(-0.4, 0.4, (400, 3))
+    s.x, s.y, s.z = (p[:, k].copy() for k in range(3))
+    _check(s, tpb, monkeypatch)
+
+
+def test_items_of_several_columns(monkeypatch):
+    s = plain(seed=6, n_per_type=6100)
+    _check(s, 17, monkeypatch)
