@@ -3,10 +3,12 @@
 // Every replica owns a contiguous range of particle slots [off, off + cap) in shared
 // arrays; the pair tables, the repulsion map and the BD constants are shared, each replica
 // has its own static field and GCMC buffers.  One BD step of all replicas is one launch of
-// k_batch_step: its wavefronts take (replica, moving ion) work items -- ordered by replica
-// size, largest first -- from a device queue (or one item each in the non-persistent
-// shape), gather the ion's pair forces over its own replica's particles (all pairs, as
-// energy.mono.f90:117-194), its grid corners, and apply DYNAMICS0/1/2.  k_batch_gcmc runs
+// k_batch_step: its wavefronts take (replica, slot) work items -- a fixed table ordered by
+// replica size, largest first; a slot beyond the replica's present count is passed over --
+// from a device queue (or one item each in the non-persistent shape), gather the ion's pair
+// forces over its own replica's particles (all pairs, as energy.mono.f90:117-194), its grid
+// corners, and apply DYNAMICS0/1/2.  k_batch_noise draws the Gaussians of several steps at
+// once.  k_batch_gcmc runs
 // GRAND (grand.f90:40-118) for every replica at once, one workgroup per replica, with
 // INTERACT energies (interact.f90:19-419, ions only) reduced across the workgroup.
 #include <hip/hip_runtime.h>
@@ -18,71 +20,52 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "device.h"
 
 namespace bromoc {
 
-// ---- work-item prefix (one block of 1024 threads) and step / cycle counters
-constexpr int PREP_THREADS = 1024;
-constexpr int BATCH_LDS_WSTART = 4096;   // work-item prefix held in LDS up to this size
-
-__global__ __launch_bounds__(PREP_THREADS) void k_batch_prep(BatchParams B, int gcmc) {
-    const int tid = threadIdx.x;
+// ---- step and cycle counters: before GRAND (gcmc), or before `steps` BD steps whose noise
+// follows (ctl[4]: the counter of the first of them); and the queue counter of one step
+__global__ void k_batch_prep(BatchParams B, int gcmc, int steps) {
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
     if (gcmc) {
-        if (tid == 0) {
-            B.ctl[5] = B.ctl[6] + B.ctl[2];
-            B.ctl[2] += 1;
-        }
-        return;
-    }
-    __shared__ int s_wave[PREP_THREADS / WAVE];
-    __shared__ int s_carry;
-    if (tid == 0) {
+        B.ctl[5] = B.ctl[6] + B.ctl[2];
+        B.ctl[2] += 1;
+    } else {
         B.ctl[4] = B.ctl[1] + B.ctl[0];
-        B.ctl[0] += 1;
-        B.queue[0] = 0;
-        s_carry = 0;
+        B.ctl[0] += steps;
     }
-    __syncthreads();
-    const int lane = tid & (WAVE - 1), wv = tid / WAVE;
-    for (int base = 0; base < B.nrep; base += PREP_THREADS) {
-        const int k = base + tid;
-        int v = 0;
-        if (k < B.nrep) {
-            const int r = B.order[k];
-            v = max(0, B.ntot[r] - B.nfix[r]);
-        }
-        // inclusive scan within the wavefront
-        int x = v;
-#pragma unroll
-        for (int d = 1; d < WAVE; d <<= 1) {
-            const int y = __shfl_up(x, d, WAVE);
-            if (lane >= d) x += y;
-        }
-        if (lane == WAVE - 1) s_wave[wv] = x;
-        __syncthreads();
-        if (tid == 0) {
-            int acc = 0;
-            for (int q = 0; q < PREP_THREADS / WAVE; q++) {
-                const int t = s_wave[q];
-                s_wave[q] = acc;
-                acc += t;
-            }
-        }
-        __syncthreads();
-        const int excl = s_carry + s_wave[wv] + x - v;
-        if (k < B.nrep) B.wstart[k] = excl;
-        __syncthreads();
-        if (tid == PREP_THREADS - 1) s_carry = excl + v;
-        __syncthreads();
-    }
-    if (tid == 0) B.wstart[B.nrep] = s_carry;
+}
+__global__ void k_batch_queue(int32_t *queue) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) queue[0] = 0;
 }
 
-hipError_t launch_batch_prep(const BatchParams &b, int gcmc, hipStream_t s) {
-    hipLaunchKernelGGL(k_batch_prep, dim3(1), dim3(PREP_THREADS), 0, s, b, gcmc);
+hipError_t launch_batch_prep(const BatchParams &b, int gcmc, int steps, hipStream_t s) {
+    hipLaunchKernelGGL(k_batch_prep, dim3(1), dim3(64), 0, s, b, gcmc, steps);
+    return hipGetLastError();
+}
+
+// The Gaussians of `steps` steps from the counter ctl[4], row per step, three per item: one
+// thread per item and step.  Drawn in the step kernel they took every lane of a wavefront for
+// the three that need one (a tenth of a step at 4000 ions a replica, a third at 200).
+__global__ __launch_bounds__(BLOCK) void k_batch_noise(BatchParams B, int steps) {
+    const int w = blockIdx.x * BLOCK + threadIdx.x;
+    if (w >= B.nitems) return;
+    const int2 it = B.items[w];   // replica, slot in it
+    if (it.y >= B.ntot[it.x]) return;
+    const int row = blockIdx.y;
+    double g[3];
+    philox_gauss3((uint64_t)B.ctl[3], (uint64_t)B.ctl[4] + row, (uint64_t)it.x, it.y, g);
+    double *o = B.noise + 3 * ((size_t)row * B.nitems + w);
+    o[0] = g[0]; o[1] = g[1]; o[2] = g[2];
+}
+
+hipError_t launch_batch_noise(const BatchParams &b, int steps, hipStream_t s) {
+    if (b.nitems <= 0 || steps <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_batch_noise, dim3((b.nitems + BLOCK - 1) / BLOCK, steps), dim3(BLOCK), 0, s, b, steps);
     return hipGetLastError();
 }
 
@@ -91,6 +74,14 @@ hipError_t launch_batch_prep(const BatchParams &b, int gcmc, hipStream_t s) {
 // its own work item (a moving ion of some replica), strides over that replica's particles
 // and reduces its sums within the group.  Small replicas want small groups (more targets
 // in flight, the per-item latencies overlap); the autotuner picks G.
+//
+// A lane evaluates the analytic tail of 32 partners straight through, leaving out the pairs
+// within table range and noting each as a bit, then works the bits off.  With a branch to the
+// table per pair a wavefront took it at most iterations for the 2 % of its lanes that have a
+// pair in range (some other replica's or part of the box in each lane), and waited for the
+// knots each time.  The grid corners are loaded before the pair loop and used after it.
+// Measured per step, before and after (with the noise drawn beforehand, and no prefix kernel):
+// 256 replicas of 100..4000 ions 1.79 -> 0.86 ms, 256 replicas of 200 ions 101 -> 53 us.
 // feature bits of the k_batch_step specialisations
 constexpr int BF_PHIX = 1;       // static field grids
 constexpr int BF_PHIV = 2;       // repulsion map
@@ -99,54 +90,29 @@ constexpr int BF_ANALYTIC = 4;   // some pair type is analytic (else every pair 
 template <int G>
 __device__ __forceinline__ double group_sum(double v) {
 #pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-    return v;
-}
-
-// component c of philox_gauss3 (the same operations, so the same bits)
-__device__ __forceinline__ double philox_gauss1(uint64_t seed, uint64_t step, uint64_t stream,
-                                                int64_t i, int c) {
-    uint64_t w[4] = {step, (uint64_t)i, stream, 0};
-    philox4x64(w, seed, 0);
-    const double inv53 = 1.0 / 9007199254740992.0;
-    const double twopi = 2.0 * PI;
-    if (c < 2) {
-        const double u1 = (double)((w[0] >> 11) + 1) * inv53;
-        const double u2 = (double)(w[1] >> 11) * inv53;
-        const double r1 = sqrt(-2.0 * log(u1));
-        return c == 0 ? r1 * cos(twopi * u2) : r1 * sin(twopi * u2);
-    }
-    const double u3 = (double)((w[2] >> 11) + 1) * inv53;
-    const double u4 = (double)(w[3] >> 11) * inv53;
-    const double r2 = sqrt(-2.0 * log(u3));
-    return r2 * cos(twopi * u4);
+    for (int off = 16; off < G; off <<= 1) v += __shfl_xor(v, off, WAVE);
+    return G == 8 ? half_row_sum(v) : row_sum(v);
 }
 
 template <int FEAT, int G>
-__global__ __launch_bounds__(BLOCK) void k_batch_step(BatchParams B) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu((FEAT & BF_ANALYTIC) ? 2 : 4)))
+void k_batch_step(BatchParams B) {
     static_assert(G >= 8 && G <= WAVE && (WAVE % G) == 0, "lane group");
+    constexpr bool ANA = (FEAT & BF_ANALYTIC) != 0;
     const StepParams &P = B.sp;
-    // every (target type, partner type) row of the shared tables, and the work-item
-    // prefix when it fits
+    // every (target type, partner type) row of the shared tables
     extern __shared__ double4 s_dyn[];
     const int nt1 = P.nttyp + 1, nrow = nt1 * nt1;
     DevPair *s_rows = reinterpret_cast<DevPair *>(s_dyn);
     double4 *s_tail = s_dyn + (size_t)nrow * (sizeof(DevPair) / sizeof(double4));
-    int32_t *s_ws = reinterpret_cast<int32_t *>(s_tail + nrow);
-    const bool ws_lds = B.nrep + 1 <= BATCH_LDS_WSTART;
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid >> 6;
     const int sub = lane / G, sl = lane % G;
     for (int k = tid; k < nrow; k += BLOCK) {
         const DevPair d = P.rows[k];
         s_rows[k] = d;
-        s_tail[k] = make_double4(d.sc3, d.fct, d.dm2hi, 0.0);
+        s_tail[k] = make_double4(d.sc3, d.fct, ANA && !(d.flags & PF_EFPOT) ? -1.0 : d.dm2hi, 0.0);
     }
-    if (ws_lds)
-        for (int k = tid; k <= B.nrep; k += BLOCK) s_ws[k] = B.wstart[k];
     __syncthreads();
-    const int32_t *ws = ws_lds ? s_ws : B.wstart;
-    const int W = ws[B.nrep];
-    const uint64_t step = (uint64_t)B.ctl[4], seed = (uint64_t)B.ctl[3];
     const bool nonbond = (P.flags & QNONBOND) && (P.flags & QPAR);
     int next = (blockIdx.x * WPB + wv) * (WAVE / G) + sub;
     for (;;) {
@@ -159,106 +125,132 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchParams B) {
             w = next;
             next = INT_MAX;
         }
-        if (w >= W) break;
-        // the replica of item w: the last k with wstart[k] <= w
-        int lo = 0, hi = B.nrep;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (ws[mid] <= w) lo = mid;
-            else hi = mid;
-        }
-        const int r = B.order[lo];
+        if (w >= B.nitems) break;
+        const int2 it = B.items[w];
+        const int r = it.x, t = it.y;
         const int off = B.off[r], n = B.ntot[r];
-        const int t = B.nfix[r] + (w - ws[lo]);
-        const double4 pa = B.pos[off + t];
-        const int t2 = __double2loint(pa.w);
+        if (t >= n) continue;   // no particle in this slot now
+        const double4 *const pos = B.pos + off;
+        const double4 pa = pos[t];
         const int itype = abs(B.typei[off + t]);
+        const int t2 = __double2loint(pa.w);
         const DevPair *rowp = s_rows + t2 * nt1;
         const double4 *tailp = s_tail + t2 * nt1;
-        double fx = 0.0, fy = 0.0, fz = 0.0, et = 0.0, eel = 0.0, evd = 0.0, esr = 0.0;
-        if (nonbond) {
-            for (int p = sl; p < n; p += G) {
-                if (p == t) continue;
-                const double4 q = B.pos[off + p];
-                const int tj = __double2loint(q.w);
-                const double dx = pa.x - q.x, dy = pa.y - q.y, dz = pa.z - q.z;
-                const double d2 = dx * dx + dy * dy + dz * dz;
-                // an ion pair's energy is counted by its higher-index ion (energy.mono.f90:117)
-                const bool ce = p < t;
-                double y, de;
-                if ((FEAT & BF_ANALYTIC) == 0 || (rowp[tj].flags & PF_EFPOT)) {
-                    de = pair_near_far(rowp[tj], tailp[tj], P.ep, P.ires, d2, y);
-                    et += ce ? y : 0.0;
-                } else {
-                    double q0 = 0.0, q1 = 0.0, q2 = 0.0;
-                    de = pair_analytic(rowp[tj], P, d2, q0, q1, q2);
-                    eel += ce ? q0 : 0.0;
-                    evd += ce ? q1 : 0.0;
-                    esr += ce ? q2 : 0.0;
-                }
-                fx += de * dx;
-                fy += de * dy;
-                fz += de * dz;
-            }
-        }
-        // grids: lanes 0..7 of the group take the corners (staticf1.f90:45-118,
-        // vdwgd1trln.f90:50-161)
-        double egx = 0.0, egv = 0.0;
-        bool warned = false;
+        // grid corners: lanes 0..7 of the group (staticf1.f90:45-118, vdwgd1trln.f90:50-161)
+        bool okx = false, okv = false;
+        double xx = 0.0, xy = 0.0, xz = 0.0, vx = 0.0, vy = 0.0, vz = 0.0;
+        int xi = 0, xj = 0, xk = 0, vi = 0, vj = 0, vk = 0;
+        float phx = 0.0f;
+        int8_t phv = 0;
         if constexpr ((FEAT & BF_PHIX) != 0) {
             const GridGeom &g = P.gx;
-            const bool ok = pa.x <= g.xbcen + g.tranx && pa.x >= g.xbcen - g.tranx &&
-                            pa.y <= g.ybcen + g.trany && pa.y >= g.ybcen - g.trany &&
-                            pa.z <= g.zbcen + g.tranz && pa.z >= g.zbcen - g.tranz;
-            if (ok && sl < 8) {
-                const float *phix = B.phix[r];
-                double gx_, gy_, gz_;
-                int ix, iy, iz;
-                grid_cell(g, pa.x, pa.y, pa.z, gx_, gy_, gz_, ix, iy, iz);
-                const double chi = P.cg[itype];
-                const double one1 = 1.0;
-                const int n1 = ix + (sl >> 2), n2 = iy + ((sl >> 1) & 1), n3 = iz + (sl & 1);
-                double ai = gx_ - n1 * g.dcel;
-                const double aisign = fsign(one1, ai);
-                ai = one1 - fabs(ai) * g.idcel;
-                double bi = gy_ - n2 * g.dcel;
-                const double bisign = fsign(one1, bi);
-                bi = one1 - fabs(bi) * g.idcel;
-                double ci = gz_ - n3 * g.dcel;
-                const double cisign = fsign(one1, ci);
-                ci = one1 - fabs(ci) * g.idcel;
-                const double fi = ai * bi * ci;
-                const double ph = (double)phix[((size_t)n1 * g.ny + n2) * g.nz + n3];
-                const double prefac = ph * P.celec * chi * g.idcel;
-                if (ai < (1.0 - RSMALL) && ai > RSMALL) fx += aisign * bi * ci * prefac;
-                if (bi < (1.0 - RSMALL) && bi > RSMALL) fy += bisign * ai * ci * prefac;
-                if (ci < (1.0 - RSMALL) && ci > RSMALL) fz += cisign * ai * bi * prefac;
-                egx += fi * chi * ph * P.celec;
+            okx = pa.x <= g.xbcen + g.tranx && pa.x >= g.xbcen - g.tranx &&
+                  pa.y <= g.ybcen + g.trany && pa.y >= g.ybcen - g.trany &&
+                  pa.z <= g.zbcen + g.tranz && pa.z >= g.zbcen - g.tranz;
+            if (okx && sl < 8) {
+                grid_cell(g, pa.x, pa.y, pa.z, xx, xy, xz, xi, xj, xk);
+                phx = B.phix[r][tri_node(g, xi, xj, xk, sl)];
             }
         }
         if constexpr ((FEAT & BF_PHIV) != 0) {
             const GridGeom &g = P.gv;
-            const bool ok = pa.x <= g.xbcen + g.tranx && pa.x >= g.xbcen - g.tranx &&
-                            pa.y <= g.ybcen + g.trany && pa.y >= g.ybcen - g.trany &&
-                            pa.z <= P.vzmax && pa.z >= P.vzmin;
+            okv = pa.x <= g.xbcen + g.tranx && pa.x >= g.xbcen - g.tranx &&
+                  pa.y <= g.ybcen + g.trany && pa.y >= g.ybcen - g.trany &&
+                  pa.z <= P.vzmax && pa.z >= P.vzmin;
+            if (okv && sl < 8) {
+                grid_cell(g, pa.x, pa.y, pa.z, vx, vy, vz, vi, vj, vk);
+                phv = P.phiv[tri_node(g, vi, vj, vk, sl)];
+            }
+        }
+        double gk[3] = {0.0, 0.0, 0.0};   // Gaussians of the update
+        if (B.mode == 1 && sl == 0) {
+            const double *nr = B.noise + 3 * ((size_t)B.noise_row * B.nitems + w);
+            gk[0] = nr[0]; gk[1] = nr[1]; gk[2] = nr[2];
+        }
+        double fx = 0.0, fy = 0.0, fz = 0.0, et = 0.0, eel = 0.0, evd = 0.0, esr = 0.0;
+        auto pair_loop = [&](auto en) {
+            constexpr bool EN = decltype(en)::value;
+            constexpr int PU = 2;   // one: 1.00 ms, four: 1.00 ms (registers) against 0.86
+            for (int base = sl; base < n; base += 32 * G) {
+                uint32_t m = 0u;
+                const int cnt = min(32, (n - base + G - 1) / G);
+                // PU partners per iteration: their loads and chains overlap
+#pragma unroll 1
+                for (int k0 = 0; k0 < cnt; k0 += PU) {
+                    double4 q[PU];
+#pragma unroll
+                    for (int u = 0; u < PU; u++) q[u] = pos[min(base + (k0 + u) * G, n - 1)];
+#pragma unroll
+                    for (int u = 0; u < PU; u++) {
+                        const int p = base + (k0 + u) * G;
+                        const bool on = p < n && p != t;
+                        const int tj = __double2loint(q[u].w);
+                        const double4 tl = tailp[tj];
+                        const double dx = pa.x - q[u].x, dy = pa.y - q[u].y, dz = pa.z - q[u].z;
+                        const double d2 = on ? pair_d2(dx, dy, dz) : 1e30;
+                        double f;
+                        if (ANA && tl.z < 0.0) {
+                            double q0 = 0.0, q1 = 0.0, q2 = 0.0;
+                            f = pair_analytic(rowp[tj], P, d2, q0, q1, q2);
+                            f = on ? f : 0.0;
+                            if constexpr (EN) {
+                                // an ion pair's energy is counted by its higher-index ion
+                                // (energy.mono.f90:117)
+                                const bool ce = on && p < t;
+                                eel += ce ? q0 : 0.0;
+                                evd += ce ? q1 : 0.0;
+                                esr += ce ? q2 : 0.0;
+                            }
+                        } else {
+                            const double ri = rsqrt_c3(d2), i2 = ri * ri, c = tl.x * (i2 * i2 * i2);
+                            const double fr = tl.y * ri;
+                            const bool near = d2 <= tl.z;   // false for a masked pair
+                            f = (6.0 * c + fr) * i2;
+                            f = on && !near ? f : 0.0;
+                            if constexpr (EN) et += on && !near && p < t ? c + fr : 0.0;
+                            m |= near ? 1u << (k0 + u) : 0u;
+                        }
+                        fx = fma(f, dx, fx);
+                        fy = fma(f, dy, fy);
+                        fz = fma(f, dz, fz);
+                    }
+                }
+                while (m) {   // the pairs within table range
+                    const int k = __ffs(m) - 1, p = base + k * G;
+                    m &= m - 1u;
+                    const double4 q = pos[p];
+                    const DevPair &row = rowp[__double2loint(q.w)];
+                    const double dx = pa.x - q.x, dy = pa.y - q.y, dz = pa.z - q.z;
+                    const double d2 = pair_d2(dx, dy, dz), ri = rsqrt_c3(d2);
+                    double y;
+                    const double f = pair_table(row, P.ep, P.ires, d2, ri, y);
+                    if constexpr (EN) et += p < t ? y : 0.0;
+                    fx = fma(f, dx, fx);
+                    fy = fma(f, dy, fy);
+                    fz = fma(f, dz, fz);
+                }
+            }
+        };
+        if (nonbond) {
+            if (B.write_energy) pair_loop(std::true_type{});
+            else pair_loop(std::false_type{});
+        }
+        double egx = 0.0, egv = 0.0;
+        bool warned = false;
+        if constexpr ((FEAT & BF_PHIX) != 0) {
+            if (okx && sl < 8)
+                tri_apply(P.gx, (double)phx, xx, xy, xz, xi, xj, xk, sl, P.celec * P.cg[itype], fx, fy, fz, egx);
+        }
+        if constexpr ((FEAT & BF_PHIV) != 0) {
             double ph = 0.0;
-            if (ok && sl < 8) {
-                double gx_, gy_, gz_;
-                int ix, iy, iz;
-                grid_cell(g, pa.x, pa.y, pa.z, gx_, gy_, gz_, ix, iy, iz);
+            if (okv && sl < 8) {
+                ph = (double)phv;
                 double esvdw = P.svdw;
                 if (P.flags & QSVDW) esvdw = P.svdw * P.scal[t2];
-                ph = tri_corner(g, P.phiv, gx_, gy_, gz_, ix, iy, iz, sl, esvdw, fx, fy, fz, egv);
+                tri_apply(P.gv, ph, vx, vy, vz, vi, vj, vk, sl, esvdw, fx, fy, fz, egv);
             }
-            double sum = ph;
-            sum += __shfl_xor(sum, 1, WAVE);
-            sum += __shfl_xor(sum, 2, WAVE);
-            sum += __shfl_xor(sum, 4, WAVE);
-            warned = ok && sum >= P.thold8;
+            warned = okv && half_row_sum(ph) >= P.thold8;   // integers: exact
         }
-        // Gaussians of the update: component sl on lanes 0..2 of the group
-        double gk = 0.0;
-        if (B.mode == 1 && sl < 3) gk = philox_gauss1(seed, step, (uint64_t)r, t, sl);
         fx = group_sum<G>(fx);
         fy = group_sum<G>(fy);
         fz = group_sum<G>(fz);
@@ -270,7 +262,6 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchParams B) {
             egx = group_sum<G>(egx);
             egv = group_sum<G>(egv);
         }
-        const double g1 = __shfl(gk, sub * G + 1, WAVE), g2 = __shfl(gk, sub * G + 2, WAVE);
         if (sl == 0) {
             const int64_t i = off + t;
             if (warned) atomicAdd(&B.warn[(size_t)r * B.warn_stride + t2], 1);
@@ -290,9 +281,8 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchParams B) {
                 B.fz[i] = fz;
             }
             if (B.mode == 1) {
-                const double g[3] = {gk, g1, g2};
                 const double F[3] = {fx, fy, fz};
-                B.poso[i] = bd_move(P, false, itype, pa, F, g,
+                B.poso[i] = bd_move(P, false, itype, pa, F, gk,
                                     B.nfwd + (size_t)r * B.flux_stride,
                                     B.nbwd + (size_t)r * B.flux_stride);
             }
@@ -303,7 +293,9 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchParams B) {
 template <int FEAT>
 static void launch_batch_feat(const BatchParams &q, int lanes, dim3 grid, size_t lds,
                               hipStream_t s) {
-    if (lanes == 16)
+    if (lanes == 8)
+        hipLaunchKernelGGL((k_batch_step<FEAT, 8>), grid, dim3(BLOCK), lds, s, q);
+    else if (lanes == 16)
         hipLaunchKernelGGL((k_batch_step<FEAT, 16>), grid, dim3(BLOCK), lds, s, q);
     else if (lanes == 32)
         hipLaunchKernelGGL((k_batch_step<FEAT, 32>), grid, dim3(BLOCK), lds, s, q);
@@ -316,14 +308,14 @@ hipError_t launch_batch_step(const BatchParams &b, int blocks, int lanes, hipStr
     if (b.sp.flags & QPHIX) feat |= BF_PHIX;
     if (b.sp.flags & QPHIV) feat |= BF_PHIV;
     if (!b.sp.all_efpot) feat |= BF_ANALYTIC;
-    if (lanes != 16 && lanes != 32) lanes = 64;
+    if (lanes != 8 && lanes != 16 && lanes != 32) lanes = 64;
     BatchParams q = b;
     q.persistent = blocks > 0 ? 1 : 0;
     const int per_block = WPB * (WAVE / lanes);
-    dim3 grid(blocks > 0 ? blocks : std::max(1, (b.sp.ntargets + per_block - 1) / per_block));
+    dim3 grid(blocks > 0 ? blocks : std::max(1, (b.nitems + per_block - 1) / per_block));
     const int nt1 = b.sp.nttyp + 1;
-    size_t lds = (size_t)nt1 * nt1 * (sizeof(DevPair) + sizeof(double4));
-    if (b.nrep + 1 <= BATCH_LDS_WSTART) lds += sizeof(int32_t) * (b.nrep + 1);
+    const size_t lds = (size_t)nt1 * nt1 * (sizeof(DevPair) + sizeof(double4));
+    if (q.persistent) hipLaunchKernelGGL(k_batch_queue, dim3(1), dim3(64), 0, s, q.queue);
     switch (feat) {
         case 0: launch_batch_feat<0>(q, lanes, grid, lds, s); break;
         case 1: launch_batch_feat<1>(q, lanes, grid, lds, s); break;
@@ -563,6 +555,9 @@ using namespace bromoc;
 namespace {
 
 constexpr int BATCH_GRAPH_K = 32;   // steps per captured graph without GCMC
+// steps whose noise is drawn by one launch, within a bounded buffer
+constexpr int BATCH_NOISE_ROWS = 16;
+constexpr size_t BATCH_NOISE_BYTES = size_t(256) << 20;
 
 template <typename T>
 hipError_t balloc(std::vector<void *> &al, T **p, size_t n) {
@@ -608,6 +603,7 @@ struct bromoc_batch {
     double *ered = nullptr;
     int blocks = -1;   // autotuned launch shape (0: one item per lane group, no queue)
     int lanes = 64;    // lanes per target
+    int noise_rows = 1;   // steps the noise buffer holds
     int64_t h_ctl[8] = {};
     struct Graph {
         hipGraphExec_t exec = nullptr;
@@ -652,14 +648,15 @@ void batch_energies(const double *r, bromoc_energies *out) {
     *out = E;
 }
 
-hipError_t enqueue_batch_step(bromoc_batch *b, BatchParams p, hipStream_t s) {
-    hipError_t e = launch_batch_prep(p, 0, s);
+// the counters and noise of the next n <= BATCH_NOISE_ROWS steps
+hipError_t enqueue_batch_noise(const BatchParams &p, int n, hipStream_t s) {
+    hipError_t e = launch_batch_prep(p, 0, n, s);
     if (e != hipSuccess) return e;
-    return launch_batch_step(p, b->blocks, b->lanes, s);
+    return launch_batch_noise(p, n, s);
 }
 
 hipError_t enqueue_batch_gcmc(const BatchParams &p, hipStream_t s) {
-    hipError_t e = launch_batch_prep(p, 1, s);
+    hipError_t e = launch_batch_prep(p, 1, 0, s);
     if (e != hipSuccess) return e;
     return launch_batch_gcmc(p, s);
 }
@@ -670,52 +667,49 @@ int batch_sync(bromoc_batch *b) {
     return BROMOC_OK;
 }
 
-// Autotuner: 16, 32 or 64 lanes per target, and a persistent queue with 2 or 8
-// workgroups per CU or one work item per lane group; timed on ENERGY-only launches whose
-// warnings go to a scratch counter.  BROMOC_BATCH_BLOCKS and BROMOC_BATCH_LANES force a
-// shape (blocks 0: one item per lane group).
+// Autotuner: 8, 16, 32 or 64 lanes per target, one work item per lane group, timed on
+// ENERGY-only launches whose warnings go to a scratch counter, the best of two rounds (the first
+// launches of a process run slow).  The queue is not among the candidates: its persistent
+// workgroups take twice the time (256 replicas of 100..4000 ions 2.0 ms against 0.86, of 200
+// ions 200 us against 53), since the hardware hands out blocks in the same largest-first order.
+// BROMOC_BATCH_BLOCKS and BROMOC_BATCH_LANES force a shape (blocks 0: no queue).
 int batch_autotune(bromoc_batch *b) {
     if (b->blocks >= 0) return BROMOC_OK;
     const char *eb = std::getenv("BROMOC_BATCH_BLOCKS"), *el = std::getenv("BROMOC_BATCH_LANES");
     if (eb || el) {
         b->blocks = eb ? std::max(0, std::atoi(eb)) : 0;
         b->lanes = el ? std::atoi(el) : 64;
-        if (b->lanes != 16 && b->lanes != 32) b->lanes = 64;
+        if (b->lanes != 8 && b->lanes != 16 && b->lanes != 32) b->lanes = 64;
         return BROMOC_OK;
     }
-    hipDeviceProp_t prop;
-    BCHK(b, hipGetDeviceProperties(&prop, b->device));
-    const int ncu = prop.multiProcessorCount;
-    const int cb[3] = {0, 2 * ncu, 8 * ncu}, cl[3] = {16, 32, 64};
+    const int cl[4] = {8, 16, 32, 64};
     hipEvent_t e0, e1;
     BCHK(b, hipEventCreate(&e0));
     BCHK(b, hipEventCreate(&e1));
     double best = 1e300;
-    int pick_b = 0, pick_l = 64;
-    for (int l : cl) {
-        for (int c : cb) {
-            b->blocks = c;
-            b->lanes = l;
+    int pick = 64;
+    for (int round = 0; round < 2; round++) {
+        for (int l : cl) {
             BatchParams p = params_now(b);
             p.mode = 0;
             p.write_energy = 0;
             p.write_forces = 0;
             p.warn = b->warn_scratch;
-            for (int r = 0; r < 2; r++) BCHK(b, enqueue_batch_step(b, p, b->stream));
+            BCHK(b, launch_batch_step(p, 0, l, b->stream));
             BCHK(b, hipEventRecord(e0, b->stream));
-            for (int r = 0; r < 4; r++) BCHK(b, enqueue_batch_step(b, p, b->stream));
+            for (int r = 0; r < 3; r++) BCHK(b, launch_batch_step(p, 0, l, b->stream));
             BCHK(b, hipEventRecord(e1, b->stream));
             int st = batch_sync(b);
             if (st) return st;
             float ms = 0.f;
             BCHK(b, hipEventElapsedTime(&ms, e0, e1));
-            if (ms < best) { best = ms; pick_b = c; pick_l = l; }
+            if (ms < best) { best = ms; pick = l; }
         }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    b->blocks = pick_b;
-    b->lanes = pick_l;
+    b->blocks = 0;
+    b->lanes = pick;
     return BROMOC_OK;
 }
 
@@ -865,12 +859,24 @@ int bromoc_batch_create(const bromoc_system *s, int32_t nrep, const bromoc_repli
     for (int r = 0; r < nrep; r++) B.sp.ntargets += reps[r].capacity - reps[r].nfix;
     B.nrep = nrep;
     int32_t *d_i = nullptr;
-    ACHK(bupload(al, &d_i, order.data(), nrep)); B.order = d_i;
+    // the work items: every slot that can hold a moving ion, replicas by decreasing capacity
+    {
+        std::vector<int2> items;
+        items.reserve(B.sp.ntargets);
+        for (int r : order)
+            for (int t = reps[r].nfix; t < reps[r].capacity; t++) items.push_back(make_int2(r, t));
+        int2 *d_it = nullptr;
+        ACHK(bupload(al, &d_it, items.data(), items.size()));
+        B.items = d_it;
+        B.nitems = (int)items.size();
+        const size_t row = 3 * sizeof(double) * std::max<size_t>(items.size(), 1);
+        b->noise_rows = (int)std::min<size_t>(BATCH_NOISE_ROWS, std::max<size_t>(1, BATCH_NOISE_BYTES / row));
+        ACHK(balloc(al, &B.noise, b->noise_rows * 3 * std::max<size_t>(items.size(), 1)));
+    }
     ACHK(bupload(al, &d_i, b->h_off.data(), nrep)); B.off = d_i;
     ACHK(bupload(al, &d_i, b->h_cap.data(), nrep)); B.cap = d_i;
     ACHK(bupload(al, &d_i, b->h_nfix.data(), nrep)); B.nfix = d_i;
     ACHK(bupload(al, &B.ntot, ntot.data(), nrep));
-    ACHK(balloc(al, &B.wstart, nrep + 1));
     ACHK(balloc(al, &B.queue, 2));
     ACHK(bupload(al, &B.typei, ty.data(), total));
     ACHK(bupload(al, &B.ibuffer, ibuf.data(), total));
@@ -974,10 +980,13 @@ int bromoc_batch_run(bromoc_batch *b, int32_t nsteps, uint64_t seed, uint64_t co
         for (int k = 0; k < nst; k++) {
             BatchParams p = params_now(b);
             p.mode = 1;
+            p.noise_row = k % b->noise_rows;
+            if (p.noise_row == 0)
+                BCHK(b, enqueue_batch_noise(p, std::min(b->noise_rows, nst - k), b->stream));
             const bool wr = last_energy && k == nst - 1;
             p.write_energy = wr ? 1 : 0;
             p.write_forces = wr ? 1 : 0;
-            BCHK(b, enqueue_batch_step(b, p, b->stream));
+            BCHK(b, launch_batch_step(p, b->blocks, b->lanes, b->stream));
             b->cur ^= 1;
         }
         return BROMOC_OK;
@@ -1044,7 +1053,7 @@ int bromoc_batch_energy(bromoc_batch *b, bromoc_energies *energies) {
     p.mode = 0;
     p.write_energy = 1;
     p.write_forces = 1;
-    BCHK(b, enqueue_batch_step(b, p, b->stream));
+    BCHK(b, launch_batch_step(p, b->blocks, b->lanes, b->stream));
     BCHK(b, launch_batch_reduce(p, b->ered, b->stream));
     std::vector<double> r((size_t)b->nrep * NE);
     BCHK(b, hipMemcpyAsync(r.data(), b->ered, r.size() * sizeof(double), hipMemcpyDeviceToHost, b->stream));
@@ -1129,7 +1138,8 @@ int bromoc_batch_time_steps(bromoc_batch *b, int32_t nsteps, uint64_t seed, uint
     for (int k = 0; k < nsteps; k++) {
         BatchParams p = params_now(b);
         p.mode = 1;
-        BCHK(b, launch_batch_prep(p, 0, b->stream));
+        p.noise_row = 0;
+        BCHK(b, enqueue_batch_noise(p, 1, b->stream));
         BCHK(b, hipEventRecord(ev[2 * k], b->stream));
         BCHK(b, launch_batch_step(p, b->blocks, b->lanes, b->stream));
         BCHK(b, hipEventRecord(ev[2 * k + 1], b->stream));

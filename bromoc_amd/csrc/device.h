@@ -58,6 +58,18 @@ __device__ __forceinline__ double wave_last(double v) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), WAVE - 1),
                             __builtin_amdgcn_readlane(__double2loint(v), WAVE - 1));
 }
+// sums over each 8 and each row of 16 lanes, on every lane of them
+__device__ __forceinline__ double half_row_sum(double v) {
+    v += dpp<0xB1>(v, v);    // quad_perm [1,0,3,2]
+    v += dpp<0x4E>(v, v);    // quad_perm [2,3,0,1]
+    v += dpp<0x141>(v, v);   // row_half_mirror
+    return v;
+}
+__device__ __forceinline__ double row_sum(double v) {
+    v = half_row_sum(v);
+    v += dpp<0x140>(v, v);   // row_mirror
+    return v;
+}
 // a value that is the same on every lane, in scalar registers
 __device__ __forceinline__ double wave_uniform(double v) {
     return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
@@ -219,13 +231,15 @@ __device__ __forceinline__ void fixcoor(const StepParams &P, double &x, double &
     else if (z > P.lz2p) z = P.lz2p;
 }
 
-// One trilinear corner (lane c = 0..7) of staticf1/vdwgd1trln.  Adds the corner's force
-// and energy to the lane's accumulators; returns the corner's grid value.
-template <typename T>
-__device__ __forceinline__ double tri_corner(const GridGeom &g, const T *__restrict__ data,
-                                             double xi, double yi, double zi, int ix, int iy,
-                                             int iz, int c, double scale, double &fx, double &fy,
-                                             double &fz, double &e) {
+// Node of trilinear corner c = 0..7 of a cell, and the corner's share (staticf1/vdwgd1trln)
+// given its grid value ph: force and energy added to the lane's accumulators.  In two parts, so
+// that a kernel can load its corners early and use them late.
+__device__ __forceinline__ size_t tri_node(const GridGeom &g, int ix, int iy, int iz, int c) {
+    return ((size_t)(ix + (c >> 2)) * g.ny + (iy + ((c >> 1) & 1))) * g.nz + (iz + (c & 1));
+}
+__device__ __forceinline__ void tri_apply(const GridGeom &g, double ph, double xi, double yi,
+                                          double zi, int ix, int iy, int iz, int c, double scale,
+                                          double &fx, double &fy, double &fz, double &e) {
     const double one = 1.0;
     int n1 = ix + (c >> 2), n2 = iy + ((c >> 1) & 1), n3 = iz + (c & 1);
     double ai = xi - n1 * g.dcel;
@@ -238,13 +252,21 @@ __device__ __forceinline__ double tri_corner(const GridGeom &g, const T *__restr
     double cisign = fsign(one, ci);
     ci = one - fabs(ci) * g.idcel;
     double fi = ai * bi * ci;
-    size_t in3 = ((size_t)n1 * g.ny + n2) * g.nz + n3;
-    double ph = (double)data[in3];
     double prefac = ph * scale * g.idcel;
     if (ai < (1.0 - RSMALL) && ai > RSMALL) fx += aisign * bi * ci * prefac;
     if (bi < (1.0 - RSMALL) && bi > RSMALL) fy += bisign * ai * ci * prefac;
     if (ci < (1.0 - RSMALL) && ci > RSMALL) fz += cisign * ai * bi * prefac;
     e += fi * scale * ph;
+}
+
+// Both at once.  Returns the corner's grid value.
+template <typename T>
+__device__ __forceinline__ double tri_corner(const GridGeom &g, const T *__restrict__ data,
+                                             double xi, double yi, double zi, int ix, int iy,
+                                             int iz, int c, double scale, double &fx, double &fy,
+                                             double &fz, double &e) {
+    const double ph = (double)data[tri_node(g, ix, iy, iz, c)];
+    tri_apply(g, ph, xi, yi, zi, ix, iy, iz, c, scale, fx, fy, fz, e);
     return ph;
 }
 

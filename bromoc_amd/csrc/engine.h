@@ -471,10 +471,11 @@ struct BatchParams {
     int32_t nrep, persistent;   // replicas; 1: waves take items from queue[0]
     int32_t mode, write_energy; // mode 1: BD step, 0: ENERGY only
     int32_t write_forces, ngcmc;
-    const int32_t *order;       // [nrep] replicas by decreasing capacity
+    const int2 *items;          // [nitems] (replica, slot) of every slot for a moving ion
+    int32_t nitems, noise_row;  // noise_row: this step's row of noise
+    double *noise;              // [rows][nitems][3] Gaussians (k_batch_noise)
     const int32_t *off, *cap, *nfix;   // [nrep] first slot, slots, leading fixed ions
     int32_t *ntot;              // [nrep] particles now (GRAND changes it)
-    int32_t *wstart;            // [nrep+1] work-item prefix over `order` (k_batch_prep)
     int32_t *queue;             // [2] work counter, error flag
     const float *const *phix;   // [nrep] static field of each replica
     const double4 *pos;         // [slots] (x, y, z, atnam2 type in the low word)
@@ -499,7 +500,8 @@ struct BatchParams {
     int64_t *ctl;               // [8]: steps, counter0, cycles, seed, step counter, cycle,
                                 //      cycle0, spare
 };
-hipError_t launch_batch_prep(const BatchParams &b, int gcmc, hipStream_t s);
+hipError_t launch_batch_prep(const BatchParams &b, int gcmc, int steps, hipStream_t s);
+hipError_t launch_batch_noise(const BatchParams &b, int steps, hipStream_t s);
 hipError_t launch_batch_step(const BatchParams &b, int blocks, int lanes, hipStream_t s);
 hipError_t launch_batch_gcmc(const BatchParams &b, hipStream_t s);
 hipError_t launch_batch_reduce(const BatchParams &b, double *out, hipStream_t s);
