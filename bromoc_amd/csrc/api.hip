@@ -123,7 +123,6 @@ struct bromoc_ctx {
     void *pin = nullptr;               // pinned staging of a call's small copies
     size_t pin_cap = 0;
     double4 h_move{};                  // staging of one particle moved by GRAND
-    double *iout = nullptr;
     std::vector<void *> allocs;
     // host mirrors
     std::vector<int32_t> h_typei, h_nwtype, h_typtyp;
@@ -145,7 +144,6 @@ struct bromoc_ctx {
         int32_t *ibfftyp = nullptr, *ntotat = nullptr, *nat = nullptr;
         int32_t *natlog = nullptr;        // [lcap] buffer counts after each attempt
         int64_t lcap = 0;
-        std::vector<int32_t> h_natlog;
         int32_t *ibuffer = nullptr;
         bool ib_current = false;          // ibuffer equals the host's copy
         int8_t *bias = nullptr;
@@ -523,10 +521,11 @@ int ensure_sorted(bromoc_ctx *c, bool force = false) {
     return ensure_sorted(c, force, tile_mode(c->tpb) ? c->tpb - TPB_TILE : 0);
 }
 
-// Pinned host staging for a call's small copies (the step loop's control words, GRAND's
-// uniforms, counts and state): from pageable memory each such copy is a slow staged
-// transfer that leaves the GPU idle between calls.  Every call synchronises before it
-// returns, so the next call may reuse or regrow the buffer.
+// Pinned host staging for a call's transfers (the step loop's control words, positions,
+// forces, energies, GRAND's uniforms, counts and state): from pageable memory each such copy
+// is a slow staged transfer that leaves the GPU idle between calls.  Every call synchronises
+// before it returns, so the next call may reuse or regrow the buffer.
+constexpr size_t PIN_MIN = 4096, PIN_ENER = 2048, PIN_INTER = 3072;
 static unsigned char *pinned(bromoc_ctx *c, size_t bytes) {
     if (bytes > c->pin_cap) {
         if (c->pin) (void)hipHostFree(c->pin);
@@ -547,10 +546,11 @@ int sync_err(bromoc_ctx *c) {
 int reduce_energies(bromoc_ctx *c, bromoc_energies *out) {
     const StepParams p = params_for(c);
     const bool tiles = tile_mode(p.tpb);
-    HIPCHK(c, launch_reduce_energy(c->epart, c->cap, c->ntot, c->ered, c->stream,
+    unsigned char *pin = pinned(c, PIN_MIN);
+    if (!pin) return fail(c, BROMOC_E_HIP, "pinned staging");
+    double *r = (double *)(pin + PIN_ENER);   // apart from the step loop's control words
+    HIPCHK(c, launch_reduce_energy(c->epart, c->cap, c->ntot, c->ered, r, c->stream,
                                    tiles ? c->tener : nullptr, tiles ? p.titems : 0));
-    double r[NE];
-    HIPCHK(c, hipMemcpyAsync(r, c->ered, sizeof(r), hipMemcpyDeviceToHost, c->stream));
     int st = sync_err(c);
     if (st) return st;
     energies_from(r, (c->sys.flags & BROMOC_QRFPAR) != 0, (c->sys.flags & BROMOC_QMMIJ) != 0, out);
@@ -696,7 +696,10 @@ int bromoc_create(const bromoc_system *s, int device, bromoc_ctx **out) {
     ACHK(dalloc(c, &c->fz, cap));
     ACHK(dalloc(c, &c->fdna, std::max(ns, 1)));
     ACHK(dalloc(c, &c->epart, (size_t)NE * cap));
-    ACHK(dalloc(c, &c->ered, (size_t)NE * (1 + 2 * RED_BLOCKS)));
+    ACHK(dalloc(c, &c->ered, (size_t)NE * 2 * RED_BLOCKS));
+    // enough for a call's transfers at usual sizes; `pinned` grows it for larger ones
+    if (!pinned(c, std::max(PIN_MIN, std::min<size_t>((size_t)cap * 32, 1 << 20))))
+        return cleanup(BROMOC_E_HIP);
     ACHK(dupload(c, &c->pairidx, s->pairidx, (size_t)nt1 * nt1));
     c->h_pairs.assign(s->pairs, s->pairs + s->npair + 1);
     c->h_pairidx.assign(s->pairidx, s->pairidx + (size_t)nt1 * nt1);
@@ -865,7 +868,6 @@ int bromoc_create(const bromoc_system *s, int device, bromoc_ctx **out) {
                  std::max(0, s->cntpts)));
     ACHK(dalloc(c, &c->ctl, 4));
     ACHK(dalloc(c, &c->pbuf, (size_t)GRAPH_K * 3 * cap));
-    ACHK(dalloc(c, &c->iout, 2));
     // position-dependent diffusion (DYNAMICS1 / DYNAMICS2)
     const bool dyn12 = (s->flags & (BROMOC_QDIFFUSE | BROMOC_QPROFILE)) != 0;
     const int nsp = (s->flags & BROMOC_QPROFILE) ? s->nspline : 0;
@@ -1040,7 +1042,6 @@ int bromoc_set_positions(bromoc_ctx *c, int32_t ntot, const double *x, const dou
     if (ntot < c->ns + c->nf || ntot > c->cap) return fail(c, BROMOC_E_ARG, "ntot out of range");
     (void)hipSetDevice(c->device);
     c->gd.ib_current = false;   // the particle count may change: upload ibuffer again
-    std::vector<int32_t> t2(ntot);
     if (typei) {
         for (int i = c->ns; i < ntot; i++) {
             int t = std::abs(typei[i]);
@@ -1052,14 +1053,18 @@ int bromoc_set_positions(bromoc_ctx *c, int32_t ntot, const double *x, const dou
     } else if (ntot > c->ntot) {
         return fail(c, BROMOC_E_ARG, "typei required when ntot grows");
     }
+    const size_t n = ntot;
+    double *px = (double *)pinned(c, std::max(PIN_MIN, n * (3 * sizeof(double) + 2 * sizeof(int32_t))));
+    if (!px) return fail(c, BROMOC_E_HIP, "pinned staging");
+    double *py = px + n, *pz = py + n;
+    int32_t *pt = (int32_t *)(pz + n), *pty = pt + n;
+    std::copy(x, x + n, px);
+    std::copy(y, y + n, py);
+    std::copy(z, z + n, pz);
     for (int i = 0; i < ntot; i++)
-        t2[i] = i < c->ns ? c->h_typtyp[i] : c->h_nwtype[std::abs(c->h_typei[i])];
-    std::vector<double4> p4(ntot);
-    for (int i = 0; i < ntot; i++) p4[i] = make_double4(x[i], y[i], z[i], pack_type(t2[i], i));
-    for (int b = 0; b < 2; b++)
-        HIPCHK(c, hipMemcpyAsync(c->pos[b], p4.data(), sizeof(double4) * ntot, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->typei, c->h_typei.data(), sizeof(int32_t) * ntot, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->t2, t2.data(), sizeof(int32_t) * ntot, hipMemcpyHostToDevice, c->stream));
+        pt[i] = i < c->ns ? c->h_typtyp[i] : c->h_nwtype[std::abs(c->h_typei[i])];
+    std::copy(c->h_typei.begin(), c->h_typei.begin() + n, pty);
+    HIPCHK(c, launch_stage_pos_in(px, py, pz, pt, pty, ntot, c->pos[0], c->pos[1], c->t2, c->typei, c->stream));
     int st = sync_err(c);
     c->ntot = ntot;
     c->sort_dirty = true;
@@ -1073,14 +1078,13 @@ int bromoc_get_positions(bromoc_ctx *c, double *x, double *y, double *z, int32_t
     const size_t n = c->ntot;
     int st = BROMOC_OK;
     if (x || y || z) {
-        std::vector<double4> p4(n);
-        HIPCHK(c, hipMemcpyAsync(p4.data(), c->pos[c->cur], sizeof(double4) * n, hipMemcpyDeviceToHost, c->stream));
+        double *p = (double *)pinned(c, std::max(PIN_MIN, 3 * sizeof(double) * n));
+        if (!p) return fail(c, BROMOC_E_HIP, "pinned staging");
+        HIPCHK(c, launch_stage_pos_out(c->pos[c->cur], c->ntot, p, p + n, p + 2 * n, c->stream));
         st = sync_err(c);
-        for (size_t i = 0; i < n; i++) {
-            if (x) x[i] = p4[i].x;
-            if (y) y[i] = p4[i].y;
-            if (z) z[i] = p4[i].z;
-        }
+        if (x) std::copy(p, p + n, x);
+        if (y) std::copy(p + n, p + 2 * n, y);
+        if (z) std::copy(p + 2 * n, p + 3 * n, z);
     }
     if (typei) std::memcpy(typei, c->h_typei.data(), sizeof(int32_t) * n);
     if (ntot) *ntot = c->ntot;
@@ -1091,10 +1095,19 @@ int bromoc_get_forces(bromoc_ctx *c, double *fx, double *fy, double *fz) {
     if (!c || !fx || !fy || !fz) return BROMOC_E_ARG;
     (void)hipSetDevice(c->device);
     const size_t n = c->ntot;
-    HIPCHK(c, hipMemcpyAsync(fx, c->fx, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(fy, c->fy, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(fz, c->fz, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-    return sync_err(c);
+    double *p = (double *)pinned(c, std::max(PIN_MIN, 3 * sizeof(double) * n));
+    if (!p) return fail(c, BROMOC_E_HIP, "pinned staging");
+    StageCopies q{};
+    q.add(p, c->fx, sizeof(double) * n);
+    q.add(p + n, c->fy, sizeof(double) * n);
+    q.add(p + 2 * n, c->fz, sizeof(double) * n);
+    HIPCHK(c, launch_stage_copy(q, c->stream));
+    int st = sync_err(c);
+    if (st) return st;
+    std::copy(p, p + n, fx);
+    std::copy(p + n, p + 2 * n, fy);
+    std::copy(p + 2 * n, p + 3 * n, fz);
+    return BROMOC_OK;
 }
 
 int bromoc_energy(bromoc_ctx *c, int32_t want_forces, bromoc_energies *out) {
@@ -1285,7 +1298,7 @@ static int run_steps(bromoc_ctx *c, int32_t nsteps, int32_t noise_mode, int32_t 
     int st0 = autotune(c);
     if (st0) return st0;
     c->h_ctl[0] = 0; c->h_ctl[1] = first_row; c->h_ctl[2] = (int64_t)counter0; c->h_ctl[3] = (int64_t)seed;
-    int64_t *hc = (int64_t *)pinned(c, 4096);
+    int64_t *hc = (int64_t *)pinned(c, PIN_MIN);
     if (!hc) return fail(c, BROMOC_E_HIP, "pinned staging");
     std::memcpy(hc, c->h_ctl, sizeof(c->h_ctl));
     HIPCHK(c, hipMemcpyAsync(c->ctl, hc, sizeof(c->h_ctl), hipMemcpyHostToDevice, c->stream));
@@ -1606,7 +1619,9 @@ static int interact_async(bromoc_ctx *c, double xj, double yj, double zj, int32_
     q.sp = params_for(c);
     q.xj = xj; q.yj = yj; q.zj = zj;
     q.jtype = jtype; q.j = j; q.alert = alert;
-    q.out = c->iout + slot;
+    unsigned char *pin = pinned(c, PIN_MIN);
+    if (!pin) return fail(c, BROMOC_E_HIP, "pinned staging");
+    q.out = (double *)(pin + PIN_INTER) + slot;
     HIPCHK(c, launch_rfpar(q.sp, false, c->stream));
     HIPCHK(c, launch_interact(q, c->stream));
     HIPCHK(c, launch_mmij_interact(q.sp, xj, yj, zj, jtype, j, q.out, c->stream));
@@ -1619,8 +1634,9 @@ int bromoc_interact(bromoc_ctx *c, double xj, double yj, double zj, int32_t jtyp
     (void)hipSetDevice(c->device);
     int st = interact_async(c, xj, yj, zj, jtype, j, alert);
     if (st) return st;
-    HIPCHK(c, hipMemcpyAsync(dener, c->iout, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    return sync_err(c);
+    st = sync_err(c);
+    *dener = *(const double *)((unsigned char *)c->pin + PIN_INTER);
+    return st;
 }
 
 int bromoc_set_gcmc(bromoc_ctx *c, const bromoc_gcmc *g) {
@@ -1727,26 +1743,31 @@ static int grand_device(bromoc_ctx *c, int32_t ngcmc, const double *u, int64_t n
         D.lcap = nlog;
     }
     const int n0 = c->ntot;
-    // pinned staging: uniforms, nat and the state up; the state, nat and the log back
+    // pinned staging: uniforms, nat, the state (and ibuffer) up in one launch; the state, nat,
+    // the log, ibuffer and the types back in another
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const int nmax = (int)std::min<int64_t>(c->cap, (int64_t)n0 + ngcmc);   // an attempt adds at most one
     const size_t o_nat = al(sizeof(double) * nu), o_st = o_nat + al(sizeof(int32_t) * (nb + 1));
-    const size_t o_st2 = o_st + al(sizeof(GcState)), o_nat2 = o_st2 + al(sizeof(GcState));
-    const size_t o_log = o_nat2 + al(sizeof(int32_t) * (nb + 1));
-    unsigned char *pin = pinned(c, o_log + sizeof(int32_t) * (size_t)nlog);
+    const size_t o_ib = o_st + al(sizeof(GcState)), o_st2 = o_ib + al(sizeof(int32_t) * (size_t)n0);
+    const size_t o_nat2 = o_st2 + al(sizeof(GcState)), o_log = o_nat2 + al(sizeof(int32_t) * (nb + 1));
+    const size_t o_ib2 = o_log + al(sizeof(int32_t) * (size_t)nlog), o_ty2 = o_ib2 + al(sizeof(int32_t) * (size_t)nmax);
+    unsigned char *pin = pinned(c, std::max(PIN_MIN, o_ty2 + sizeof(int32_t) * (size_t)nmax));
     if (!pin) return fail(c, BROMOC_E_HIP, "pinned staging");
-    if (nu > 0) {
-        std::memcpy(pin, u, sizeof(double) * nu);
-        HIPCHK(c, hipMemcpyAsync(D.u, pin, sizeof(double) * nu, hipMemcpyHostToDevice, c->stream));
-    }
+    if (nu > 0) std::memcpy(pin, u, sizeof(double) * nu);
     std::memcpy(pin + o_nat, nat, sizeof(int32_t) * (nb + 1));
-    HIPCHK(c, hipMemcpyAsync(D.nat, pin + o_nat, sizeof(int32_t) * (nb + 1), hipMemcpyHostToDevice, c->stream));
-    // the device's ibuffer is the host's unless the host changed it since the last call
-    if (!D.ib_current)
-        HIPCHK(c, hipMemcpyAsync(D.ibuffer, c->ibuffer.data(), sizeof(int32_t) * n0, hipMemcpyHostToDevice, c->stream));
     GcState h{};
     h.k = 0; h.ntot = n0; h.err = GCE_OK; h.ener = *ener;
     std::memcpy(pin + o_st, &h, sizeof(h));
-    HIPCHK(c, hipMemcpyAsync(D.st, pin + o_st, sizeof(h), hipMemcpyHostToDevice, c->stream));
+    StageCopies up{};
+    up.add(D.u, pin, sizeof(double) * nu);
+    up.add(D.nat, pin + o_nat, sizeof(int32_t) * (nb + 1));
+    up.add(D.st, pin + o_st, sizeof(h));
+    // the device's ibuffer is the host's unless the host changed it since the last call
+    if (!D.ib_current) {
+        std::memcpy(pin + o_ib, c->ibuffer.data(), sizeof(int32_t) * n0);
+        up.add(D.ibuffer, pin + o_ib, sizeof(int32_t) * n0);
+    }
+    HIPCHK(c, launch_stage_copy(up, c->stream));
     GcParams G{};
     G.sp = params_for(c);
     G.pos0 = c->pos[0]; G.pos1 = c->pos[1];
@@ -1762,28 +1783,26 @@ static int grand_device(bromoc_ctx *c, int32_t ngcmc, const double *u, int64_t n
     G.cap = c->cap;
     G.st = D.st; G.part = D.part;
     HIPCHK(c, launch_grand(G, ngcmc, c->stream));
-    HIPCHK(c, hipMemcpyAsync(pin + o_st2, D.st, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+    StageCopies down{};
+    down.add(pin + o_st2, D.st, sizeof(h));
+    down.add(pin + o_nat2, D.nat, sizeof(int32_t) * (nb + 1));
+    down.add(pin + o_log, D.natlog, sizeof(int32_t) * (size_t)nlog);
+    down.add(pin + o_ib2, D.ibuffer, sizeof(int32_t) * (size_t)nmax);
+    down.add(pin + o_ty2, c->typei, sizeof(int32_t) * (size_t)nmax);
+    HIPCHK(c, launch_stage_copy(down, c->stream));
     int st = sync_err(c);
     if (st) return st;
     std::memcpy(&h, pin + o_st2, sizeof(h));
     const int n1 = h.ntot;
-    HIPCHK(c, hipMemcpyAsync(pin + o_nat2, D.nat, sizeof(int32_t) * (nb + 1), hipMemcpyDeviceToHost, c->stream));
-    D.h_natlog.resize((size_t)nlog);
-    if (nb > 0 && h.natt > 0)
-        HIPCHK(c, hipMemcpyAsync(pin + o_log, D.natlog, sizeof(int32_t) * (size_t)h.natt * nb,
-                                 hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->ibuffer.data(), D.ibuffer, sizeof(int32_t) * n1, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->h_typei.data(), c->typei, sizeof(int32_t) * n1, hipMemcpyDeviceToHost, c->stream));
-    st = sync_err(c);
-    if (st) return st;
+    std::memcpy(c->ibuffer.data(), pin + o_ib2, sizeof(int32_t) * (size_t)n1);
+    std::memcpy(c->h_typei.data(), pin + o_ty2, sizeof(int32_t) * (size_t)n1);
     std::memcpy(nat, pin + o_nat2, sizeof(int32_t) * (nb + 1));
-    if (nb > 0 && h.natt > 0)
-        std::memcpy(D.h_natlog.data(), pin + o_log, sizeof(int32_t) * (size_t)h.natt * nb);
+    const int32_t *natlog = (const int32_t *)(pin + o_log);
     D.ib_current = true;
     // prob(b, count) += 1 for every logged count, attempt by attempt
     for (int a = 0; a < h.natt; a++)
         for (int b = 1; b <= nb; b++)
-            prob[(size_t)(b - 1) * pstride + D.h_natlog[(size_t)a * nb + (b - 1)]] += 1;
+            prob[(size_t)(b - 1) * pstride + natlog[(size_t)a * nb + (b - 1)]] += 1;
     if (h.nacc > 0) c->sort_dirty = true;
     c->ntot = n1;
     *ener = h.ener;
@@ -1978,9 +1997,8 @@ int bromoc_metropolis(bromoc_ctx *c, int32_t nmcm, double mcmax, double ikbt,
         const double4 pa = hp[iat];
         if ((st = interact_async(c, pa.x, pa.y, pa.z, jt, iat, 1, 0))) return st;
         if ((st = interact_async(c, xn, yn, zn, jt, iat, 0, 1))) return st;
-        double eo[2];
-        HIPCHK(c, hipMemcpyAsync(eo, c->iout, sizeof(eo), hipMemcpyDeviceToHost, c->stream));
         if ((st = sync_err(c))) return st;
+        const double *eo = (const double *)((unsigned char *)c->pin + PIN_INTER);
         const double eold = eo[0], enew = eo[1];
         bool acc = enew <= eold;
         if (!acc) {

@@ -604,6 +604,8 @@ struct bromoc_batch {
     int blocks = -1;   // autotuned launch shape (0: one item per lane group, no queue)
     int lanes = 64;    // lanes per target
     int noise_rows = 1;   // steps the noise buffer holds
+    void *pin = nullptr;  // pinned staging of bromoc_batch_get
+    size_t pin_cap = 0;
     int64_t h_ctl[8] = {};
     struct Graph {
         hipGraphExec_t exec = nullptr;
@@ -734,6 +736,7 @@ int bromoc_batch_destroy(bromoc_batch *b) {
     for (auto &g : b->graph)
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
     for (void *p : b->allocs) (void)hipFree(p);
+    if (b->pin) (void)hipHostFree(b->pin);
     if (b->shared) bromoc_destroy(b->shared);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
@@ -1067,27 +1070,43 @@ int bromoc_batch_get(bromoc_batch *b, int32_t r, double *x, double *y, double *z
                      int32_t *ntot, int32_t *ibuffer, int32_t *nat, double *gcmc_ener) {
     if (!b || r < 0 || r >= b->nrep) return BROMOC_E_ARG;
     (void)hipSetDevice(b->device);
-    int32_t n = 0;
-    BCHK(b, hipMemcpy(&n, b->base.ntot + r, sizeof(n), hipMemcpyDeviceToHost));
-    const int64_t off = b->h_off[r];
-    if (x || y || z) {
-        std::vector<double4> p4(std::max(n, 1));
-        if (n) BCHK(b, hipMemcpy(p4.data(), b->pos[b->cur] + off, sizeof(double4) * n, hipMemcpyDeviceToHost));
-        for (int i = 0; i < n; i++) {
-            if (x) x[i] = p4[i].x;
-            if (y) y[i] = p4[i].y;
-            if (z) z[i] = p4[i].z;
-        }
+    // everything in one launch through pinned memory, laid out by the replica's capacity
+    const size_t cap = b->h_cap[r], nb = b->h_nbuf[r];
+    const size_t bytes = sizeof(double) * (3 * cap + 1) + sizeof(int32_t) * (2 * cap + nb + 1);
+    if (bytes > b->pin_cap) {
+        if (b->pin) (void)hipHostFree(b->pin);
+        b->pin = nullptr;
+        b->pin_cap = 0;
+        BCHK(b, hipHostMalloc(&b->pin, bytes));
+        b->pin_cap = bytes;
     }
-    if (typei && n) BCHK(b, hipMemcpy(typei, b->base.typei + off, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-    if (ibuffer && n) BCHK(b, hipMemcpy(ibuffer, b->base.ibuffer + off, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    StageReplica a{};
+    const BatchParams &B = b->base;
+    a.r = r;
+    a.nbuf = (int32_t)nb;
+    a.ntot = B.ntot; a.off = B.off;
+    a.pos = b->pos[b->cur];
+    a.typei = B.typei; a.ibuffer = B.ibuffer;
+    a.nat = B.nat + (size_t)r * b->gstride + 1;
+    a.gener = B.gener;
+    a.o_ener = (double *)b->pin;
+    a.o_x = a.o_ener + 1; a.o_y = a.o_x + cap; a.o_z = a.o_y + cap;
+    a.o_n = (int32_t *)(a.o_z + cap);
+    a.o_nat = a.o_n + 1; a.o_ty = a.o_nat + nb; a.o_ib = a.o_ty + cap;
+    BCHK(b, launch_stage_replica(a, (int)cap, b->stream));
+    int st = batch_sync(b);
+    if (st) return st;
+    const int32_t n = a.o_n[0];
+    if (x) std::copy(a.o_x, a.o_x + n, x);
+    if (y) std::copy(a.o_y, a.o_y + n, y);
+    if (z) std::copy(a.o_z, a.o_z + n, z);
+    if (typei) std::copy(a.o_ty, a.o_ty + n, typei);
+    if (ibuffer) std::copy(a.o_ib, a.o_ib + n, ibuffer);
     if (nat) {
         nat[0] = 0;
-        if (b->h_nbuf[r] > 0)
-            BCHK(b, hipMemcpy(nat + 1, b->base.nat + (size_t)r * b->gstride + 1,
-                              sizeof(int32_t) * b->h_nbuf[r], hipMemcpyDeviceToHost));
+        std::copy(a.o_nat, a.o_nat + nb, nat + 1);
     }
-    if (gcmc_ener) BCHK(b, hipMemcpy(gcmc_ener, b->base.gener + r, sizeof(double), hipMemcpyDeviceToHost));
+    if (gcmc_ener) *gcmc_ener = a.o_ener[0];
     if (ntot) *ntot = n;
     return BROMOC_OK;
 }

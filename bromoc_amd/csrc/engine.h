@@ -320,9 +320,9 @@ hipError_t launch_mmij(const StepParams &p, hipStream_t s);
 hipError_t launch_mmij_interact(const StepParams &p, double xj, double yj, double zj, int jtype,
                                 int j, double *out, hipStream_t s);
 // out[cat] = sum over particles of epart[cat], plus for the pair categories the sum over
-// the tile pairs of tener (tile mode), both in a fixed order; out holds NE * (1 +
-// 2 * RED_BLOCKS) doubles (the range sums and their errors follow the NE results)
-hipError_t launch_reduce_energy(const double *epart, int ecap, int n, double *out,
+// the tile pairs of tener (tile mode), both in a fixed order; part holds the range
+// sums and their errors, NE * 2 * RED_BLOCKS doubles; out (device-visible) the NE results
+hipError_t launch_reduce_energy(const double *epart, int ecap, int n, double *part, double *out,
                                 hipStream_t s, const double *tener = nullptr, int titems = 0);
 // tile mode (tiles.hip): k_tiles over every tile pair (which & 1), then k_tfin over every
 // slot (which & 2)
@@ -345,6 +345,34 @@ struct InteractParams {
     double *out;                // [1]
 };
 hipError_t launch_interact(const InteractParams &p, hipStream_t s);
+
+// ---- transfers through pinned host memory (stage.hip)
+constexpr int STAGE_MAX = 6;
+struct StageCopies {           // arrays of 32-bit words, copied by one launch
+    int32_t n, pad;
+    const void *src[STAGE_MAX];
+    void *dst[STAGE_MAX];
+    int64_t words[STAGE_MAX];
+    void add(void *d, const void *s, size_t bytes) {
+        src[n] = s; dst[n] = d; words[n] = (int64_t)(bytes / 4); n++;
+    }
+};
+struct StageReplica {          // one replica of a batch
+    int32_t r, nbuf;
+    const int32_t *ntot, *off;
+    const double4 *pos;
+    const int32_t *typei, *ibuffer, *nat;
+    const double *gener;
+    int32_t *o_n, *o_nat, *o_ty, *o_ib;
+    double *o_ener, *o_x, *o_y, *o_z;
+};
+hipError_t launch_stage_pos_out(const double4 *pos, int n, double *x, double *y, double *z,
+                                hipStream_t s);
+hipError_t launch_stage_pos_in(const double *x, const double *y, const double *z,
+                               const int32_t *t2h, const int32_t *tyh, int n, double4 *p0,
+                               double4 *p1, int32_t *t2, int32_t *ty, hipStream_t s);
+hipError_t launch_stage_copy(const StageCopies &c, hipStream_t s);
+hipError_t launch_stage_replica(const StageReplica &a, int cap, hipStream_t s);
 
 // ---- GRAND of one system on the device (grand.hip)
 constexpr int GC_BLOCKS = 256;   // workgroups of k_gc_interact (partials per attempt)

@@ -1221,10 +1221,9 @@ __global__ void k_reduce_finish(const Sum2 *part, double *out) {
     out[cat] = isfinite(acc.s) ? acc.s + acc.c : acc.s;   // the error of an infinite sum is not a number
 }
 
-hipError_t launch_reduce_energy(const double *epart, int ecap, int n, double *out,
+hipError_t launch_reduce_energy(const double *epart, int ecap, int n, double *part_, double *out,
                                 hipStream_t s, const double *tener, int titems) {
-    // the caller's buffer holds NE * (1 + 2 * RED_BLOCKS) doubles
-    Sum2 *part = reinterpret_cast<Sum2 *>(out + NE);
+    Sum2 *part = reinterpret_cast<Sum2 *>(part_);
     hipLaunchKernelGGL(k_reduce_energy, dim3(NE, RED_BLOCKS), dim3(BLOCK), 0, s, epart, ecap, n,
                        part, tener, titems);
     hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(64), 0, s, (const Sum2 *)part, out);
