@@ -35,18 +35,18 @@ FP64_PEAK_TFLOPS = 78.6
 # the same counters read for a 256 MiB device copy (bench.py --copy-probe 256): FETCH_SIZE
 # x 2.0, WRITE_SIZE x 1.0.  The counters cannot be read from inside this process; a shape
 # without a measurement reports null.
-TRAFFIC_KIB = {("translocation", 18): (378440.4, 732727.8), ("pore_dna", 1): (3541.9, 215.0)}
+TRAFFIC_KIB = {}   # none of the kernels as they are now
 # L2 hit rate of the same launches, TCC_HIT_sum / (TCC_HIT_sum + TCC_MISS_sum) from the
 # WRITE_SIZE run's two L2 counters
-L2_HIT = {("translocation", 18): 0.777, ("pore_dna", 1): 0.930}
+L2_HIT = {}
 TRAFFIC_SCALE = (2.0, 1.0)
 # FP64 operations per pair evaluation: a table pair ~34 (r^2 8, sqrt 1, index 2, U 4, F/r 3,
 # energy 1, force update on both particles ~15); the reaction-field cross term of an ion
 # pair ~30 (reff and srfe products 2, 1/sqrt 1, rfcf, aux0-aux3 9, energy 2, the srfe and
 # reff variation of both ions 4, the radial force on both 12)
 FLOP_PAIR, FLOP_RF = 34.0, 30.0
-TPB_NAMES = {1: "k_step, 1 target per block", 2: "k_step, 2 targets per block",
-             4: "k_step, 4 targets per block", 8: "k_wave, 1 target per wavefront",
+TPB_NAMES = {1: "k_step, 1 target per block", 2: "k_step_wave, 1 target per wavefront",
+             4: "k_step_wave, 2 targets per wavefront", 8: "k_wave, 1 target per wavefront",
              17: "tile mode, tiles of 64", 18: "tile mode, tiles of 128",
              20: "tile mode, tiles of 256"}
 

@@ -89,7 +89,7 @@ struct bromoc_ctx {
     int since_sort = 0;
     double r2near = 0.0;
     int cur = 0;
-    int tpb = 0;                             // targets per block chosen by the autotuner
+    int tpb = 0;                             // launch shape chosen by the autotuner
                                              // (TPB_TILE + targets per lane: tile mode)
     double *tpart = nullptr, *tener = nullptr;   // tile-mode partial sums and pair energies
     size_t tpart_n = 0, tener_n = 0;
@@ -1192,9 +1192,9 @@ static hipError_t enqueue_step(bromoc_ctx *c, const StepParams &p, hipEvent_t t0
     return launch_notrans(p, c->stream);
 }
 
-// Autotuner: the pair kernel's launch shape for this system -- k_step with 1, 2 or 4
-// targets per block, k_wave (8), or tile mode with 1, 2 or 4 targets per lane (17, 18,
-// 20) -- chosen by timing ENERGY-only launches (warnings go to a scratch counter) on the
+// Autotuner: the pair kernel's launch shape for this system -- k_step with a block per
+// target (1), k_step_wave with one or two targets a wavefront (2, 4), k_wave (8), or tile mode
+// with 1, 2 or 4 targets per lane (17, 18, 20) -- chosen by timing ENERGY-only launches (warnings go to a scratch counter) on the
 // ctx's stream: the reaction-field kernels the shape needs, the CG-DNA kernel and its pair
 // kernels.  The environment variable BROMOC_TPB forces a value.
 static int autotune(bromoc_ctx *c) {
@@ -1242,7 +1242,7 @@ static int autotune(bromoc_ctx *c) {
             p.warn = c->warn_scratch;
             // one whole ENERGY (the DNA, reaction-field and fixed-ion terms the pair kernel
             // reads), then the shape's reaction-field, CG-DNA and pair kernels are timed (the
-            // one-target shape computes the CG-DNA terms in its pair kernel)
+            // k_step shape computes the CG-DNA terms in its pair kernel)
             HIPCHK(c, launch_step(p, c->stream));
             HIPCHK(c, hipEventRecord(e0, c->stream));
             for (int r = 0; r < 5; r++) {
@@ -1406,7 +1406,7 @@ int bromoc_step(bromoc_ctx *c, int32_t nsteps, int32_t noise_mode, int32_t first
 // nsteps BD steps with a HIP event pair around every launch of the pair kernel (k_step,
 // k_wave or, in tile mode, k_tiles), on the stream the kernels run on: *total_ms is
 // first-to-last, *kernel_ms the mean pair-kernel duration.  A separate k_dna launch (tile
-// mode, several targets per block) falls outside the pair; the one-target k_step's own
+// mode, k_step_wave, k_wave) falls outside the pair; k_step's own
 // CG-DNA terms fall inside it.
 int bromoc_time_steps(bromoc_ctx *c, int32_t nsteps, int32_t noise_mode, int32_t first_row,
                       uint64_t seed, uint64_t counter0, double *total_ms, double *kernel_ms) {

@@ -32,12 +32,6 @@ constexpr uint32_t QDEBYHYB = 1u << 20, QNMCDEN = 1u << 19;
 constexpr double PI = 3.14159265358979323846264338327950288419716939937510;
 constexpr double RSMALL = 1E-3;
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-    return v;
-}
-
 // Lane moves within the wavefront by DPP: no LDS crossbar, two moves per double.  A lane
 // without a source keeps `old`.
 template <int CTRL, int ROWS = 0xf>
@@ -69,6 +63,13 @@ __device__ __forceinline__ double row_sum(double v) {
     v = half_row_sum(v);
     v += dpp<0x140>(v, v);   // row_mirror
     return v;
+}
+// the sum over the wavefront, on every lane (all 64 active)
+__device__ __forceinline__ double wave_sum(double v) {
+    v = row_sum(v);
+    v += dpp<DPP_BCAST15, 0xa>(0.0, v);   // rows 1 and 3: the sums of two rows
+    v += dpp<DPP_BCAST31, 0xc>(0.0, v);   // row 3: of four
+    return wave_last(v);
 }
 // a value that is the same on every lane, in scalar registers
 __device__ __forceinline__ double wave_uniform(double v) {
@@ -151,13 +152,24 @@ __device__ __forceinline__ void getyd(const DevPair &p, const double4 *__restric
     }
 }
 
+// 1/sqrt(d2) and 1/d2 for the analytic pair forms, each within about an ulp (1/d2 corrected by
+// its residual), with the limits of the division and the root: 0 gives infinity, infinity 0.
+__device__ __forceinline__ void recip_pair(double d2, double &ri, double &i2) {
+    const double r = __builtin_amdgcn_rsq(d2);
+    const double e = fma(-d2 * r, r, 1.0);
+    const bool reg = e == e;   // not 0 * infinity
+    ri = reg ? fma(r * e, fma(0.375, e, 0.5), r) : r;
+    i2 = ri * ri;
+    i2 = reg ? fma(i2, fma(-d2, i2, 1.0), i2) : i2;
+}
+
 // analytic pair branch, energy.mono.f90:135-178
 __device__ __forceinline__ double pair_analytic(const DevPair &p, const StepParams &P, double dist2,
                                                 double &eel, double &evd, double &esr) {
-    double idist2 = 1.0 / dist2, idist = 0.0, cofo = 0.0, dist6 = 0.0, dist12 = 0.0, dist = 0.0;
+    double idist, idist2, cofo = 0.0, dist6 = 0.0, dist12 = 0.0, dist = 0.0;
     double e1 = 0.0, e2 = 0.0, e3 = 0.0, fdf = 0.0, fdv = 0.0;
     const bool srp = (p.flags & PF_SRPMF) && dist2 <= P.rth;
-    if (p.flags & (PF_CHR | PF_SRPMF)) idist = sqrt(idist2);
+    recip_pair(dist2, idist, idist2);
     if (p.flags & PF_CHR) {
         cofo = p.fct * idist;
         eel += cofo;
@@ -665,34 +677,40 @@ __device__ __forceinline__ void ion_factors(const StepParams &P, int itype, doub
 // (dynamics0nuc.f90:31-44) for sites; fixcoor unless the site is free of the box
 // (dnafree).  dids (DYNAMICS3 only): the ion's nearest-site record of ENERGY
 // (energy.mono.f90:603-620): dist - dmi, dist, and the ion-minus-site vector.
-__device__ __forceinline__ double4 bd_move(const StepParams &P, bool is_site, int itype,
-                                           const double4 &pa, const double F[3],
-                                           const double *g, int32_t *nfwd, int32_t *nbwd,
-                                           const double *dids = nullptr) {
-    double fac1, fac2, ddz = 0.0;
+// In two parts, so that a kernel can fetch the factors early: bd_factors, then bd_shift.
+struct MoveFac { double fac1, fac2, ddz; };
+__device__ __forceinline__ void bd_factors(const StepParams &P, bool is_site, int itype, double z,
+                                           MoveFac &m) {
+    m.ddz = 0.0;
+    if (is_site) {
+        m.fac1 = P.fact0n1;
+        m.fac2 = P.fact0n2;
+    } else if (P.dmode == 3) {
+        m.fac1 = P.fact1a[itype];
+        m.fac2 = P.fact2a[itype];
+    } else {
+        ion_factors(P, itype, z, m.fac1, m.fac2, m.ddz);
+    }
+}
+__device__ __forceinline__ double4 bd_shift(const StepParams &P, bool is_site, int itype,
+                                            const double4 &pa, const double F[3], const double *g,
+                                            const MoveFac &m, int32_t *nfwd, int32_t *nbwd,
+                                            const double *dids = nullptr) {
+    double fac1 = m.fac1, fac2 = m.fac2;
+    const double ddz = m.ddz;
     double ddx3 = 0.0, ddy3 = 0.0, ddz3 = 0.0;
     const bool prox = !is_site && P.dmode == 3;
-    if (is_site) {
-        fac1 = P.fact0n1;
-        fac2 = P.fact0n2;
-    } else if (prox) {
-        if (dids[0] > 0.0 && dids[0] <= P.diffcutoff) {
-            const double D = P.diffusion[itype];
-            const double ebet = exp(-dids[0] * P.ibeta);
-            const double idf = D - (D - P.diff0) * ebet;
-            const double didf = (D - P.diff0) * P.ibeta * ebet;
-            const double idist = 1.0 / dids[1];
-            fac1 = idf * P.kbtdt;
-            fac2 = sqrt(2.0 * P.dt * idf);
-            ddx3 = didf * P.dt * dids[2] * idist;
-            ddy3 = didf * P.dt * dids[3] * idist;
-            ddz3 = didf * P.dt * dids[4] * idist;
-        } else {
-            fac1 = P.fact1a[itype];
-            fac2 = P.fact2a[itype];
-        }
-    } else {
-        ion_factors(P, itype, pa.z, fac1, fac2, ddz);
+    if (prox && dids[0] > 0.0 && dids[0] <= P.diffcutoff) {
+        const double D = P.diffusion[itype];
+        const double ebet = exp(-dids[0] * P.ibeta);
+        const double idf = D - (D - P.diff0) * ebet;
+        const double didf = (D - P.diff0) * P.ibeta * ebet;
+        const double idist = 1.0 / dids[1];
+        fac1 = idf * P.kbtdt;
+        fac2 = sqrt(2.0 * P.dt * idf);
+        ddx3 = didf * P.dt * dids[2] * idist;
+        ddy3 = didf * P.dt * dids[3] * idist;
+        ddz3 = didf * P.dt * dids[4] * idist;
     }
     const double bdmax = P.bdmax;
     double delx = F[0] * fac1, dely = F[1] * fac1, delz = F[2] * fac1;
@@ -719,6 +737,14 @@ __device__ __forceinline__ double4 bd_move(const StepParams &P, bool is_site, in
     }
     if (!is_site || !(P.flags & QDNAFREE)) fixcoor(P, xn, yn, zn);
     return make_double4(xn, yn, zn, pa.w);
+}
+__device__ __forceinline__ double4 bd_move(const StepParams &P, bool is_site, int itype,
+                                           const double4 &pa, const double F[3],
+                                           const double *g, int32_t *nfwd, int32_t *nbwd,
+                                           const double *dids = nullptr) {
+    MoveFac m;
+    bd_factors(P, is_site, itype, pa.z, m);
+    return bd_shift(P, is_site, itype, pa, F, g, m, nfwd, nbwd, dids);
 }
 
 __device__ __forceinline__ double4 bd_update(const StepParams &P, int i, bool is_site,

@@ -132,7 +132,7 @@ struct StepParams {
     uint32_t flags;
     int32_t mode;            // 0: ENERGY (forces out, no update), 1: ENERGY + DYNAMICS
     int32_t write_energy, write_forces;
-    int32_t tpb, all_efpot;  // k_step targets per block (1, 2, 4) or 8: k_wave; all tabulated
+    int32_t tpb, all_efpot;  // 1: k_step, 2, 4: k_step_wave, 8: k_wave; all tabulated
     int32_t tbeg, tend;      // target range of this launch (sites 0..nsites-1 come first)
     // positions (x, y, z, atnam2 type in the low word of w) in, updated positions out
     const double4 *pos;

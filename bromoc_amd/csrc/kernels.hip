@@ -1,9 +1,9 @@
 // kernels.hip -- gfx950 kernels of the BROMOC force / Brownian-dynamics step of one system.
 //
 // One BD step is k_rfpar/k_rfpair (reaction-field parameters, when present), the CG-DNA
-// list terms of each site (energy.mono.f90:196-508; in the one-target k_step's own site
-// blocks when the launch writes no energies, else k_dna_multi + k_dna) and k_step (or
-// k_wave): every target particle -- each free DNA site and each moving ion -- gathers its
+// list terms of each site (energy.mono.f90:196-508; in k_step's own site blocks when the
+// launch writes no energies, else k_dna_multi + k_dna) and k_step (or k_step_wave, k_wave):
+// every target particle -- each free DNA site and each moving ion -- gathers its
 // pair forces over all other particles (the reference's ENERGY has no cutoff:
 // energy.mono.f90:117-194,584-687), its 8 trilinear corners of the static-field and
 // repulsion grids (staticf1.f90:45-118, vdwgd1trln.f90:50-161), then applies the
@@ -219,314 +219,155 @@ __device__ inline double dna_site_finish(const StepParams &P, int i, int c,
     return acc;
 }
 
-// k_step: T target particles per block of NW wavefronts (targets tbeg.. of the launch).
-// Every thread walks the partner set with stride NW*64, two partners per iteration, and
-// evaluates each partner against all T targets.  Per-target sums: butterfly within each
-// wavefront, then a fixed-order sum over the NW wavefronts in LDS.  Wavefront w < T also
-// handles target w's 8 grid corners; thread a < T finishes target a (force, energies,
-// BD update).  In a launch that writes no energies (the step loop) a one-target block
-// computes its site target's CG-DNA list terms itself (dna_site_terms, before the pair
-// loop); otherwise the site targets read them from k_dna (fdna).
-template <int FEAT, int T, int NW>
-__global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(T == 1 ? 5 : 1)))
-void k_step(StepParams P) {
-    constexpr int NB = NW * WAVE;   // threads of the block
-    __shared__ DevPair s_row[T][MAX_LDS_TYPES];   // pair parameters by partner type
-    __shared__ double4 s_tail[T][MAX_LDS_TYPES];  // (sc3, tail fct, dm2hi, 0) by partner type
-    __shared__ double s_red[NW][T][7];
-    __shared__ double s_dg[T][5];
-    __shared__ double s_g[T][3];
-    __shared__ int s_warn[T];
-
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid >> 6;
-    const int ns = P.nsites, nf = P.nfix, ntot = P.ntot;
-    const int nt1 = P.nttyp + 1;
-    const int wbase = P.tbeg + blockIdx.x * T;
-
-    int ti[T];
-    bool tval[T], tsite[T], tfree[T];
-    double tx[T], ty[T], tz[T];
-#pragma unroll
-    for (int a = 0; a < T; a++) {
-        const int w = wbase + a;
-        tval[a] = w < P.tend;
-        const int i = !tval[a] ? 0 : (w < ns ? w : w + nf);
-        ti[a] = i;
-        tsite[a] = i < ns;
-        const double4 pa = P.pos[i];
-        tx[a] = pa.x; ty[a] = pa.y; tz[a] = pa.z;
-        tfree[a] = !tsite[a] || ((FEAT & F_DNA) && P.stfree[i] != 0);
-        // pair rows of this block's targets
-        const int row = __double2loint(pa.w) * nt1;
-        for (int k = tid; k < nt1; k += NB) {
-            const DevPair d = P.rows[row + k];
-            s_row[a][k] = d;
-            s_tail[a][k] = make_double4(d.sc3, d.fct, d.dm2hi, 0.0);
-        }
+// The far form of a pair type: r^-6, r^-12 and 1/r factors, range^2 (< 0: none).  A table pair's
+// tail, or LJ 4 eps (s^12 - s^6) and the Coulomb term.
+__device__ __forceinline__ double4 pair_far(const StepParams &P, bool tab, const DevPair &d) {
+    if (tab || (d.flags & PF_EFPOT)) return make_double4(d.sc3, 0.0, d.fct, d.dm2hi);
+    const double s6 = (d.flags & PF_LJ) ? pow3(d.sgp2) : 0.0;
+    return make_double4(-d.epp4 * s6, d.epp4 * (s6 * s6), (d.flags & PF_CHR) ? d.fct : 0.0,
+                        (d.flags & PF_SRPMF) ? P.rth : -1.0);
+}
+// n pair rows from `src` and their far forms into LDS by the whole block; the caller
+// synchronises.
+__device__ __forceinline__ void pair_lds(const StepParams &P, bool tab, const DevPair *src, int n,
+                                         DevPair *rows, double4 *far) {
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+        const DevPair d = src[k];
+        rows[k] = d;
+        far[k] = pair_far(P, tab, d);
     }
-    __syncthreads();
+}
+static size_t pair_lds_bytes(int nrow) { return (size_t)nrow * (sizeof(DevPair) + sizeof(double4)); }
 
-    // CG-DNA list terms of a site target (the block-uniform branch of a one-target block),
-    // in the launches that write no energies; the others read k_dna's (fdna)
-    constexpr bool DNA_HERE = (FEAT & F_DNA) != 0 && T == 1;
-    const bool dna_here = DNA_HERE && !P.write_energy;
-    __shared__ double s_dn[DNA_HERE ? NW : 1][3 + 8];
-    if constexpr (DNA_HERE) {
-        if (dna_here && tval[0] && tsite[0]) {
-            V3 f = {0.0, 0.0, 0.0};
-            double e[8];
-            dna_site_terms<NB, DNA_DU, true, false>(P, ti[0], tid, f, e);
-            dna_block_sums<NW, false>(P, lane, wv, f, e, s_dn);
-        }
-    }
-
-    // Gaussians of the BD update, fetched by the last wavefront (lanes 0..T-1) before its
-    // share of the pair loop
+// What a target's end needs, loaded at its start: the lane that will finish it (`fin`) holds
+// the particle, its type, sorted slot, Gaussians and diffusion factors, and 8 lanes the grid
+// corners.  In two parts around pair_lds: its stores wait for every load issued before them.
+struct Target {
+    int i, rank, itype;
+    bool site, free, ok_x, ok_v;
+    double4 p;
+    double chi, g[3];
+    MoveFac mv;
+    float ph_x;
+    int8_t ph_v;
+};
+template <int FEAT>
+__device__ __forceinline__ void target_load(const StepParams &P, Target &t, int i, bool on, bool fin) {
+    t = Target{};
+    if (!on) return;
+    t.i = i;
+    t.site = i < P.nsites;
+    t.p = P.pos[i];
+    t.free = !t.site || ((FEAT & F_DNA) && P.stfree[i] != 0);
+    if (!t.site) t.itype = abs(P.typei[i]);
     if constexpr ((FEAT & F_UPDATE) != 0) {
-        const int a = tid - (NB - WAVE);
-        if (a >= 0 && a < T && tval[a]) {
-            const int i = ti[a];
+        if (fin) {
+            t.rank = P.rank[i];
             const double *nr = noise_row(P, i);
-            s_g[a][0] = nr[0]; s_g[a][1] = nr[1]; s_g[a][2] = nr[2];
+            t.g[0] = nr[0]; t.g[1] = nr[1]; t.g[2] = nr[2];
         }
     }
-
-    double fx[T], fy[T], fz[T], et[T], eel[T], evd[T], esr[T];
-#pragma unroll
-    for (int a = 0; a < T; a++) fx[a] = fy[a] = fz[a] = et[a] = eel[a] = evd[a] = esr[a] = 0.0;
-    // PROXDIFF: per target ion, the tabulated site partner within its table range of least
-    // dist - dmi, ties to the lower site index (energy.mono.f90:603-620 in site order)
-    double pxd[T];
-    int pxj[T];
-#pragma unroll
-    for (int a = 0; a < T; a++) { pxd[a] = INFINITY; pxj[a] = 0x7fffffff; }
-
-    // ---- pair loop (energy.mono.f90:117-194, 584-687), compiled twice: with the energy
-    // sums, and without them for the steps that write no energies
-    const bool nonbond = (P.flags & QNONBOND) && (P.flags & QPAR);
-    auto pair_loop = [&](auto en) {
-        constexpr bool EN = decltype(en)::value;
-        // partners per iteration: two (with the next iteration's partners loaded during
-        // this one's, measured best for every shape; three or four only added registers)
-        constexpr int PU = 2;
-        // the next iteration's partners are loaded while this one's are evaluated
-        double4 nx[PU];
-#pragma unroll
-        for (int u = 0; u < PU; u++) nx[u] = P.spos[min(tid + u * NB, ntot - 1)];
-        for (int k0 = tid; k0 < ntot; k0 += PU * NB) {
-            // partners in spatial order, PU per iteration
-            double4 pp[PU];
-            bool pok[PU];
-#pragma unroll
-            for (int u = 0; u < PU; u++) {
-                pp[u] = nx[u];
-                pok[u] = k0 + u * NB < ntot;
-                nx[u] = P.spos[min(k0 + (PU + u) * NB, ntot - 1)];
-            }
-#pragma unroll
-            for (int u = 0; u < PU; u++) {
-                const double4 pj = pp[u];
-                const bool jok = pok[u];
-                const int t2j = __double2loint(pj.w);
-                const int j = __double2hiint(pj.w);
-#pragma unroll
-                for (int a = 0; a < T; a++) {
-                    const bool skip = !jok || !tval[a] || j == ti[a] || (tsite[a] && j < ns);
-                    const double dx = tx[a] - pj.x, dy = ty[a] - pj.y, dz = tz[a] - pj.z;
-                    double d2 = dx * dx + dy * dy + dz * dz;
-                    d2 = skip ? 1e30 : d2;
-                    // a pair's energy is counted once: by the site of a site-ion pair, by
-                    // the higher-index ion of an ion-ion pair
-                    const bool ce = !skip && (tsite[a] || (j >= ns && j < ti[a]));
-                    double y, de;
-                    if constexpr ((FEAT & F_TAB) != 0) {
-                        de = pair_near_far(s_row[a][t2j], s_tail[a][t2j], P.ep, P.ires, d2, y);
-                        if constexpr (EN) et[a] += ce ? y : 0.0;
-                    } else if (s_row[a][t2j].flags & PF_EFPOT) {
-                        de = pair_near_far(s_row[a][t2j], s_tail[a][t2j], P.ep, P.ires, d2, y);
-                        if constexpr (EN) et[a] += ce ? y : 0.0;
-                    } else {
-                        double q0 = 0.0, q1 = 0.0, q2 = 0.0;
-                        de = pair_analytic(s_row[a][t2j], P, d2, q0, q1, q2);
-                        if constexpr (EN) {
-                            eel[a] += ce ? q0 : 0.0;
-                            evd[a] += ce ? q1 : 0.0;
-                            esr[a] += ce ? q2 : 0.0;
-                        }
-                    }
-                    if constexpr ((FEAT & F_PROX) != 0) {
-                        const DevPair &pr = s_row[a][t2j];
-                        if (!skip && !tsite[a] && j < ns && ((FEAT & F_TAB) || (pr.flags & PF_EFPOT)) &&
-                            !(d2 < pr.dm2lo) && !(d2 > pr.dm2hi)) {
-                            const double dd = sqrt(d2) - pr.dmi;
-                            if (dd < pxd[a] || (dd == pxd[a] && j < pxj[a])) { pxd[a] = dd; pxj[a] = j; }
-                        }
-                    }
-                    de = (skip || !tfree[a]) ? 0.0 : de;
-                    fx[a] += de * dx;
-                    fy[a] += de * dy;
-                    fz[a] += de * dz;
-                }
-            }
-        }
-    };
-    if (nonbond) {
-        if (P.write_energy) pair_loop(std::true_type{});
-        else pair_loop(std::false_type{});
-    }
-    __shared__ double s_pxd[(FEAT & F_PROX) ? NW : 1][T];
-    __shared__ int s_pxj[(FEAT & F_PROX) ? NW : 1][T];
-    if constexpr ((FEAT & F_PROX) != 0) {
-#pragma unroll
-        for (int a = 0; a < T; a++) {
-            double d = pxd[a];
-            int jj = pxj[a];
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const double od = __shfl_xor(d, off, WAVE);
-                const int oj = __shfl_xor(jj, off, WAVE);
-                if (od < d || (od == d && oj < jj)) { d = od; jj = oj; }
-            }
-            if (lane == 0) { s_pxd[wv][a] = d; s_pxj[wv][a] = jj; }
-        }
-    }
-
-    // pair sums to LDS (the pair accumulators are dead after this)
-#pragma unroll
-    for (int a = 0; a < T; a++) {
-        double v[7] = {fx[a], fy[a], fz[a], et[a], eel[a], evd[a], esr[a]};
-#pragma unroll
-        for (int k = 0; k < 7; k++) {
-            if (k >= 3 && !P.write_energy) break;
-            v[k] = wave_sum(v[k]);
-            if (lane == 0) s_red[wv][a][k] = v[k];
-        }
-    }
-
-    // ---- grids of target `wv` (if any), lanes 0..7 of wavefront wv
-    double gfx = 0.0, gfy = 0.0, gfz = 0.0, egx = 0.0, egv = 0.0;
-    bool warned = false;
-    const bool mine = wv < T;
-    int i_me = 0;
-    bool val_me = false, site_me = false;
-    double xi = 0.0, yi = 0.0, zi = 0.0;
-    int t2i = 0;
-    if (mine) {
-        const int w = wbase + wv;
-        val_me = w < P.tend;
-        i_me = !val_me ? 0 : (w < ns ? w : w + nf);
-        site_me = i_me < ns;
-        const double4 pa = P.pos[i_me];
-        xi = pa.x; yi = pa.y; zi = pa.z;
-        t2i = __double2loint(pa.w);
-    }
+}
+template <int FEAT>
+__device__ __forceinline__ void target_load2(const StepParams &P, Target &t, bool on, bool fin, int c) {
+    if (!on) return;
+    const int i = t.i;
+    // static field and trilinear repulsion map (staticf1.f90:45-118, vdwgd1trln.f90:50-161)
     if constexpr ((FEAT & F_PHIX) != 0) {
-        if (mine && val_me && lane < 8) {
-            const GridGeom &g = P.gx;
-            double chi;
-            bool ok;
-            if (site_me) { ok = P.namsite[i_me] == 1; chi = P.cgnuc; }
-            else { ok = true; chi = P.cg[abs(P.typei[i_me])]; }
-            ok = ok && xi <= g.xbcen + g.tranx && xi >= g.xbcen - g.tranx &&
-                 yi <= g.ybcen + g.trany && yi >= g.ybcen - g.trany &&
-                 zi <= g.zbcen + g.tranz && zi >= g.zbcen - g.tranz;
-            if (ok) {
-                double gx_, gy_, gz_;
-                int ix, iy, iz;
-                grid_cell(g, xi, yi, zi, gx_, gy_, gz_, ix, iy, iz);
-                const double one1 = 1.0;
-                const int n1 = ix + (lane >> 2), n2 = iy + ((lane >> 1) & 1), n3 = iz + (lane & 1);
-                double ai = gx_ - n1 * g.dcel;
-                const double aisign = fsign(one1, ai);
-                ai = one1 - fabs(ai) * g.idcel;
-                double bi = gy_ - n2 * g.dcel;
-                const double bisign = fsign(one1, bi);
-                bi = one1 - fabs(bi) * g.idcel;
-                double ci = gz_ - n3 * g.dcel;
-                const double cisign = fsign(one1, ci);
-                ci = one1 - fabs(ci) * g.idcel;
-                const double fi = ai * bi * ci;
-                const double ph = (double)P.phix[((size_t)n1 * g.ny + n2) * g.nz + n3];
-                const double prefac = ph * P.celec * chi * g.idcel;
-                if (ai < (1.0 - RSMALL) && ai > RSMALL) gfx += aisign * bi * ci * prefac;
-                if (bi < (1.0 - RSMALL) && bi > RSMALL) gfy += bisign * ai * ci * prefac;
-                if (ci < (1.0 - RSMALL) && ci > RSMALL) gfz += cisign * ai * bi * prefac;
-                egx += fi * chi * ph * P.celec;
-            }
+        const GridGeom &g = P.gx;
+        t.ok_x = (!t.site || P.namsite[i] == 1) && t.p.x <= g.xbcen + g.tranx && t.p.x >= g.xbcen - g.tranx &&
+                 t.p.y <= g.ybcen + g.trany && t.p.y >= g.ybcen - g.trany &&
+                 t.p.z <= g.zbcen + g.tranz && t.p.z >= g.zbcen - g.tranz && c < 8;
+        if (t.ok_x) {
+            double x, y, z;
+            int ix, iy, iz;
+            grid_cell(g, t.p.x, t.p.y, t.p.z, x, y, z, ix, iy, iz);
+            t.ph_x = P.phix[tri_node(g, ix, iy, iz, c)];
+            t.chi = t.site ? P.cgnuc : P.cg[t.itype];
         }
     }
     if constexpr ((FEAT & F_PHIV) != 0) {
-        if (mine && val_me) warned = vdw_grid(P, xi, yi, zi, t2i, gfx, gfy, gfz, egv, vdw_map_of(P, i_me));
-    }
-    if (mine) {
-        gfx = wave_sum(gfx);
-        gfy = wave_sum(gfy);
-        gfz = wave_sum(gfz);
-        if (P.write_energy) {
-            egx = wave_sum(egx);
-            egv = wave_sum(egv);
-        }
-        if (lane == 0) {
-            s_dg[wv][0] = gfx; s_dg[wv][1] = gfy; s_dg[wv][2] = gfz;
-            s_dg[wv][3] = egx; s_dg[wv][4] = egv;
-            s_warn[wv] = warned ? 1 : 0;
+        const GridGeom &g = P.gv;
+        t.ok_v = !(P.flags & QBSPLINE) && t.p.x <= g.xbcen + g.tranx && t.p.x >= g.xbcen - g.tranx &&
+                 t.p.y <= g.ybcen + g.trany && t.p.y >= g.ybcen - g.trany && t.p.z <= P.vzmax &&
+                 t.p.z >= P.vzmin && c < 8;
+        if (t.ok_v) {
+            double x, y, z;
+            int ix, iy, iz;
+            grid_cell(g, t.p.x, t.p.y, t.p.z, x, y, z, ix, iy, iz);
+            t.ph_v = P.phiv[vdw_map_of(P, i) + tri_node(g, ix, iy, iz, c)];
         }
     }
-    __syncthreads();
-    if (tid >= T) return;
+    if constexpr ((FEAT & F_UPDATE) != 0) {
+        if (fin) bd_factors(P, t.site, t.itype, t.p.z, t.mv);
+    }
+}
 
-    // ---- thread a finishes target a
-    const int a = tid;
-    const int w = wbase + a;
-    if (w >= P.tend) return;
-    const int i = w < ns ? w : w + nf;
-    const bool is_site = i < ns;
-    double F[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        double acc = 0.0;
-#pragma unroll
-        for (int q = 0; q < NW; q++) acc += s_red[q][a][k];
-        F[k] = acc + s_dg[a][k];
-    }
-    if constexpr ((FEAT & F_DNA) != 0) {
-        if (is_site && dna_here) {
-#pragma unroll
-            for (int k = 0; k < 3; k++) F[k] += dna_site_finish<NW>(P, i, k, s_dn);
-        } else if (is_site) {
-            const double4 fd = P.fdna[i];   // CG-DNA list terms from k_dna
-            F[0] += fd.x; F[1] += fd.y; F[2] += fd.z;
+// Grid force and energies from the corners of target_load, summed over its 8 lanes (on every
+// one of them); whether the map's wall was reached.
+template <int FEAT>
+__device__ __forceinline__ bool target_grids(const StepParams &P, const Target &t, int c, double g[3],
+                                             double &egx, double &egv) {
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    bool warned = false;
+    egx = egv = 0.0;
+    if constexpr ((FEAT & F_PHIX) != 0) {
+        if (t.ok_x) {
+            double x, y, z;
+            int ix, iy, iz;
+            grid_cell(P.gx, t.p.x, t.p.y, t.p.z, x, y, z, ix, iy, iz);
+            tri_apply(P.gx, (double)t.ph_x, x, y, z, ix, iy, iz, c, P.celec * t.chi, fx, fy, fz, egx);
         }
     }
-    if ((P.rfon || P.mmon) && !is_site) {   // reaction-field forces (k_rfpair or k_mm_force)
-        const double4 fr = P.frf[i];
-        F[0] += fr.x; F[1] += fr.y; F[2] += fr.z;
+    if constexpr ((FEAT & F_PHIV) != 0) {
+        if (t.ok_v) {
+            double x, y, z;
+            int ix, iy, iz;
+            grid_cell(P.gv, t.p.x, t.p.y, t.p.z, x, y, z, ix, iy, iz);
+            const double esvdw = (P.flags & QSVDW) ? P.svdw * P.scal[__double2loint(t.p.w)] : P.svdw;
+            tri_apply(P.gv, (double)t.ph_v, x, y, z, ix, iy, iz, c, esvdw, fx, fy, fz, egv);
+        }
+        warned = half_row_sum((double)t.ph_v) >= P.thold8 && t.ok_v;   // integers: exact
     }
-    const double4 pa = P.pos[i];
-    const int t2a = __double2loint(pa.w);
-    if (s_warn[a]) atomicAdd(&P.warn[t2a], 1);
+    g[0] = half_row_sum(fx);
+    g[1] = half_row_sum(fy);
+    g[2] = half_row_sum(fz);
+    if (P.write_energy) { egx = half_row_sum(egx); egv = half_row_sum(egv); }
+    return warned;
+}
+// The B-spline repulsion map of one target by the whole wavefront, on every lane.
+template <int FEAT>
+__device__ __forceinline__ bool target_spline(const StepParams &P, double4 p, int i, double g[3], double &egv) {
+    bool warned = false;
+    double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
+    if constexpr ((FEAT & F_PHIV) != 0)
+        warned = vdw_grid(P, p.x, p.y, p.z, __double2loint(p.w), fx, fy, fz, e, vdw_map_of(P, i));
+    g[0] = wave_sum(fx); g[1] = wave_sum(fy); g[2] = wave_sum(fz);
+    egv = wave_sum(e);
+    return warned;
+}
+
+// One lane ends a target: membrane, energies, forces, BD update.  F: the whole force but the
+// membrane's; pe: the pair energies (table, Coulomb, LJ, SRPMF).
+template <int FEAT>
+__device__ __forceinline__ void target_finish(const StepParams &P, const Target &t, double F[3], bool warned,
+                                              const double pe[4], double egx, double egv) {
+    const int i = t.i, t2 = __double2loint(t.p.w);
+    if (warned) atomicAdd(&P.warn[t2], 1);
     if (P.flags & QMEMB) {   // MEMBRANE, membrane.f90:36-104
-        const double chg = is_site ? (P.namsite[i] == 1 ? P.cgnuc : 0.0) : P.cg[abs(P.typei[i])];
+        const double chg = t.site ? (P.namsite[i] == 1 ? P.cgnuc : 0.0) : P.cg[t.itype];
         bool mw;
-        const double em = membrane_energy(P, pa.x, pa.y, pa.z, chg, t2a, F, mw);
-        if (mw) atomicAdd(&P.warn[t2a], 1);
+        const double em = membrane_energy(P, t.p.x, t.p.y, t.p.z, chg, t2, F, mw);
+        if (mw) atomicAdd(&P.warn[t2], 1);
         if (P.write_energy) P.epart[(size_t)E_MEMB * P.ecap + i] = em;
     }
     if (P.write_energy) {
-        double pe[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            double acc = 0.0;
-#pragma unroll
-            for (int q = 0; q < NW; q++) acc += s_red[q][a][3 + k];
-            pe[k] = acc;
-        }
         // this kernel owns the pair and grid categories; k_dna writes the DNA ones
         double *ep_ = P.epart + i;
         const size_t cs = P.ecap;
-        ep_[E_GSBPA * cs] = s_dg[a][3];
-        ep_[E_VDWGD * cs] = s_dg[a][4];
-        if (is_site) {
+        ep_[E_GSBPA * cs] = egx;
+        ep_[E_VDWGD * cs] = egv;
+        if (t.site) {
             ep_[E_EFPOTMX * cs] = pe[0]; ep_[E_QQMX * cs] = pe[1];
             ep_[E_VDWMX * cs] = pe[2]; ep_[E_SRPMFMX * cs] = pe[3];
         } else {
@@ -542,21 +383,607 @@ void k_step(StepParams P) {
     if constexpr ((FEAT & F_UPDATE) != 0) {
         // virial of the step, F . x at the positions the forces were taken at
         // (simul1.f90:365-367); fixed ions carry no force and add nothing
-        if (P.vacc) P.vacc[i] += F[0] * pa.x + F[1] * pa.y + F[2] * pa.z;
-        const bool fr = !is_site || ((FEAT & F_DNA) && P.stfree[i] != 0);
-        if (!fr) {
-            P.poso[i] = pa;
-            P.sposo[P.rank[i]] = pa;
+        if (P.vacc) P.vacc[i] += F[0] * t.p.x + F[1] * t.p.y + F[2] * t.p.z;
+        double4 pn = t.p;
+        if (t.free) pn = bd_shift(P, t.site, t.itype, t.p, F, t.g, t.mv, P.nfwd, P.nbwd);
+        P.poso[i] = pn;
+        P.sposo[t.rank] = pn;
+    }
+}
+
+// The pair sums of T targets over the partners tid, tid + NB, ..: the far form straight
+// through, analytic pair types by the same expression with an r^-12 term; the few pairs in
+// range (table, or SRPMF) are noted as bits and worked off after every 32 partners a thread (a
+// branch per pair took the table's dependent loads in most iterations).  PU partners are in
+// flight, the next PU loaded meanwhile.  row0: the first of a target's rows in LDS.  Energies (EN) only where
+// they are written.
+template <int T> struct PairAcc {
+    double fx[T], fy[T], fz[T], et[T], eel[T], evd[T], esr[T];
+};
+template <int FEAT, int T, int NB, int PU, bool EN>
+__device__ __forceinline__ void pair_sums(const StepParams &P, const DevPair *s_rows, const double4 *s_far,
+                                          int tid, const int ti[T], const int row0[T],
+                                          const double4 tp[T], double4 nx[PU], PairAcc<T> &A) {
+    constexpr bool TAB = (FEAT & F_TAB) != 0;
+    const int ns = P.nsites, ntot = P.ntot;
+    for (int base = tid; base < ntot; base += 32 * NB) {
+        uint32_t m[T];
+#pragma unroll
+        for (int a = 0; a < T; a++) m[a] = 0u;
+        const int cnt = min(32, (ntot - base + NB - 1) / NB);
+#pragma unroll 1
+        for (int k0 = 0; k0 < cnt; k0 += PU) {
+            double4 pp[PU];
+#pragma unroll
+            for (int u = 0; u < PU; u++) {
+                pp[u] = nx[u];
+                nx[u] = P.spos[min(base + (k0 + PU + u) * NB, ntot - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < PU; u++) {
+                const double4 pj = pp[u];
+                const bool jok = base + (k0 + u) * NB < ntot;
+                const int t2j = __double2loint(pj.w);
+                const int j = __double2hiint(pj.w);
+#pragma unroll
+                for (int a = 0; a < T; a++) {
+                    const bool tsite = ti[a] < ns;
+                    const bool on = jok && j != ti[a] && !(tsite && j < ns);
+                    const int row = row0[a] + t2j;
+                    const double4 fa = s_far[row];
+                    const double dx = tp[a].x - pj.x, dy = tp[a].y - pj.y, dz = tp[a].z - pj.z;
+                    const double d2 = on ? pair_d2(dx, dy, dz) : 1e30;
+                    const bool near = on && d2 <= fa.w;
+                    double ri, i2;
+                    if constexpr (TAB) {
+                        ri = rsqrt_c3(d2);
+                        i2 = ri * ri;
+                    } else {
+                        recip_pair(d2, ri, i2);
+                    }
+                    const double i6 = i2 * i2 * i2, c = fa.x * i6, q = fa.z * ri;
+                    double f = 6.0 * c + q;
+                    double b = 0.0;
+                    if constexpr (!TAB) {
+                        b = fa.y * (i6 * i6);
+                        f = fma(12.0, b, f);
+                    }
+                    f = on && !near ? f * i2 : 0.0;
+                    if constexpr (EN) {
+                        // a pair's energy is counted once: by the site of a site-ion pair,
+                        // by the higher-index ion of an ion-ion pair
+                        const bool ce = on && !near && (tsite || (j >= ns && j < ti[a]));
+                        const int fl = TAB ? (int)PF_EFPOT : s_rows[row].flags;
+                        A.et[a] += ce && (fl & PF_EFPOT) ? c + q : 0.0;
+                        if constexpr (!TAB) {
+                            A.eel[a] += ce && (fl & (PF_EFPOT | PF_CHR)) == PF_CHR ? q : 0.0;
+                            A.evd[a] += ce && (fl & (PF_EFPOT | PF_LJ)) == PF_LJ ? b + c : 0.0;
+                        }
+                    }
+                    m[a] |= near ? 1u << (k0 + u) : 0u;
+                    A.fx[a] = fma(f, dx, A.fx[a]);
+                    A.fy[a] = fma(f, dy, A.fy[a]);
+                    A.fz[a] = fma(f, dz, A.fz[a]);
+                }
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < T; a++) {
+            while (m[a]) {   // the pairs in range
+                const int k = __ffs(m[a]) - 1;
+                m[a] &= m[a] - 1u;
+                const double4 pj = P.spos[base + k * NB];
+                const int j = __double2hiint(pj.w);
+                const DevPair &row = s_rows[row0[a] + __double2loint(pj.w)];
+                const double dx = tp[a].x - pj.x, dy = tp[a].y - pj.y, dz = tp[a].z - pj.z;
+                const double d2 = pair_d2(dx, dy, dz);
+                const bool ce = ti[a] < ns || (j >= ns && j < ti[a]);
+                double f;
+                if (TAB || (row.flags & PF_EFPOT)) {
+                    double y;
+                    f = pair_table(row, P.ep, P.ires, d2, rsqrt_c3(d2), y);
+                    if constexpr (EN) A.et[a] += ce ? y : 0.0;
+                } else {
+                    double q0 = 0.0, q1 = 0.0, q2 = 0.0;
+                    f = pair_analytic(row, P, d2, q0, q1, q2);
+                    if constexpr (EN) {
+                        A.eel[a] += ce ? q0 : 0.0;
+                        A.evd[a] += ce ? q1 : 0.0;
+                        A.esr[a] += ce ? q2 : 0.0;
+                    }
+                }
+                A.fx[a] = fma(f, dx, A.fx[a]);
+                A.fy[a] = fma(f, dy, A.fy[a]);
+                A.fz[a] = fma(f, dz, A.fz[a]);
+            }
+        }
+    }
+}
+template <int FEAT, int T, int NB, int PU>
+__device__ __forceinline__ void pair_sums(const StepParams &P, const DevPair *s_rows, const double4 *s_far,
+                                          int tid, const int ti[T], const int row0[T],
+                                          const double4 tp[T], double4 nx[PU], PairAcc<T> &A) {
+#pragma unroll
+    for (int a = 0; a < T; a++) {
+        A.fx[a] = A.fy[a] = A.fz[a] = A.et[a] = A.eel[a] = A.evd[a] = A.esr[a] = 0.0;
+    }
+    if (!(P.flags & QNONBOND) || !(P.flags & QPAR)) return;
+    if (P.write_energy) pair_sums<FEAT, T, NB, PU, true>(P, s_rows, s_far, tid, ti, row0, tp, nx, A);
+    else pair_sums<FEAT, T, NB, PU, false>(P, s_rows, s_far, tid, ti, row0, tp, nx, A);
+}
+
+// k_step_wave: T targets by each wavefront, four wavefronts a block, each lane partners lane,
+// lane + 64, ..; 8 lanes a target hold its grid corners, the first of them ends it.  Blocks
+// start at a limited rate (an empty k_step over 1531 targets takes 9.9 us, over 400 5.5), so
+// fewer, fuller ones are faster where the chain of one target is not the longest part: 1531
+// ions of analytic pairs 25.0 us a step with k_step's two targets a block before, 14.8 with
+// one target a wavefront, 16.5 with two; 2300 particles with DNA 24.4 us, k_step 22.0.
+template <int FEAT, int T>
+__global__ __launch_bounds__(BLOCK) void k_step_wave(StepParams P) {
+    constexpr int PU = T == 1 ? 4 : 2;
+    extern __shared__ double4 s_dyn[];
+    const int nt1 = P.nttyp + 1;
+    DevPair *s_rows = reinterpret_cast<DevPair *>(s_dyn);
+    double4 *s_far = s_dyn + (size_t)nt1 * nt1 * (sizeof(DevPair) / sizeof(double4));
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int w0 = P.tbeg + ((int)blockIdx.x * WPB + wv) * T;
+    auto index = [&](int w) { return w < P.nsites ? w : w + P.nfix; };
+    const int lane = threadIdx.x & (WAVE - 1), ntot = P.ntot, last = P.tend - 1;
+    double4 nx[PU];
+#pragma unroll
+    for (int u = 0; u < PU; u++) nx[u] = P.spos[min(lane + u * WAVE, ntot - 1)];
+    int ti[T], row0[T];
+    double4 tp[T];
+#pragma unroll
+    for (int a = 0; a < T; a++) {   // past the last target: that one again
+        ti[a] = index(min(w0 + a, last));
+        tp[a] = P.pos[ti[a]];
+    }
+    const int a_me = lane >> 3, c = lane & 7;
+    const bool mine = a_me < T && w0 + a_me <= last;
+    Target t;
+    target_load<FEAT>(P, t, index(min(w0 + a_me, last)), mine, c == 0);
+    pair_lds(P, (FEAT & F_TAB) != 0, P.rows, nt1 * nt1, s_rows, s_far);
+    target_load2<FEAT>(P, t, mine, c == 0, c);
+    __syncthreads();
+    if (w0 > last) return;   // the wavefront has no target
+#pragma unroll
+    for (int a = 0; a < T; a++) row0[a] = __double2loint(tp[a].w) * nt1;
+    PairAcc<T> A;
+    pair_sums<FEAT, T, WAVE, PU>(P, s_rows, s_far, lane, ti, row0, tp, nx, A);
+    // forces that other kernels computed: k_dna's, k_rfpair's or k_mm_force's
+    double4 fo = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (mine && c == 0) {
+        if ((FEAT & F_DNA) && t.site) fo = P.fdna[t.i];
+        if ((P.rfon || P.mmon) && !t.site) fo = P.frf[t.i];
+    }
+    double g[3], egx, egv;
+    bool warned = target_grids<FEAT>(P, t, c, g, egx, egv);
+    double F[3] = {0.0, 0.0, 0.0}, pe[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int a = 0; a < T; a++) {
+        const double x = wave_sum(A.fx[a]), y = wave_sum(A.fy[a]), z = wave_sum(A.fz[a]);
+        if (a_me == a) { F[0] = x; F[1] = y; F[2] = z; }
+        if (P.write_energy) {
+            const double e0 = wave_sum(A.et[a]), e1 = wave_sum(A.eel[a]), e2 = wave_sum(A.evd[a]),
+                         e3 = wave_sum(A.esr[a]);
+            if (a_me == a) { pe[0] = e0; pe[1] = e1; pe[2] = e2; pe[3] = e3; }
+        }
+        if ((FEAT & F_PHIV) && (P.flags & QBSPLINE)) {
+            double gs[3], es;
+            const bool ws = target_spline<FEAT>(P, tp[a], ti[a], gs, es);
+            if (a_me == a) { g[0] += gs[0]; g[1] += gs[1]; g[2] += gs[2]; egv = es; warned = ws; }
+        }
+    }
+    if (!mine || c != 0) return;
+    if (!t.free) F[0] = F[1] = F[2] = 0.0;   // a fixed site's pair forces are not formed
+    F[0] = F[0] + g[0] + fo.x;
+    F[1] = F[1] + g[1] + fo.y;
+    F[2] = F[2] + g[2] + fo.z;
+    target_finish<FEAT>(P, t, F, warned, pe, egx, egv);
+}
+
+// k_step: a block of NW wavefronts for each target tbeg..tend-1 of the launch.  Every thread walks
+// the partner set with stride NW*64, two partners per iteration; the sums go over each
+// wavefront by DPP, then over the NW wavefronts in LDS in a fixed order.  The first wavefront
+// also handles the target's grid corners, and its lane 0 finishes the target.  In a launch that
+// writes no energies (the step loop) the block computes its site target's CG-DNA list terms
+// itself (dna_site_terms); otherwise the site targets read them from k_dna (fdna).  The pair
+// loop is pair_sums' with one target and the block's registers in mind (five wavefronts a
+// SIMD): what the end needs is parked in LDS.
+//
+// A step of a small system is one chain of loads behind the launch (5.0 us a step with two
+// ions): 400 ions 7.3 us, 2300 with DNA 22.8 -> 22.0 us, of that 10 us without pair loop and
+// list terms, mostly the rate at which blocks start.
+template <int FEAT, int NW>
+__global__ __launch_bounds__(NW * WAVE)
+__attribute__((amdgpu_waves_per_eu((FEAT & F_TAB) ? 5 : 4)))
+void k_step(StepParams P) {
+    constexpr int NB = NW * WAVE;   // threads of the block
+    constexpr bool TAB = (FEAT & F_TAB) != 0;
+    __shared__ DevPair s_row[MAX_LDS_TYPES];   // pair parameters by partner type
+    // by partner type: the far form's r^-6, r^-12 and 1/r factors, range^2 (< 0: none)
+    __shared__ double4 s_far[MAX_LDS_TYPES];
+    __shared__ double s_red[NW][7];
+    __shared__ double s_mv[6];   // Gaussians and factors of the update
+
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid >> 6;
+    const int ns = P.nsites, nf = P.nfix, ntot = P.ntot;
+    const int nt1 = P.nttyp + 1;
+    const int wbase = P.tbeg + blockIdx.x;
+
+    // CG-DNA list terms of a site target (a block-uniform branch),
+    // in the launches that write no energies; the others read k_dna's (fdna)
+    constexpr bool DNA_HERE = (FEAT & F_DNA) != 0;
+    const bool dna_here = DNA_HERE && !P.write_energy;
+    __shared__ double s_dn[DNA_HERE ? NW : 1][3 + 8];
+    if constexpr (DNA_HERE) {
+        if (dna_here && wbase < ns) {
+            V3 f = {0.0, 0.0, 0.0};
+            double e[8];
+            dna_site_terms<NB, DNA_DU, true, false>(P, wbase, tid, f, e);
+            dna_block_sums<NW, false>(P, lane, wv, f, e, s_dn);
+        }
+    }
+
+    // the first partners of the pair loop, in spatial order
+    constexpr int PU = 2;   // partners per iteration (three or four only added registers)
+    double4 nx[PU];
+#pragma unroll
+    for (int u = 0; u < PU; u++) nx[u] = P.spos[min(tid + u * NB, ntot - 1)];
+
+    // the target this wavefront finishes
+    const bool mine = wv == 0;
+    int i_me = 0, rank_me = 0, itype_me = 0;
+    bool site_me = false, free_me = false;
+    double4 p_me = make_double4(0.0, 0.0, 0.0, 0.0);
+    double g_me[3] = {0.0, 0.0, 0.0};
+    if (mine) {
+        const int w = wbase;
+        i_me = w < ns ? w : w + nf;
+        site_me = i_me < ns;
+        p_me = P.pos[i_me];
+        free_me = !site_me || ((FEAT & F_DNA) && P.stfree[i_me] != 0);
+        if (!site_me) itype_me = abs(P.typei[i_me]);
+        if constexpr ((FEAT & F_UPDATE) != 0) {
+            rank_me = P.rank[i_me];
+            if (lane == 0) {
+                const double *nr = noise_row(P, i_me);
+                g_me[0] = nr[0]; g_me[1] = nr[1]; g_me[2] = nr[2];
+            }
+        }
+    }
+
+    int ti;
+    bool tsite;
+    double tx, ty, tz;
+    {
+        const int w = wbase;
+            const int i = w < ns ? w : w + nf;
+        ti = i;
+        tsite = i < ns;
+        const double4 pa = P.pos[i];
+        tx = pa.x; ty = pa.y; tz = pa.z;
+        // pair rows of this block's targets
+        const int row = __double2loint(pa.w) * nt1;
+        for (int k = tid; k < nt1; k += NB) {
+            const DevPair d = P.rows[row + k];
+            s_row[k] = d;
+            if (TAB || (d.flags & PF_EFPOT)) {
+                s_far[k] = make_double4(d.sc3, 0.0, d.fct, d.dm2hi);
+            } else {   // LJ 4 eps (s^12 - s^6) and the Coulomb term
+                const double s6 = (d.flags & PF_LJ) ? pow3(d.sgp2) : 0.0;
+                s_far[k] = make_double4(-d.epp4 * s6, d.epp4 * (s6 * s6),
+                                           (d.flags & PF_CHR) ? d.fct : 0.0,
+                                           (d.flags & PF_SRPMF) ? P.rth : -1.0);
+            }
+        }
+    }
+    // the grid corners of this wavefront's target: static field, trilinear repulsion map
+    float ph_x = 0.0f;
+    int8_t ph_v = 0;
+    bool ok_x = false, ok_v = false;
+    double chi = 0.0;
+    if constexpr ((FEAT & F_PHIX) != 0) {
+        if (mine) {
+            const GridGeom &g = P.gx;
+            ok_x = (!site_me || P.namsite[i_me] == 1) && p_me.x <= g.xbcen + g.tranx &&
+                   p_me.x >= g.xbcen - g.tranx && p_me.y <= g.ybcen + g.trany &&
+                   p_me.y >= g.ybcen - g.trany && p_me.z <= g.zbcen + g.tranz &&
+                   p_me.z >= g.zbcen - g.tranz && lane < 8;
+            if (ok_x) {
+                double x, y, z;
+                int ix, iy, iz;
+                grid_cell(g, p_me.x, p_me.y, p_me.z, x, y, z, ix, iy, iz);
+                ph_x = P.phix[tri_node(g, ix, iy, iz, lane)];
+                chi = site_me ? P.cgnuc : P.cg[itype_me];
+            }
+        }
+    }
+    if constexpr ((FEAT & F_PHIV) != 0) {
+        if (mine && !(P.flags & QBSPLINE)) {
+            const GridGeom &g = P.gv;
+            ok_v = p_me.x <= g.xbcen + g.tranx && p_me.x >= g.xbcen - g.tranx &&
+                   p_me.y <= g.ybcen + g.trany && p_me.y >= g.ybcen - g.trany &&
+                   p_me.z <= P.vzmax && p_me.z >= P.vzmin && lane < 8;
+            if (ok_v) {
+                double x, y, z;
+                int ix, iy, iz;
+                grid_cell(g, p_me.x, p_me.y, p_me.z, x, y, z, ix, iy, iz);
+                ph_v = P.phiv[vdw_map_of(P, i_me) + tri_node(g, ix, iy, iz, lane)];
+            }
+        }
+    }
+    if constexpr ((FEAT & F_UPDATE) != 0) {
+        if (mine && lane == 0) {
+            MoveFac m;
+            bd_factors(P, site_me, itype_me, p_me.z, m);
+            s_mv[0] = g_me[0]; s_mv[1] = g_me[1]; s_mv[2] = g_me[2];
+            s_mv[3] = m.fac1; s_mv[4] = m.fac2; s_mv[5] = m.ddz;
+        }
+    }
+    __syncthreads();
+
+    double fx, fy, fz, et, eel, evd, esr;
+    fx = fy = fz = et = eel = evd = esr = 0.0;
+    // PROXDIFF: per target ion, the tabulated site partner within its table range of least
+    // dist - dmi, ties to the lower site index (energy.mono.f90:603-620 in site order)
+    double pxd;
+    int pxj;
+    { pxd = INFINITY; pxj = 0x7fffffff; }
+
+    // ---- pair loop (energy.mono.f90:117-194, 584-687), compiled twice: with the energy
+    // sums, and without them for the steps that write no energies
+    const bool nonbond = (P.flags & QNONBOND) && (P.flags & QPAR);
+    auto pair_loop = [&](auto en) {
+        constexpr bool EN = decltype(en)::value;
+        for (int base = tid; base < ntot; base += 32 * NB) {
+            uint32_t m;
+            m = 0u;
+            const int cnt = min(32, (ntot - base + NB - 1) / NB);
+#pragma unroll 1
+            for (int k0 = 0; k0 < cnt; k0 += PU) {
+                // the next iteration's partners are loaded while this one's are evaluated
+                double4 pp[PU];
+#pragma unroll
+                for (int u = 0; u < PU; u++) {
+                    pp[u] = nx[u];
+                    nx[u] = P.spos[min(base + (k0 + PU + u) * NB, ntot - 1)];
+                }
+#pragma unroll
+                for (int u = 0; u < PU; u++) {
+                    const double4 pj = pp[u];
+                    const bool jok = base + (k0 + u) * NB < ntot;
+                    const int t2j = __double2loint(pj.w);
+                    const int j = __double2hiint(pj.w);
+                    {
+                        const bool on = jok && j != ti && !(tsite && j < ns);
+                        const double4 fa = s_far[t2j];
+                        const double dx = tx - pj.x, dy = ty - pj.y, dz = tz - pj.z;
+                        const double d2 = on ? pair_d2(dx, dy, dz) : 1e30;
+                        const bool near = on && d2 <= fa.w;
+                        double ri, i2;
+                        if constexpr (TAB) {
+                            ri = rsqrt_c3(d2);
+                            i2 = ri * ri;
+                        } else {
+                            recip_pair(d2, ri, i2);
+                        }
+                        const double i6 = i2 * i2 * i2, c = fa.x * i6, q = fa.z * ri;
+                        double f = 6.0 * c + q;
+                        double b = 0.0;
+                        if constexpr (!TAB) {
+                            b = fa.y * (i6 * i6);
+                            f = fma(12.0, b, f);
+                        }
+                        f = on && !near ? f * i2 : 0.0;
+                        if constexpr (EN) {
+                            // a pair's energy is counted once: by the site of a site-ion pair,
+                            // by the higher-index ion of an ion-ion pair
+                            const bool ce = on && !near && (tsite || (j >= ns && j < ti));
+                            const int fl = TAB ? (int)PF_EFPOT : s_row[t2j].flags;
+                            et += ce && (fl & PF_EFPOT) ? c + q : 0.0;
+                            if constexpr (!TAB) {
+                                eel += ce && (fl & (PF_EFPOT | PF_CHR)) == PF_CHR ? q : 0.0;
+                                evd += ce && (fl & (PF_EFPOT | PF_LJ)) == PF_LJ ? b + c : 0.0;
+                            }
+                        }
+                        m |= near ? 1u << (k0 + u) : 0u;
+                        if constexpr ((FEAT & F_PROX) != 0) {
+                            const DevPair &pr = s_row[t2j];
+                            if (near && !tsite && j < ns && (TAB || (pr.flags & PF_EFPOT)) &&
+                                !(d2 < pr.dm2lo)) {
+                                const double dd = sqrt(d2) - pr.dmi;
+                                if (dd < pxd || (dd == pxd && j < pxj)) { pxd = dd; pxj = j; }
+                            }
+                        }
+                        fx = fma(f, dx, fx);
+                        fy = fma(f, dy, fy);
+                        fz = fma(f, dz, fz);
+                    }
+                }
+            }
+            {
+                while (m) {   // the pairs in range
+                    const int k = __ffs(m) - 1;
+                    m &= m - 1u;
+                    const double4 pj = P.spos[base + k * NB];
+                    const int j = __double2hiint(pj.w);
+                    const DevPair &row = s_row[__double2loint(pj.w)];
+                    const double dx = tx - pj.x, dy = ty - pj.y, dz = tz - pj.z;
+                    const double d2 = pair_d2(dx, dy, dz);
+                    const bool ce = tsite || (j >= ns && j < ti);
+                    double f;
+                    if (TAB || (row.flags & PF_EFPOT)) {
+                        double y;
+                        f = pair_table(row, P.ep, P.ires, d2, rsqrt_c3(d2), y);
+                        if constexpr (EN) et += ce ? y : 0.0;
+                    } else {
+                        double q0 = 0.0, q1 = 0.0, q2 = 0.0;
+                        f = pair_analytic(row, P, d2, q0, q1, q2);
+                        if constexpr (EN) {
+                            eel += ce ? q0 : 0.0;
+                            evd += ce ? q1 : 0.0;
+                            esr += ce ? q2 : 0.0;
+                        }
+                    }
+                    fx = fma(f, dx, fx);
+                    fy = fma(f, dy, fy);
+                    fz = fma(f, dz, fz);
+                }
+            }
+        }
+    };
+    if (nonbond) {
+        if (P.write_energy) pair_loop(std::true_type{});
+        else pair_loop(std::false_type{});
+    }
+    __shared__ double s_pxd[(FEAT & F_PROX) ? NW : 1][1];
+    __shared__ int s_pxj[(FEAT & F_PROX) ? NW : 1][1];
+    if constexpr ((FEAT & F_PROX) != 0) {
+        {
+            double d = pxd;
+            int jj = pxj;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                const double od = __shfl_xor(d, off, WAVE);
+                const int oj = __shfl_xor(jj, off, WAVE);
+                if (od < d || (od == d && oj < jj)) { d = od; jj = oj; }
+            }
+            if (lane == 0) { s_pxd[wv][0] = d; s_pxj[wv][0] = jj; }
+        }
+    }
+
+    // forces that other kernels computed, before the sums
+    double4 f_add = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (mine && lane == 0) {
+        if constexpr ((FEAT & F_DNA) != 0) {
+            if (site_me && !dna_here) f_add = P.fdna[i_me];   // CG-DNA list terms from k_dna
+        }
+        // reaction-field forces (k_rfpair or k_mm_force)
+        if ((P.rfon || P.mmon) && !site_me) f_add = P.frf[i_me];
+    }
+
+    // pair sums to LDS (the pair accumulators are dead after this)
+    {
+        double v[7] = {fx, fy, fz, et, eel, evd, esr};
+#pragma unroll
+        for (int k = 0; k < 7; k++) {
+            if (k >= 3 && !P.write_energy) break;
+            v[k] = wave_sum(v[k]);
+            if (lane == 0) s_red[wv][k] = v[k];
+        }
+    }
+
+    // ---- grids of this wavefront's target
+    double gfx = 0.0, gfy = 0.0, gfz = 0.0, egx = 0.0, egv = 0.0;
+    bool warned = false;
+    const int t2_me = __double2loint(p_me.w);
+    if constexpr ((FEAT & F_PHIX) != 0) {
+        if (ok_x) {
+            double x, y, z;
+            int ix, iy, iz;
+            grid_cell(P.gx, p_me.x, p_me.y, p_me.z, x, y, z, ix, iy, iz);
+            tri_apply(P.gx, (double)ph_x, x, y, z, ix, iy, iz, lane, P.celec * chi, gfx, gfy, gfz, egx);
+        }
+    }
+    if constexpr ((FEAT & F_PHIV) != 0) {
+        if (P.flags & QBSPLINE) {
+            if (mine) warned = vdw_grid(P, p_me.x, p_me.y, p_me.z, t2_me, gfx, gfy, gfz, egv, vdw_map_of(P, i_me));
+        } else if (mine) {
+            if (ok_v) {
+                double x, y, z;
+                int ix, iy, iz;
+                grid_cell(P.gv, p_me.x, p_me.y, p_me.z, x, y, z, ix, iy, iz);
+                const double esvdw = (P.flags & QSVDW) ? P.svdw * P.scal[t2_me] : P.svdw;
+                tri_apply(P.gv, (double)ph_v, x, y, z, ix, iy, iz, lane, esvdw, gfx, gfy, gfz, egv);
+            }
+            warned = half_row_sum((double)ph_v) >= P.thold8 && ok_v;   // integers: exact
+        }
+    }
+    if (mine) {   // the shares of lanes 0..7, or of 27 with the B-spline
+        if (P.flags & QBSPLINE) {
+            gfx = wave_sum(gfx); gfy = wave_sum(gfy); gfz = wave_sum(gfz);
+            egx = wave_sum(egx); egv = wave_sum(egv);
+        } else {
+            gfx = half_row_sum(gfx); gfy = half_row_sum(gfy); gfz = half_row_sum(gfz);
+            if (P.write_energy) { egx = half_row_sum(egx); egv = half_row_sum(egv); }
+        }
+    }
+    __syncthreads();
+    if (!mine || lane != 0) return;
+
+    // ---- lane 0 finishes the wavefront's target
+    const int i = i_me;
+    double F[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        double acc = 0.0;
+#pragma unroll
+        for (int q = 0; q < NW; q++) acc += s_red[q][k];
+        F[k] = free_me ? acc : 0.0;   // a fixed site's pair forces are not formed
+    }
+    F[0] += gfx; F[1] += gfy; F[2] += gfz;
+    if constexpr ((FEAT & F_DNA) != 0) {
+        if (site_me && dna_here) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) F[k] += dna_site_finish<NW>(P, i, k, s_dn);
+        }
+    }
+    F[0] += f_add.x; F[1] += f_add.y; F[2] += f_add.z;
+    if (warned) atomicAdd(&P.warn[t2_me], 1);
+    if (P.flags & QMEMB) {   // MEMBRANE, membrane.f90:36-104
+        const double chg = site_me ? (P.namsite[i] == 1 ? P.cgnuc : 0.0) : P.cg[itype_me];
+        bool mw;
+        const double em = membrane_energy(P, p_me.x, p_me.y, p_me.z, chg, t2_me, F, mw);
+        if (mw) atomicAdd(&P.warn[t2_me], 1);
+        if (P.write_energy) P.epart[(size_t)E_MEMB * P.ecap + i] = em;
+    }
+    if (P.write_energy) {
+        double pe[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            double acc = 0.0;
+#pragma unroll
+            for (int q = 0; q < NW; q++) acc += s_red[q][3 + k];
+            pe[k] = acc;
+        }
+        // this kernel owns the pair and grid categories; k_dna writes the DNA ones
+        double *ep_ = P.epart + i;
+        const size_t cs = P.ecap;
+        ep_[E_GSBPA * cs] = egx;
+        ep_[E_VDWGD * cs] = egv;
+        if (site_me) {
+            ep_[E_EFPOTMX * cs] = pe[0]; ep_[E_QQMX * cs] = pe[1];
+            ep_[E_VDWMX * cs] = pe[2]; ep_[E_SRPMFMX * cs] = pe[3];
+        } else {
+            ep_[E_EFPOT * cs] = pe[0]; ep_[E_ELEC * cs] = pe[1];
+            ep_[E_VDW * cs] = pe[2]; ep_[E_SRPMF * cs] = pe[3];
+        }
+    }
+    if (P.write_forces) {
+        P.fx[i] = F[0];
+        P.fy[i] = F[1];
+        P.fz[i] = F[2];
+    }
+    if constexpr ((FEAT & F_UPDATE) != 0) {
+        // virial of the step, F . x at the positions the forces were taken at
+        // (simul1.f90:365-367); fixed ions carry no force and add nothing
+        if (P.vacc) P.vacc[i] += F[0] * p_me.x + F[1] * p_me.y + F[2] * p_me.z;
+        if (!free_me) {
+            P.poso[i] = p_me;
+            P.sposo[rank_me] = p_me;
             return;
         }
-        const double g[3] = {s_g[a][0], s_g[a][1], s_g[a][2]};
         double dids[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
         if constexpr ((FEAT & F_PROX) != 0) {
-            if (!is_site) prox_record<T, NW>(P, i, pa, a, s_pxd, s_pxj, s_row[a], dids);
+            if (!site_me) prox_record<1, NW>(P, i, p_me, 0, s_pxd, s_pxj, s_row, dids);
         }
-        const double4 pn = bd_update(P, i, is_site, pa, F, g, dids);
+        const double g[3] = {s_mv[0], s_mv[1], s_mv[2]};
+        const MoveFac m = {s_mv[3], s_mv[4], s_mv[5]};
+        const double4 pn = bd_shift(P, site_me, itype_me, p_me, F, g, m, P.nfwd, P.nbwd, dids);
         P.poso[i] = pn;
-        P.sposo[P.rank[i]] = pn;
+        P.sposo[rank_me] = pn;
     }
 }
 
@@ -921,18 +1348,28 @@ static void dispatch_wave(const StepParams &p, int feat, hipStream_t s) {
 #undef CASE
 }
 
-template <int T, int NW>
 static void dispatch_step(const StepParams &p, int feat, hipStream_t s) {
-    dim3 grid((p.tend - p.tbeg + T - 1) / T), block(NW * WAVE);
-#define CASE(F) case F: hipLaunchKernelGGL((k_step<F, T, NW>), grid, block, 0, s, p); break;
+    constexpr int NW = 2;   // four: 2300 targets 25.4 us against 22.2 (the rate blocks start at)
+    dim3 grid(p.tend - p.tbeg), block(NW * WAVE);
+#define CASE(F) case F: hipLaunchKernelGGL((k_step<F, NW>), grid, block, 0, s, p); break;
     switch (feat) { CASES16(0) CASES16(16) }
 #undef CASE
 }
 
-// BD steps of DYNAMICS3 (DNA and ions present, update on): one target per block
+template <int T>
+static void dispatch_step_wave(const StepParams &p, int feat, hipStream_t s) {
+    const int per = T * WPB;
+    dim3 grid((p.tend - p.tbeg + per - 1) / per), block(BLOCK);
+    const size_t lds = pair_lds_bytes((p.nttyp + 1) * (p.nttyp + 1));
+#define CASE(F) case F: hipLaunchKernelGGL((k_step_wave<F, T>), grid, block, lds, s, p); break;
+    switch (feat) { CASES16(0) CASES16(16) }
+#undef CASE
+}
+
+// BD steps of DYNAMICS3 (DNA and ions present, update on)
 static void dispatch_prox(const StepParams &p, int feat, hipStream_t s) {
     dim3 grid(p.tend - p.tbeg), block(BLOCK);
-#define CASE(F) case F: hipLaunchKernelGGL((k_step<F | F_PROX, 1, WPB>), grid, block, 0, s, p); break;
+#define CASE(F) case F: hipLaunchKernelGGL((k_step<F | F_PROX, WPB>), grid, block, 0, s, p); break;
     switch (feat) {
         CASE(9) CASE(11) CASE(13) CASE(15) CASE(25) CASE(27) CASE(29) CASE(31)
     }
@@ -940,8 +1377,7 @@ static void dispatch_prox(const StepParams &p, int feat, hipStream_t s) {
 }
 
 // Whether the pair kernel launch_pairs picks computes the CG-DNA list terms of its site
-// targets itself: the one-target k_step (tpb 1, and every DYNAMICS3 step) in a launch that
-// writes no energies.
+// targets itself: k_step in a launch that writes no energies.
 static bool dna_in_pairs(const StepParams &p) {
     if (tile_mode(p.tpb) || p.write_energy) return false;
     if (p.dmode == 3 && p.mode == 1) return true;
@@ -972,11 +1408,9 @@ hipError_t launch_pairs(const StepParams &p, hipStream_t s) {
         return hipGetLastError();
     }
     switch (p.tpb) {
-        // one target: two wavefronts per block, so a small system's blocks all fit in one
-        // round of waves on the 256 CUs (measured faster than four at 2300 targets)
-        case 1: dispatch_step<1, 2>(p, feat, s); break;
-        case 2: dispatch_step<2, WPB>(p, feat, s); break;
-        case 4: dispatch_step<4, WPB>(p, feat, s); break;
+        case 1: dispatch_step(p, feat, s); break;
+        case 2: dispatch_step_wave<1>(p, feat, s); break;
+        case 4: dispatch_step_wave<2>(p, feat, s); break;
         default: dispatch_wave(p, feat, s); break;   // one wavefront per target
     }
     return hipGetLastError();
