@@ -85,7 +85,7 @@ struct bromoc_ctx {
     SortBufs sb{};
     bool sort_dirty = true;
     int sort_tile = 0;                      // spos is in tile order, targets per lane (0: not)
-    int truns = 1;                          // classes and ion types that begin a tile
+    int truns = 1;                          // runs (a class and type each) that begin a tile
     int since_sort = 0;
     double r2near = 0.0;
     int cur = 0;
@@ -646,15 +646,15 @@ int bromoc_create(const bromoc_system *s, int device, bromoc_ctx **out) {
     // tile mode's order has empty slots at the end of each run: at most a tile less one each
     for (int b = 0; b < 2; b++) ACHK(dalloc(c, &c->spos[b], (size_t)cap + TILE_MAX_RUNS * 256));
     {
-        std::vector<char> seen(MAX_LDS_TYPES + 1, 0);
-        auto run_of = [&](int t2v) {
-            t2v = std::min(std::max(t2v, 0), MAX_LDS_TYPES);
-            c->truns += seen[t2v] ? 0 : 1;
-            seen[t2v] = 1;
+        // runs: the fixed ions, the sites of each type, the moving ions of each type
+        std::vector<char> seen(2 * MAX_LDS_TYPES, 0);
+        auto run_of = [&](int key) {
+            c->truns += seen[key] ? 0 : 1;
+            seen[key] = 1;
         };
         c->truns = s->nfix > 0 ? 1 : 0;
         for (int i = 0; i < ns; i++) run_of(s->typtyp[i]);
-        for (int t = s->nold + 1; t <= s->ntype; t++) run_of(s->nwtype[t]);
+        for (int t = s->nold + 1; t <= s->ntype; t++) run_of(MAX_LDS_TYPES + s->nwtype[t]);
         c->truns = std::max(c->truns, 1);
     }
     ACHK(dalloc(c, &c->sb.keys, cap));

@@ -410,17 +410,18 @@ hipError_t sort_partners(const SortBufs &b, const double4 *pos, int n, double4 *
     return hipGetLastError();
 }
 
-// key of slot k of the spatial order in the tile order: fixed ion 0, else the atnam2 type (sites
-// and ions have types of their own, sites the lower ones)
+// key of slot k of the spatial order in the tile order: fixed ions 0, then the sites by atnam2
+// type, then the moving ions by theirs.  The class is part of the key: a site and an ion may be
+// of one atnam2 type, and a tile holds one class.
 __global__ void k_type_keys(const double4 *__restrict__ spos, int n, SortGeom g, uint32_t *keys) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const double w = spos[k].w;
     const int i = __double2hiint(w), t = __double2loint(w);
-    keys[k] = i >= g.nsites && i < g.nsites + g.nfix ? 0u : (uint32_t)t;
+    keys[k] = i < g.nsites ? (uint32_t)t : i < g.nsites + g.nfix ? 0u : (uint32_t)(MAX_LDS_TYPES + t);
 }
 
-// spos over the padded slots: run t of the tile order (its first particle at hist[t * nb],
+// spos over the padded slots: run t of the tile order (key t, its first particle at hist[t * nb],
 // the scanned histogram) begins at the next multiple of tt after the run before it; slots
 // past a run's last particle are empty (index -1, at the middle of the box)
 __global__ void k_tile_gather(const double4 *__restrict__ pos, const int32_t *__restrict__ order,
@@ -429,10 +430,12 @@ __global__ void k_tile_gather(const double4 *__restrict__ pos, const int32_t *__
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nslot) return;
     int at = 0, src = -1;   // first slot of the run; the slot's place in the tile order
+    int lo = hist[0];
     for (int t = 0; t < TILE_MAX_RUNS; t++) {
-        const int lo = hist[t * nb], hi = hist[(t + 1) * nb], c = hi - lo;
+        const int hi = hist[(t + 1) * nb], c = hi - lo;
         if (s >= at && s < at + c) src = lo + (s - at);
         at += (c + tt - 1) / tt * tt;
+        lo = hi;
     }
     double4 p;
     if (src >= 0) {
@@ -447,9 +450,9 @@ __global__ void k_tile_gather(const double4 *__restrict__ pos, const int32_t *__
     spos1[s] = p;
 }
 
-// The tile order: the spatial order regrouped by type (less than MAX_LDS_TYPES of them),
-// the fixed ions first, stably, so that a tile's particles are of one type and near each
-// other.  One more radix pass over the sorted slots; order, rank and cell_start stay those of the
+// The tile order: the spatial order regrouped stably by class and type (less than
+// MAX_LDS_TYPES of them), so that a tile's particles are of one class and type (fixed ions: of
+// any) and near each other.  One more radix pass over the sorted slots; order, rank and cell_start stay those of the
 // spatial order.
 hipError_t sort_tiles(const SortBufs &b, const double4 *pos, int n, int tt, int nslot,
                       double4 *spos0, double4 *spos1, hipStream_t s) {

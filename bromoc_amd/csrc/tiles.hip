@@ -6,10 +6,10 @@
 // gathers instead, every target over all partners, which costs every pair twice.  Tile
 // mode keeps the reference's once-per-pair work and stays deterministic:
 //
-//  * the particles in tile order (sort.hip: fixed ions, then by atnam2 type, then space) are
-//    cut into tiles of TT = 64 * TPL slots; each type begins a new tile, so a tile holds
-//    fixed ions, sites of one type or moving ions of one type, and empty slots at the end
-//    of a run;
+//  * the particles in tile order (sort.hip: fixed ions, sites by atnam2 type, moving ions by
+//    theirs, each in spatial order) are cut into tiles of TT = 64 * TPL slots; each class and
+//    type begins a new tile, so a tile holds fixed ions, sites of one type or moving ions of
+//    one type, and empty slots at the end of a run;
 //  * k_tiles: one wavefront per item (I, g): tile I's particles are its targets, TPL per
 //    lane in registers, and the tiles J >= I of column group g (R consecutive tiles) pass by
 //    in chunks of 64 partners.  A chunk's positions are staged in LDS, twice in a row, so

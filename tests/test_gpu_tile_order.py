@@ -1,7 +1,8 @@
 """Tile mode's order and sweeps at their edges, against the C oracle: runs of one type that
 fill a tile exactly, miss it by one or spill one particle into the next, a type with a single
-ion, fixed ions in tiles of their own against site tiles, near and far chunks (a dense cluster
-and a far one), and enough tiles that an item takes several columns (tile_run > 1).
+ion, fixed ions in tiles of their own against site tiles, sites and ions of one atnam2 type,
+near and far chunks (a dense cluster and a far one), and enough tiles that an item takes
+several columns (tile_run > 1).
 
 Bar as the other parity tests: energies and norm-wise forces 1e-10 relative (FP64 sums of
 some 10^3 to 10^4 terms in another order, ~1e-13, and the pair forms to a few ulp).
@@ -9,7 +10,7 @@ some 10^3 to 10^4 terms in another order, ~1e-13, and the pair forms to a few ul
 import numpy as np
 import pytest
 
-from bromoc_amd import configs
+from bromoc_amd import abi, configs
 from bromoc_amd.engine import Engine
 from oracle.oracle import Oracle
 
@@ -49,6 +50,35 @@ def test_fixed_ions_against_sites(rf, tpb, monkeypatch):
     if rf:
         s = configs.with_rfpar(s, seed=3, shape=(37, 37, 55), dcel=1.0, wall_radius=12.0)
     _check(s, tpb, monkeypatch)
+
+
+@pytest.mark.parametrize("tpb", [17, 18, 20])
+@pytest.mark.parametrize("nfix", [0, 130])
+@pytest.mark.parametrize("rf", [False, True])
+def test_site_and_ion_of_one_type(rf, nfix, tpb, monkeypatch):
+    """The first ion type takes the atnam2 type of the sugars, as the C ABI allows: more than
+    a tile of sites and of ions of it.  Sites among themselves have no pair, the ions have one
+    with each other and with every site."""
+    s = configs.pore_dna(seed=9, n_bp=45, n_ions=520, box=(40.0, 40.0, 170.0), dcel=1.0,
+                         rpore=12.0, half_slab=10.0)
+    if rf:
+        s = configs.with_rfpar(s, seed=3, shape=(41, 41, 171), dcel=1.0, wall_radius=12.0)
+    s = with_fixed(s, nfix, nonfree=(0, 5, 70))
+    ion, site = s.nold + 1, int(s.typtyp[0])
+    idx = np.array(s.pairidx).reshape(s.nttyp + 1, s.nttyp + 1)
+    own = int(s.nwtype[ion])
+    for b in range(1, s.nttyp + 1):
+        if idx[own, b] and not idx[site, b]:
+            idx[site, b] = idx[b, site] = idx[own, b]
+    s.pairidx = idx.astype(np.int32).reshape(np.shape(s.pairidx))
+    s.nwtype = s.nwtype.copy()
+    s.nwtype[ion] = site
+    assert np.sum(s.typtyp == site) > 64 and np.sum(s.typei[s.nsites + nfix:] == ion) > 64
+    _check(s, tpb, monkeypatch)
+    g, o = Engine(s), Oracle(s)
+    g.step(5, abi.NOISE_PHILOX, seed=4, counter0=1)
+    o.step(5, abi.NOISE_PHILOX, seed=4, counter0=1)
+    assert float(np.max(np.abs(g.positions()[0] - o.positions()[0]))) <= 1e-9
 
 
 @pytest.mark.parametrize("tpb", [17, 18])
