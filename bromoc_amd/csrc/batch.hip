@@ -202,7 +202,7 @@ void k_batch_step(BatchParams B) {
                                 esr += ce ? q2 : 0.0;
                             }
                         } else {
-                            const double ri = rsqrt_c3(d2), i2 = ri * ri, c = tl.x * (i2 * i2 * i2);
+                            const double ri = rsqrt_s26(d2), i2 = ri * ri, c = tl.x * (i2 * i2 * i2);
                             const double fr = tl.y * ri;
                             const bool near = d2 <= tl.z;   // false for a masked pair
                             f = (6.0 * c + fr) * i2;
@@ -221,7 +221,7 @@ void k_batch_step(BatchParams B) {
                     const double4 q = pos[p];
                     const DevPair &row = rowp[__double2loint(q.w)];
                     const double dx = pa.x - q.x, dy = pa.y - q.y, dz = pa.z - q.z;
-                    const double d2 = pair_d2(dx, dy, dz), ri = rsqrt_c3(d2);
+                    const double d2 = pair_d2(dx, dy, dz), ri = rsqrt_s26(d2);
                     double y;
                     const double f = pair_table(row, P.ep, P.ires, d2, ri, y);
                     if constexpr (EN) et += p < t ? y : 0.0;

@@ -152,11 +152,19 @@ __device__ __forceinline__ void getyd(const DevPair &p, const double4 *__restric
     }
 }
 
-// 1/sqrt(d2) and 1/d2 for the analytic pair forms, each within about an ulp (1/d2 corrected by
-// its residual), with the limits of the division and the root: 0 gives infinity, infinity 0.
+// The hardware's estimate of 1/sqrt(x), good to 2^-24, cut to 26 bits: its square is exact.
+__device__ __forceinline__ double rsqrt_seed(double x) {
+    const double r = __builtin_amdgcn_rsq(x);
+    return __hiloint2double(__double2hiint(r), __double2loint(r) & (int)0xF8000000u);
+}
+
+// 1/sqrt(d2) as rsqrt_s26 forms it and 1/d2 corrected by its residual, for the analytic pair
+// forms, with the limits of the division and the root: 0 gives infinity, infinity 0.  Measured
+// against 1.0 / d2 and its sqrt over 0.1 .. 10^7: rms error 0.441 against 0.491 (units of
+// 2^-53), largest 1.00 against 1.49; of 1/d2 the same, 0.433 and 1.00.
 __device__ __forceinline__ void recip_pair(double d2, double &ri, double &i2) {
-    const double r = __builtin_amdgcn_rsq(d2);
-    const double e = fma(-d2 * r, r, 1.0);
+    const double r = rsqrt_seed(d2);
+    const double e = fma(-d2, r * r, 1.0);
     const bool reg = e == e;   // not 0 * infinity
     ri = reg ? fma(r * e, fma(0.375, e, 0.5), r) : r;
     i2 = ri * ri;
@@ -1015,10 +1023,20 @@ __device__ __forceinline__ double rsqrt_nr(double x2) {
 
 // 1/sqrt(x2) from the hardware estimate and one third-order step (the series of
 // (1 - e)^(-1/2) to e^2): the step leaves about (5/16) e^3 of the estimate's relative error
-// e, so the result is within a few ulp; for force factors, not for the table index.
+// e.  Error in units of 2^-53, rms and largest: 0.486 and 1.50 (rsqrt_nr: 0.486 and 1.24; the
+// rounding of x2 * r is in both).  For the tail and the reaction field of unmasked tile sweeps.
 __device__ __forceinline__ double rsqrt_c3(double x2) {
     const double r = __builtin_amdgcn_rsq(x2);
     const double e = fma(-x2 * r, r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
+}
+
+// The same step from an estimate whose square is exact, so that e is rounded once and the
+// result is within 2^-53 (rms 0.441): one operation more than rsqrt_c3, three fewer than
+// rsqrt_nr and closer than both.
+__device__ __forceinline__ double rsqrt_s26(double x2) {
+    const double r = rsqrt_seed(x2);
+    const double e = fma(-x2, r * r, 1.0);
     return fma(r * e, fma(0.375, e, 0.5), r);
 }
 
@@ -1036,9 +1054,11 @@ __device__ __forceinline__ double pair_d2(double dx, double dy, double dz) {
     return fma(dz, dz, fma(dy, dy, dx * dx));
 }
 
-// sqrt(d2), correctly rounded, from rinv = 1/sqrt(d2) to a few ulp: the residual of the
-// product, exact by fma, corrects it twice (the first leaves it within an ulp, the second
-// rounds the exact root, to which no double is a tie).  Zero and infinity come out as NaN.
+// sqrt(d2) from rinv = rsqrt_s26(d2): the residual of the product, exact by fma, corrects it
+// twice.  The same bits as sqrt() on 8 10^6 arguments, the 1700 whose root lies nearest a tie
+// between two doubles and the neighbours of powers of four among them (from rsqrt_c3, whose
+// error in the last place decides there, the latter came out one ulp off).  Zero and infinity
+// come out as NaN.
 __device__ __forceinline__ double root_of(double d2, double rinv) {
     const double h = 0.5 * rinv;
     double x = d2 * rinv;
@@ -1074,12 +1094,11 @@ __device__ __forceinline__ double pair_table(const DevPair &pp, const double4 *_
 // analytic tail sc3/r^6 + fct/r from rinv = 1/sqrt(d2); only lanes inside the table range
 // (d2 <= dm2hi) enter the branch that replaces it with the wall or the tabulated quadratic,
 // so far partners cost ~25 operations and near ones pay for the knot gather alone.
-// tl = (sc3, tail fct, dm2hi, unused) of the pair type.  C3: 1/r from rsqrt_c3.
-template <bool C3 = false>
+// tl = (sc3, tail fct, dm2hi, unused) of the pair type.
 __device__ __forceinline__ double pair_near_far(const DevPair &pp, const double4 &tl,
                                                const double4 *__restrict__ ep, double ires,
                                                double d2, double &y) {
-    const double rinv = C3 ? rsqrt_c3(d2) : rsqrt_nr(d2);
+    const double rinv = rsqrt_nr(d2);
     const double ix2 = rinv * rinv;
     const double c = tl.x * pow3(ix2);
     const double f = tl.y * rinv;

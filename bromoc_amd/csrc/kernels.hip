@@ -436,7 +436,7 @@ __device__ __forceinline__ void pair_sums(const StepParams &P, const DevPair *s_
                     const bool near = on && d2 <= fa.w;
                     double ri, i2;
                     if constexpr (TAB) {
-                        ri = rsqrt_c3(d2);
+                        ri = rsqrt_s26(d2);
                         i2 = ri * ri;
                     } else {
                         recip_pair(d2, ri, i2);
@@ -481,7 +481,7 @@ __device__ __forceinline__ void pair_sums(const StepParams &P, const DevPair *s_
                 double f;
                 if (TAB || (row.flags & PF_EFPOT)) {
                     double y;
-                    f = pair_table(row, P.ep, P.ires, d2, rsqrt_c3(d2), y);
+                    f = pair_table(row, P.ep, P.ires, d2, rsqrt_s26(d2), y);
                     if constexpr (EN) A.et[a] += ce ? y : 0.0;
                 } else {
                     double q0 = 0.0, q1 = 0.0, q2 = 0.0;
@@ -764,7 +764,7 @@ void k_step(StepParams P) {
                         const bool near = on && d2 <= fa.w;
                         double ri, i2;
                         if constexpr (TAB) {
-                            ri = rsqrt_c3(d2);
+                            ri = rsqrt_s26(d2);
                             i2 = ri * ri;
                         } else {
                             recip_pair(d2, ri, i2);
@@ -816,7 +816,7 @@ void k_step(StepParams P) {
                     double f;
                     if (TAB || (row.flags & PF_EFPOT)) {
                         double y;
-                        f = pair_table(row, P.ep, P.ires, d2, rsqrt_c3(d2), y);
+                        f = pair_table(row, P.ep, P.ires, d2, rsqrt_s26(d2), y);
                         if constexpr (EN) et += ce ? y : 0.0;
                     } else {
                         double q0 = 0.0, q1 = 0.0, q2 = 0.0;

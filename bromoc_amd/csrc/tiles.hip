@@ -287,9 +287,9 @@ void k_tiles(StepParams P) {
                     // w = 1/sqrt(R^2 + d2), Q = celec q srfe q' srfe' (ions' weights in qs):
                     // energy Q R w; force factor Q w^3 R; A of a target sums R w (q' srfe') and
                     // takes its factor celec q at the end, B sums Q w^3 (d2 + R / 2) reff'.
-                    auto rf_pair = [&](int u, double d2, double prr, double pqs, double &f) {
-                        const double rp = trr[u] * prr;
-                        const double w = rsqrt_c3(fma(rp, rp, d2));
+                    auto rf_pair = [&](auto masked, int u, double d2, double prr, double pqs, double &f) {
+                        const double rp = trr[u] * prr, s2 = fma(rp, rp, d2);
+                        const double w = decltype(masked)::value ? rsqrt_s26(s2) : rsqrt_c3(s2);
                         const double a = rp * w, Q = tqs[u] * pqs;
                         const double a2 = Q * w * (w * w);
                         const double a3 = a2 * fma(rp, 0.5, d2);
@@ -323,7 +323,7 @@ void k_tiles(StepParams P) {
                                 const double r = rsqrt_c3(d2), i2 = r * r, i4 = i2 * i2, fr = fc * r;
                                 double f = fma(s6 * i2, i4, fr) * i2;
                                 if constexpr (EN) e0 += fma(s3 * i2, i4, fr);
-                                if constexpr (RFW) rf_pair(u, d2, prr, pqs, f);
+                                if constexpr (RFW) rf_pair(std::false_type{}, u, d2, prr, pqs, f);
                                 add(u, f, dx, dy, dz);
                             }
                             gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
@@ -364,7 +364,7 @@ void k_tiles(StepParams P) {
                                     const bool on = !MASK || counts(u, k);
                                     if constexpr (MASK) d2 = on ? d2 : 1.0;
                                     const bool near = on && d2 <= hi;
-                                    const double r = rsqrt_c3(d2), i2 = r * r, i4 = i2 * i2, fr = fc * r;
+                                    const double r = MASK ? rsqrt_s26(d2) : rsqrt_c3(d2), i2 = r * r, i4 = i2 * i2, fr = fc * r;
                                     double f = fma(s6 * i2, i4, fr) * i2;
                                     f = on && !near ? f : 0.0;
                                     if constexpr (EN) e0 += on && !near ? fma(s3 * i2, i4, fr) : 0.0;
@@ -372,7 +372,7 @@ void k_tiles(StepParams P) {
                                     tm[w][u] |= nb;
                                     pm[w][u] |= nb;
                                     // a masked pair: zero weight and reff, so every term is zero
-                                    if constexpr (RFW) rf_pair(u, d2, on ? prr : 0.0, on ? pqs : 0.0, f);
+                                    if constexpr (RFW) rf_pair(mask_on, u, d2, on ? prr : 0.0, on ? pqs : 0.0, f);
                                     add(u, f, dx, dy, dz);
                                     pm[w][u] = wave_next(pm[w][u]);
                                 }
@@ -412,7 +412,7 @@ void k_tiles(StepParams P) {
                                     const int p = (lane + sgn * k) & (WAVE - 1);
                                     dx[h] = x0 - sx[p]; dy[h] = y0 - sy[p]; dz[h] = z0 - sz[p];
                                     d2[h] = pair_d2(dx[h], dy[h], dz[h]);
-                                    ri[h] = rsqrt_c3(d2[h]);
+                                    ri[h] = rsqrt_s26(d2[h]);
                                     int kn = (int)((root_of(d2[h], ri[h]) - dmi) * P.ires) + nxi;
                                     kn = min(max(kn, nxi), nlast);
                                     const double *kp = reinterpret_cast<const double *>(P.ep + kn);
@@ -463,7 +463,7 @@ void k_tiles(StepParams P) {
                                 if constexpr (EN) {
                                     if (on) { e1 += q0; e2 += q1; e3 += q2; }
                                 }
-                                if constexpr (RFW) rf_pair(u, d2, on ? prr : 0.0, on ? pqs : 0.0, f);
+                                if constexpr (RFW) rf_pair(std::true_type{}, u, d2, on ? prr : 0.0, on ? pqs : 0.0, f);
                                 add(u, f, dx, dy, dz);
                             }
                             gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
@@ -531,7 +531,7 @@ void k_tiles(StepParams P) {
                             const bool mx = ((tfl | pfl) & SL_SITE) != 0;
                             double y, de;
                             if (TAB || (rw.flags & PF_EFPOT)) {
-                                de = pair_near_far<false>(rw, tl, P.ep, P.ires, d2, y);
+                                de = pair_near_far(rw, tl, P.ep, P.ires, d2, y);
                                 if constexpr (EN) {
                                     if (!skip) { if (mx) en[TE_EFPOTMX] += y; else en[TE_EFPOT] += y; }
                                 }
