@@ -191,6 +191,7 @@ def test_dna_options_energy_forces(tpb, monkeypatch):
     monkeypatch.setenv("BROMOC_TPB", str(tpb))
     s = dna_options(71)
     g, o = Engine(s), Oracle(s)
+    assert g.tuning() == tpb
     eg, eo = g.energy(), o.energy()
     assert eo["ebp"] != 0.0 and eo["eqq"] != 0.0 and eo["evdwgd"] != 0.0
     _check_energy(eg, eo)

@@ -93,6 +93,7 @@ def test_debyhyb_outbox(which, tpb, monkeypatch):
     for k, i in enumerate(pk):
         s.x[i], s.y[i], s.z[i] = 18.0 - 0.05 * k, 18.0, -14.0 + 28.0 * k / len(pk)
     g, o = Engine(s), Oracle(s)
+    assert g.tuning() == tpb
     eg, eo = g.energy(), o.energy()
     bad = {k: v for k, v in energy_errs(eg, eo).items() if v > TOL}
     assert not bad, bad

@@ -32,6 +32,7 @@ def test_energy_forces(dna, bspline, tpb, monkeypatch):
     monkeypatch.setenv("BROMOC_TPB", str(tpb))
     s = _sys(61, dna, bspline)
     g, o = Engine(s), Oracle(s)
+    assert g.tuning() == tpb
     eg, eo = g.energy(), o.energy()
     assert eo["evdwgd"] != 0.0
     bad = {k: v for k, v in energy_errs(eg, eo).items() if v > TOL}

@@ -154,6 +154,7 @@ def test_repeatable_bit_for_bit(tpb, monkeypatch):
     out = []
     for _ in range(2):
         g = Engine(s)
+        assert g.tuning() == tpb
         e = g.energy()
         f = g.forces()
         g.step(33, abi.NOISE_PHILOX, seed=5, counter0=0)
@@ -173,6 +174,7 @@ def test_autotuner_picks_and_full_size_pore_dna():
         os.environ["BROMOC_TPB"] = str(tpb)
         try:
             g = Engine(s)
+            assert g.tuning() == tpb
             eg = g.energy()
         finally:
             del os.environ["BROMOC_TPB"]
