@@ -463,7 +463,7 @@ StepParams params_for(bromoc_ctx *c) {
         p.tpart = c->tpart;
         p.tener = c->tener;
         // one word per 64 slots of a row after the energies: its A and B were written
-        p.tflag = reinterpret_cast<int32_t *>(c->tener + (size_t)NTE * p.titems);
+        p.tflag = reinterpret_cast<int32_t *>(c->tener + 2 * (size_t)NTE * p.titems);
         p.rank = c->sb.trank;
     }
     return p;
@@ -476,7 +476,7 @@ constexpr size_t TILE_MAX_BYTES = size_t(3) << 30;
 int ensure_tiles(bromoc_ctx *c, int ttpl) {
     const size_t np = tile_part_doubles(c->cap, ttpl, c->truns, c->base.rfon);
     const size_t ne = tile_ener_doubles(c->cap, ttpl, c->truns);
-    if (8 * (np + ne) > TILE_MAX_BYTES)
+    if (8 * np > TILE_MAX_BYTES)
         return fail(c, BROMOC_E_CAPACITY, "tile buffers beyond their limit");
     if (np > c->tpart_n) {
         if (c->tpart) (void)hipFree(c->tpart);
@@ -1214,8 +1214,7 @@ static int autotune(bromoc_ctx *c) {
     std::vector<int> cand = {1, 2, 4, 8};
     if (tiles_allowed(c)) {
         for (int t : {1, 2, 4}) {
-            const size_t bytes = 8 * (tile_part_doubles(c->cap, t, c->truns, c->base.rfon) +
-                                      tile_ener_doubles(c->cap, t, c->truns));
+            const size_t bytes = 8 * tile_part_doubles(c->cap, t, c->truns, c->base.rfon);
             // a tile must hold enough slots for the shape to be worth timing, and the
             // partial sums must stay within their limit
             if (bytes <= TILE_MAX_BYTES && c->ntot >= 64 * t * 4 && ensure_tiles(c, t) == BROMOC_OK)

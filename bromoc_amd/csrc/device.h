@@ -87,6 +87,34 @@ __device__ __forceinline__ double wave_min(double v) {
 }
 __device__ __forceinline__ double wave_max(double v) { return -wave_min(-v); }
 
+// A sum that carries its rounding errors along (two_sum).
+struct Sum2 { double s, c; };   // sum and its accumulated error
+__device__ __forceinline__ void sum2_add(Sum2 &a, double v) {
+    const double t = a.s + v, b = t - a.s;
+    a.c += (a.s - (t - b)) + (v - b);
+    a.s = t;
+}
+__device__ __forceinline__ void sum2_add(Sum2 &a, const Sum2 &b) {
+    sum2_add(a, b.s);
+    a.c += b.c;
+}
+// the same for terms of one sign or small beside the sum (else the error is caught in part)
+__device__ __forceinline__ void sum2_fast(Sum2 &a, double v) {
+    const double t = a.s + v;
+    a.c += v - (t - a.s);
+    a.s = t;
+}
+// over the N lanes of each aligned group of a wavefront, on its first lane (all 64 active)
+template <int N>
+__device__ __forceinline__ Sum2 group_sum2(Sum2 a) {
+#pragma unroll
+    for (int off = N / 2; off > 0; off >>= 1) {
+        const Sum2 b = {__shfl_xor(a.s, off, WAVE), __shfl_xor(a.c, off, WAVE)};
+        sum2_add(a, b);
+    }
+    return a;
+}
+
 // Order-independent sums of doubles: a term v is cut at the 2^-32 grid into an integer part
 // floor(v 2^32) and W - 1 further 32-bit digits below it (units 2^-64, 2^-96), each added
 // with an integer atomic; integer addition is associative, so the total is the same

@@ -252,7 +252,8 @@ struct StepParams {
     // column groups of trun tiles; tile I's rows of partial sums are rows tile_row(I).. of
     // tpart[(row * tnc + c) * TT + t]: component c (fx, fy, fz, and with the fused reaction
     // field A, B) of slot t, first one row per lower tile, then one per group from I's own;
-    // tener[cat][item]: pair energies of each item (a tile and a group)
+    // tener[cat][item][2]: pair energies of each item (a tile and a group) and their rounding
+    // errors
     double *tpart, *tener;
     int32_t *tflag;          // [row][ttpl] 1 where a row's 64 slots hold A and B too
     int32_t ntile, ttpl, trun, titems;

@@ -1596,20 +1596,10 @@ __device__ __forceinline__ int tile_cat_of(int cat) {
 // energies (tile mode), as one sequence cut into RED_BLOCKS contiguous ranges; block b
 // sums range b (four interleaved accumulators per thread, so loads overlap, then a tree),
 // and k_reduce_finish adds the RED_BLOCKS range sums in order.  Fixed shapes throughout:
-// the same inputs give the same bits.  The sums carry their rounding errors along (two_sum):
-// tile mode's items hold pairs of one type pair, so their energies are large and of both
-// signs (10^6 against a total of 3 10^3 kcal/mol at 6000 ions), and plain sums lost a digit.
-struct Sum2 { double s, c; };   // sum and its accumulated error
-__device__ __forceinline__ void sum2_add(Sum2 &a, double v) {
-    const double t = a.s + v, b = t - a.s;
-    a.c += (a.s - (t - b)) + (v - b);
-    a.s = t;
-}
-__device__ __forceinline__ void sum2_add(Sum2 &a, const Sum2 &b) {
-    sum2_add(a, b.s);
-    a.c += b.c;
-}
-
+// the same inputs give the same bits.  The sums carry their rounding errors along, and a
+// tile item brings its sum and the error of it: tile mode's items hold pairs of one type pair,
+// so their energies are large and of both signs (10^6 against a total of 3 10^3 kcal/mol at
+// 6000 ions), and plain sums lost a digit.
 __global__ __launch_bounds__(BLOCK) void k_reduce_energy(const double *epart, int ecap, int n,
                                                          Sum2 *part, const double *tener,
                                                          int titems) {
@@ -1617,8 +1607,8 @@ __global__ __launch_bounds__(BLOCK) void k_reduce_energy(const double *epart, in
     const int cat = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     const double *src = epart + (size_t)cat * ecap;
     const int tc = tener ? tile_cat_of(cat) : -1;
-    const double *tsrc = tc >= 0 ? tener + (size_t)tc * titems : nullptr;
-    const int m = n + (tc >= 0 ? titems : 0);
+    const double *tsrc = tc >= 0 ? tener + (size_t)tc * 2 * titems : nullptr;   // (sum, error) pairs
+    const int m = n + (tc >= 0 ? 2 * titems : 0);
     const int chunk = (m + RED_BLOCKS - 1) / RED_BLOCKS;
     const int lo = b * chunk, hi = min(lo + chunk, m);
     auto val = [&](int k) { return k < n ? src[k] : tsrc[k - n]; };

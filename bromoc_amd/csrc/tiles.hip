@@ -84,7 +84,7 @@ size_t tile_ener_doubles(int cap, int ttpl, int runs) {
     const size_t nc = tile_count(cap, ttpl, runs);
     size_t m = 0;
     for (size_t n = 1; n <= nc; n++)   // energies, then the tflag words
-        m = std::max(m, (size_t)NTE * tile_items((int)n) +
+        m = std::max(m, 2 * (size_t)NTE * tile_items((int)n) +
                             ((size_t)tile_row(n, n, tile_run((int)n)) * ttpl + 1) / 2);
     return m;
 }
@@ -193,13 +193,38 @@ void k_tiles(StepParams P) {
     const int n = P.ntile, nt1 = P.nttyp + 1, R = P.trun;
     int I, g;
     item_tiles(item, R, I, g);
-    double en[EN ? NTE : 1];
-#pragma unroll
-    for (int c = 0; c < (EN ? NTE : 1); c++) en[c] = 0.0;
+    double *const eout = P.tener + 2 * (size_t)item;   // the item's pair of category 0
+    auto ener_zero = [&](int cat) { eout[2 * (size_t)cat * P.titems] = eout[2 * (size_t)cat * P.titems + 1] = 0.0; };
     if (I >= n) {   // past the last tile of a partial last group
-        if (EN && lane < NTE) P.tener[(size_t)lane * P.titems + item] = 0.0;
+        if (EN && lane < NTE) ener_zero(lane);
         return;
     }
+    // Pair energies, carried with their rounding errors: table, Coulomb, LJ, SRPMF and the
+    // reaction field.  A tile holds one class, so a chunk's pairs all are of sites and ions
+    // (mx) or none is, and along an item's chunks that changes at most once: targets that are
+    // fixed ions, whose partners go from sites to ions.  ener_end files the first four under
+    // the class that ends.  (A sum for each of the nine categories, without its error, spilled up
+    // to 193 registers and lost up to two digits of the total: 392 us an ENERGY of 12,457
+    // particles with the reaction field, 294 now.)
+    Sum2 e0 = {0.0, 0.0}, e1 = e0, e2 = e0, e3 = e0, erf = e0;
+    int eclass = -1, edone = 0;   // class of the chunks now summed; classes filed
+    auto ener_out = [&](int cat, const Sum2 &v) {
+        Sum2 t = {0.0, 0.0};
+        if (__ballot(v.s != 0.0 || v.c != 0.0) != 0ull) t = group_sum2<WAVE>(v);
+        if (lane == 0) {
+            double *const d = eout + 2 * (size_t)cat * P.titems;
+            d[0] = t.s;
+            d[1] = isfinite(t.s) ? t.c : 0.0;   // the error of an infinite sum is not a number
+        }
+    };
+    auto ener_end = [&](int mx) {
+        ener_out(mx ? TE_EFPOTMX : TE_EFPOT, e0);
+        ener_out(mx ? TE_QQMX : TE_ELEC, e1);
+        ener_out(mx ? TE_VDWMX : TE_VDW, e2);
+        ener_out(mx ? TE_SRPMFMX : TE_SRPMF, e3);
+        e0 = e1 = e2 = e3 = Sum2{0.0, 0.0};
+        edone |= 1 << mx;
+    };
     const int NC = RF ? 5 : 3;
     const int J0 = max(I, g * R), J1 = min((g + 1) * R, n);
     // targets: tile I in registers
@@ -252,6 +277,11 @@ void k_tiles(StepParams P) {
             bool rfsums = false;   // the chunk's A and B may be nonzero
             // sites among themselves and fixed ions among themselves have no pair
             if ((orI & SL_VALID) && (orJ & SL_VALID) && !(orI & orJ & (SL_SITE | SL_FIXED))) {
+                if constexpr (EN) {
+                    const int mx = ((orI | orJ) & SL_SITE) ? 1 : 0;
+                    if (eclass >= 0 && eclass != mx) ener_end(eclass);
+                    eclass = mx;
+                }
                 __builtin_amdgcn_wave_barrier();
                 C.x[lane] = o.x; C.y[lane] = o.y; C.z[lane] = o.z;
                 C.x[lane + WAVE] = o.x; C.y[lane + WAVE] = o.y; C.z[lane + WAVE] = o.z;
@@ -282,7 +312,12 @@ void k_tiles(StepParams P) {
                     // compiler from moving them across
                     __atomic_signal_fence(__ATOMIC_SEQ_CST);
                     __builtin_amdgcn_wave_barrier();
-                    double e0 = 0.0, e1 = 0.0, e2 = 0.0, e3 = 0.0, erf = 0.0;
+                    double es = 0.0, er = 0.0;   // energies of a step's TPL pairs, added at its end
+                    auto step_energies = [&] {
+                        sum2_fast(e0, es);
+                        if constexpr (RF) sum2_fast(erf, er);
+                        es = er = 0.0;
+                    };
                     // The reaction-field term of a pair (rfpar.f90:177-223) with R = reff reff',
                     // w = 1/sqrt(R^2 + d2), Q = celec q srfe q' srfe' (ions' weights in qs):
                     // energy Q R w; force factor Q w^3 R; A of a target sums R w (q' srfe') and
@@ -293,7 +328,7 @@ void k_tiles(StepParams P) {
                         const double a = rp * w, Q = tqs[u] * pqs;
                         const double a2 = Q * w * (w * w);
                         const double a3 = a2 * fma(rp, 0.5, d2);
-                        if constexpr (EN) erf = fma(Q, a, erf);
+                        if constexpr (EN) er = fma(Q, a, er);
                         wa[u] = fma(a, pqs, wa[u]);
                         wb[u] = fma(a3, prr, wb[u]);
                         ga = fma(a, tqs[u], ga);
@@ -322,10 +357,11 @@ void k_tiles(StepParams P) {
                                 const double d2 = pair_d2(dx, dy, dz);
                                 const double r = rsqrt_c3(d2), i2 = r * r, i4 = i2 * i2, fr = fc * r;
                                 double f = fma(s6 * i2, i4, fr) * i2;
-                                if constexpr (EN) e0 += fma(s3 * i2, i4, fr);
+                                if constexpr (EN) es += fma(s3 * i2, i4, fr);
                                 if constexpr (RFW) rf_pair(std::false_type{}, u, d2, prr, pqs, f);
                                 add(u, f, dx, dy, dz);
                             }
+                            if constexpr (EN) step_energies();
                             gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
                             if constexpr (RFW) { ga = wave_next(ga); gb = wave_next(gb); }
                         }
@@ -367,7 +403,7 @@ void k_tiles(StepParams P) {
                                     const double r = MASK ? rsqrt_s26(d2) : rsqrt_c3(d2), i2 = r * r, i4 = i2 * i2, fr = fc * r;
                                     double f = fma(s6 * i2, i4, fr) * i2;
                                     f = on && !near ? f : 0.0;
-                                    if constexpr (EN) e0 += on && !near ? fma(s3 * i2, i4, fr) : 0.0;
+                                    if constexpr (EN) es += on && !near ? fma(s3 * i2, i4, fr) : 0.0;
                                     const uint32_t nb = near ? bit : 0u;
                                     tm[w][u] |= nb;
                                     pm[w][u] |= nb;
@@ -376,6 +412,7 @@ void k_tiles(StepParams P) {
                                     add(u, f, dx, dy, dz);
                                     pm[w][u] = wave_next(pm[w][u]);
                                 }
+                                if constexpr (EN) step_energies();
                                 gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
                                 if constexpr (RFW) { ga = wave_next(ga); gb = wave_next(gb); }
                             }
@@ -431,7 +468,7 @@ void k_tiles(StepParams P) {
                                     if (d2[h] < lo) f = pair_wall(pr, ri[h], y);
                                     if (h == 1 && !two) f = y = 0.0;
                                     fx = fma(f, dx[h], fx); fy = fma(f, dy[h], fy); fz = fma(f, dz[h], fz);
-                                    if constexpr (EN) { if (head) e0 += y; }
+                                    if constexpr (EN) { if (head) sum2_add(e0, y); }
                                 }
                             }
                         };
@@ -461,11 +498,14 @@ void k_tiles(StepParams P) {
                                 double f = pair_analytic(pr, P, d2, q0, q1, q2);
                                 f = on ? f : 0.0;
                                 if constexpr (EN) {
-                                    if (on) { e1 += q0; e2 += q1; e3 += q2; }
+                                    sum2_fast(e1, on ? q0 : 0.0);
+                                    sum2_fast(e2, on ? q1 : 0.0);
+                                    sum2_fast(e3, on ? q2 : 0.0);
                                 }
                                 if constexpr (RFW) rf_pair(std::true_type{}, u, d2, on ? prr : 0.0, on ? pqs : 0.0, f);
                                 add(u, f, dx, dy, dz);
                             }
+                            if constexpr (EN && RFW) { sum2_fast(erf, er); er = 0.0; }
                             gx = wave_next(gx); gy = wave_next(gy); gz = wave_next(gz);
                             if constexpr (RFW) { ga = wave_next(ga); gb = wave_next(gb); }
                         }
@@ -486,13 +526,6 @@ void k_tiles(StepParams P) {
                         gb = -gb;
                     } else {
                         pick(std::false_type{});
-                    }
-                    if constexpr (EN) {
-                        en[TE_EFPOTMX] += siteI ? e0 : 0.0; en[TE_EFPOT] += siteI ? 0.0 : e0;
-                        en[TE_QQMX] += siteI ? e1 : 0.0; en[TE_ELEC] += siteI ? 0.0 : e1;
-                        en[TE_VDWMX] += siteI ? e2 : 0.0; en[TE_VDW] += siteI ? 0.0 : e2;
-                        en[TE_SRPMFMX] += siteI ? e3 : 0.0; en[TE_SRPMF] += siteI ? 0.0 : e3;
-                        en[TE_RFPAR] += erf;
                     }
                 } else {
                     C.tf[lane] = o.tf; C.tf[lane + WAVE] = o.tf;
@@ -528,22 +561,18 @@ void k_tiles(StepParams P) {
                             d2 = skip ? 1e30 : d2;
                             const DevPair &rw = P.rows[t2t * nt1 + t2p];
                             const double4 tl = make_double4(rw.sc3, rw.fct, rw.dm2hi, 0.0);
-                            const bool mx = ((tfl | pfl) & SL_SITE) != 0;
+                            const bool mx = ((tfl | pfl) & SL_SITE) != 0;   // a site: no reaction field
                             double y, de;
                             if (TAB || (rw.flags & PF_EFPOT)) {
                                 de = pair_near_far(rw, tl, P.ep, P.ires, d2, y);
-                                if constexpr (EN) {
-                                    if (!skip) { if (mx) en[TE_EFPOTMX] += y; else en[TE_EFPOT] += y; }
-                                }
+                                if constexpr (EN) sum2_add(e0, skip ? 0.0 : y);
                             } else {
                                 double q0 = 0.0, q1 = 0.0, q2 = 0.0;
                                 de = pair_analytic(rw, P, d2, q0, q1, q2);
                                 if constexpr (EN) {
-                                    if (!skip) {
-                                        en[mx ? TE_QQMX : TE_ELEC] += q0;
-                                        en[mx ? TE_VDWMX : TE_VDW] += q1;
-                                        en[mx ? TE_SRPMFMX : TE_SRPMF] += q2;
-                                    }
+                                    sum2_add(e1, skip ? 0.0 : q0);
+                                    sum2_add(e2, skip ? 0.0 : q1);
+                                    sum2_add(e3, skip ? 0.0 : q2);
                                 }
                             }
                             de = skip ? 0.0 : de;
@@ -565,7 +594,7 @@ void k_tiles(StepParams P) {
                                 const double aux2 = aux0 * srfeij * (rfdn * (rfdn * rfdn));
                                 const double aux3 = -aux2 * ((on ? d2 : 1.0) + reffij * 0.5);
                                 const double der = m * (aux2 * reffij);
-                                if constexpr (EN) en[TE_RFPAR] = fma(m, aux1 * srfeij, en[TE_RFPAR]);
+                                if constexpr (EN) sum2_add(erf, m * (aux1 * srfeij));
                                 aa_[u] = fma(m, -aux1 * psr, aa_[u]);
                                 ab_[u] = fma(m, aux3 * prr, ab_[u]);
                                 ga = fma(m, -aux1 * tsr[u], ga);
@@ -626,10 +655,11 @@ void k_tiles(StepParams P) {
         }
     }
     if constexpr (EN) {
-#pragma unroll
-        for (int c = 0; c < NTE; c++) {
-            const double v = wave_sum(en[c]);
-            if (lane == 0) P.tener[(size_t)c * P.titems + item] = v;
+        if (eclass >= 0) ener_end(eclass);
+        ener_out(TE_RFPAR, erf);
+        if (lane == 0) {   // the classes the item has no pair of
+            if (!(edone & 1)) { ener_zero(TE_EFPOT); ener_zero(TE_ELEC); ener_zero(TE_VDW); ener_zero(TE_SRPMF); }
+            if (!(edone & 2)) { ener_zero(TE_EFPOTMX); ener_zero(TE_QQMX); ener_zero(TE_VDWMX); ener_zero(TE_SRPMFMX); }
         }
     }
 }
@@ -642,10 +672,11 @@ __device__ __forceinline__ double group8_sum(double v) {
     return v;
 }
 
-// k_tfin: slot s of the spatial order, eight lanes per slot (32 slots per block).  The
-// lanes split the slot's partial rows, then its grid corners (lane c takes corner c
-// of the trilinear stencils, c, c + 8, .. of the 27-node B-spline); lane 0 of the group
-// finishes the particle.  Sites and moving ions are finished as by k_step; a fixed ion
+// k_tfin: slot s of the tile order, eight lanes per slot (32 slots per block).  The
+// lanes split the slot's partial rows -- rows of one type pull one way and those of the next
+// the other, so the sums carry their rounding errors -- then its grid corners (lane c takes
+// corner c of the trilinear stencils, c, c + 8, .. of the 27-node B-spline); lane 0 of the
+// group finishes the particle.  Sites and moving ions are finished as by k_step; a fixed ion
 // only receives its reaction-field force (rfpar.f90:177-223 applies it to both ions of a
 // pair), written when forces are asked for.
 template <int FEAT>
@@ -661,7 +692,7 @@ __global__ __launch_bounds__(BLOCK) void k_tfin(StepParams P) {
     const bool is_site = i < ns, fixed = !is_site && i < ns + P.nfix;
     const int TT = WAVE * P.ttpl, n = P.ntile, NC = RF ? 5 : 3, R = P.trun;
     const int I = ss / TT, t = ss - I * TT;
-    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    Sum2 sum[5] = {};
     // the slot's rows: one per lower tile, one per column group from its own; rows K = sub,
     // sub + 8, .. added in that order, KU of them per iteration so that their
     // loads (the flags, then the rows) are in flight together
@@ -694,16 +725,23 @@ __global__ __launch_bounds__(BLOCK) void k_tfin(StepParams P) {
                 if (ab[u]) { r[u][3] = src[u][3 * (size_t)TT]; r[u][4] = src[u][4 * (size_t)TT]; }
             }
         }
+        // KU rows plainly, their sum with its rounding error: no slower than plain sums (row by
+        // row that took 0.12 ms more of 3 at 56,000 particles)
 #pragma unroll
-        for (int u = 0; u < KU; u++) {
-            if (!ok[u]) continue;
+        for (int c = 0; c < NC; c++) {
+            double v = 0.0;
 #pragma unroll
-            for (int c = 0; c < NC; c++)
-                if (c < 3 || ab[u]) acc[c] += r[u][c];
+            for (int u = 0; u < KU; u++)
+                if (ok[u] && (c < 3 || ab[u])) v += r[u][c];
+            sum2_add(sum[c], v);
         }
     }
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = group8_sum(acc[c]);
+    for (int c = 0; c < NC; c++) {
+        const Sum2 t = group_sum2<8>(sum[c]);
+        acc[c] = isfinite(t.s) ? t.s + t.c : t.s;   // the error of an infinite sum is not a number
+    }
 
     // grids of a target (a site or a moving ion): staticf1.f90:45-118, vdwgd1trln.f90:
     // 50-161 / vdwgd1spln.f90:50-170, corners split over the group's lanes

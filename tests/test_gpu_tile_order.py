@@ -1,8 +1,8 @@
 """Tile mode's order and sweeps at their edges, against the C oracle: runs of one type that
 fill a tile exactly, miss it by one or spill one particle into the next, a type with a single
 ion, fixed ions in tiles of their own against site tiles, sites and ions of one atnam2 type,
-near and far chunks (a dense cluster and a far one), and enough tiles that an item takes
-several columns (tile_run > 1).
+near and far chunks (a dense cluster and a far one), enough tiles that an item takes
+several columns (tile_run > 1), and the rounding of the energy sum.
 
 Bar as the other parity tests: energies and norm-wise forces 1e-10 relative (FP64 sums of
 some 10^3 to 10^4 terms in another order, ~1e-13, and the pair forms to a few ulp).
@@ -91,6 +91,41 @@ def test_near_and_far_clusters(tpb, monkeypatch):
     p = np.concatenate([g, g + [60.0, 5.0, 70.0]]) + rng.uniform(-0.4, 0.4, (400, 3))
     s.x, s.y, s.z = (p[:, k].copy() for k in range(3))
     _check(s, tpb, monkeypatch)
+
+
+@pytest.mark.parametrize("tpb", [17, 18, 20])
+@pytest.mark.parametrize("analytic", [False, True])
+def test_energies_lose_nothing_to_the_order(analytic, tpb, monkeypatch):
+    """A tile holds one type, so an item's energies all have one sign and the items cancel:
+    10^5 kcal/mol of pairs in a sum of 10^1.  Ions beyond table range of each other (fct / r
+    pairs only); the sum of the exact terms, each off by at most 2^-53 or two of itself
+    (0.6 rms), is off by 0.6 2^-53 sqrt(sum of squares), and ten times that is allowed."""
+    monkeypatch.setenv("BROMOC_TPB", str(tpb))
+    m, n = 12, 1531
+    s = plain(seed=2, n_per_type=(n + 1) // 2, box=24.0 * m + 10.0).copy()
+    rng = np.random.default_rng(2)
+    g = (np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3) - 0.5 * (m - 1)) * 24.0
+    p = g[rng.permutation(len(g))[:n]] + rng.uniform(-1.5, 1.5, (n, 3))
+    s.ntot = s.capacity = n
+    s.x, s.y, s.z = (np.ascontiguousarray(p[:, k]) for k in range(3))
+    s.typei = rng.permutation(1 + np.arange(n) % 2).astype(np.int32)
+    if analytic:
+        s = configs.with_analytic(s, seed=1, lj=False, srpmf=False)
+    else:
+        s.pairs = [None if q is None else dict(q, sc3=0.0) for q in s.pairs]
+    long = np.longdouble
+    fct = np.array([0.0 if q is None else q["fct"] for q in s.pairs])[np.reshape(s.pairidx, (s.nttyp + 1, -1))]
+    t2, total, sq = s.nwtype[s.typei], long(0), long(0)
+    for i in range(1, n):
+        d = p[i].astype(long) - p[:i]
+        v = fct[t2[i], t2[:i]] / np.sqrt((d * d).sum(1))
+        total, sq = total + v.sum(), sq + (v * v).sum()
+    e = Engine(s)
+    assert e.tuning() == tpb
+    got = e.energy()["eelec" if analytic else "eefpot"]
+    err = abs(long(got) - total) / (long(2.0) ** -53 * np.sqrt(sq))
+    print(f"analytic {analytic} tpb {tpb}: energy {got:.3f}, error {float(err):.2f} 2^-53 sqrt(sum of squares)")
+    assert err <= 6.0 + abs(total) / np.sqrt(sq)
 
 
 def test_items_of_several_columns(monkeypatch):
