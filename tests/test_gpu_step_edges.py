@@ -1,15 +1,18 @@
 """The step kernels' shapes (1: a block per target; 2, 4: one, two targets a wavefront) where
 their splits have edges: one target, targets that leave a wavefront or a block part empty,
 partners about the 64 lanes and about the 32 a lane notes at once (2048 with one wavefront, 4096
-with two); table pairs, and analytic pairs with SRPMF in range.
+with two); table pairs, and analytic pairs with SRPMF in range.  And that picking among the
+shapes costs little beside a run.
 
 Against the C oracle: energies and norm-wise forces 1e-10 relative, as the other parity tests
 (FP64 sums of up to 4100 terms in another order, ~1e-13, and pair forms to a few ulp).
 """
+import time
+
 import numpy as np
 import pytest
 
-from bromoc_amd import configs
+from bromoc_amd import abi, configs
 from bromoc_amd.engine import Engine
 from oracle.oracle import Oracle
 
@@ -52,3 +55,24 @@ def test_table_pairs(n, tpb, monkeypatch):
 def test_analytic_pairs(n, tpb, monkeypatch):
     s = configs.with_analytic(_first(_ions(n), n), seed=n)
     _check(s, tpb, monkeypatch)
+
+
+def test_tuning_drops_losers():
+    """Analytic ions, where the slowest shape takes sixty times the fastest: the tuning takes
+    the time of 340 steps when slow shapes are dropped after a first round, of 1600 when every
+    shape is timed to the end."""
+    n = 1531
+    s = configs.with_analytic(_first(_ions(n), n), seed=n)
+    tune, step = [], []
+    for _ in range(3):
+        g = Engine(s)
+        t0 = time.perf_counter()
+        g.tuning()
+        tune.append(time.perf_counter() - t0)
+        g.step(64, abi.NOISE_PHILOX, seed=1, counter0=0)
+        t0 = time.perf_counter()
+        g.step(128, abi.NOISE_PHILOX, seed=1, counter0=64)
+        step.append((time.perf_counter() - t0) / 128)
+    ratio = min(tune) / min(step)
+    print(f"tuning {1e3 * min(tune):.1f} ms, {ratio:.0f} steps")
+    assert ratio < 750
