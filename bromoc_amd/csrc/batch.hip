@@ -558,6 +558,8 @@ constexpr int BATCH_GRAPH_K = 32;   // steps per captured graph without GCMC
 // steps whose noise is drawn by one launch, within a bounded buffer
 constexpr int BATCH_NOISE_ROWS = 16;
 constexpr size_t BATCH_NOISE_BYTES = size_t(256) << 20;
+// slots of a replica that bromoc_batch_get stages at a time (1 MiB of pinned memory)
+constexpr size_t BATCH_GET_SLOTS = 32768;
 
 template <typename T>
 hipError_t balloc(std::vector<void *> &al, T **p, size_t n) {
@@ -1070,8 +1072,9 @@ int bromoc_batch_get(bromoc_batch *b, int32_t r, double *x, double *y, double *z
                      int32_t *ntot, int32_t *ibuffer, int32_t *nat, double *gcmc_ener) {
     if (!b || r < 0 || r >= b->nrep) return BROMOC_E_ARG;
     (void)hipSetDevice(b->device);
-    // everything in one launch through pinned memory, laid out by the replica's capacity
-    const size_t cap = b->h_cap[r], nb = b->h_nbuf[r];
+    // everything in one launch through pinned memory, laid out by the replica's capacity; a
+    // replica of more than BATCH_GET_SLOTS particles in several, so that what is pinned is bounded
+    const size_t cap = std::min<size_t>(b->h_cap[r], BATCH_GET_SLOTS), nb = b->h_nbuf[r];
     const size_t bytes = sizeof(double) * (3 * cap + 1) + sizeof(int32_t) * (2 * cap + nb + 1);
     if (bytes > b->pin_cap) {
         if (b->pin) (void)hipHostFree(b->pin);
@@ -1084,6 +1087,7 @@ int bromoc_batch_get(bromoc_batch *b, int32_t r, double *x, double *y, double *z
     const BatchParams &B = b->base;
     a.r = r;
     a.nbuf = (int32_t)nb;
+    a.max = (int32_t)cap;
     a.ntot = B.ntot; a.off = B.off;
     a.pos = b->pos[b->cur];
     a.typei = B.typei; a.ibuffer = B.ibuffer;
@@ -1093,15 +1097,20 @@ int bromoc_batch_get(bromoc_batch *b, int32_t r, double *x, double *y, double *z
     a.o_x = a.o_ener + 1; a.o_y = a.o_x + cap; a.o_z = a.o_y + cap;
     a.o_n = (int32_t *)(a.o_z + cap);
     a.o_nat = a.o_n + 1; a.o_ty = a.o_nat + nb; a.o_ib = a.o_ty + cap;
-    BCHK(b, launch_stage_replica(a, (int)cap, b->stream));
-    int st = batch_sync(b);
-    if (st) return st;
-    const int32_t n = a.o_n[0];
-    if (x) std::copy(a.o_x, a.o_x + n, x);
-    if (y) std::copy(a.o_y, a.o_y + n, y);
-    if (z) std::copy(a.o_z, a.o_z + n, z);
-    if (typei) std::copy(a.o_ty, a.o_ty + n, typei);
-    if (ibuffer) std::copy(a.o_ib, a.o_ib + n, ibuffer);
+    int32_t n = 0;
+    do {
+        BCHK(b, launch_stage_replica(a, b->stream));
+        int st = batch_sync(b);
+        if (st) return st;
+        n = a.o_n[0];
+        const int32_t m = std::min(n - a.lo, a.max);
+        if (x) std::copy(a.o_x, a.o_x + m, x + a.lo);
+        if (y) std::copy(a.o_y, a.o_y + m, y + a.lo);
+        if (z) std::copy(a.o_z, a.o_z + m, z + a.lo);
+        if (typei) std::copy(a.o_ty, a.o_ty + m, typei + a.lo);
+        if (ibuffer) std::copy(a.o_ib, a.o_ib + m, ibuffer + a.lo);
+        a.lo += m;
+    } while (a.lo < n);
     if (nat) {
         nat[0] = 0;
         std::copy(a.o_nat, a.o_nat + nb, nat + 1);

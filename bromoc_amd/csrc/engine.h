@@ -358,8 +358,8 @@ struct StageCopies {           // arrays of 32-bit words, copied by one launch
         src[n] = s; dst[n] = d; words[n] = (int64_t)(bytes / 4); n++;
     }
 };
-struct StageReplica {          // one replica of a batch
-    int32_t r, nbuf;
+struct StageReplica {          // one replica of a batch, its slots lo .. lo + max - 1
+    int32_t r, nbuf, lo, max;
     const int32_t *ntot, *off;
     const double4 *pos;
     const int32_t *typei, *ibuffer, *nat;
@@ -373,7 +373,7 @@ hipError_t launch_stage_pos_in(const double *x, const double *y, const double *z
                                const int32_t *t2h, const int32_t *tyh, int n, double4 *p0,
                                double4 *p1, int32_t *t2, int32_t *ty, hipStream_t s);
 hipError_t launch_stage_copy(const StageCopies &c, hipStream_t s);
-hipError_t launch_stage_replica(const StageReplica &a, int cap, hipStream_t s);
+hipError_t launch_stage_replica(const StageReplica &a, hipStream_t s);
 
 // ---- GRAND of one system on the device (grand.hip)
 constexpr int GC_BLOCKS = 256;   // workgroups of k_gc_interact (partials per attempt)

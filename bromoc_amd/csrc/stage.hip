@@ -50,17 +50,18 @@ __global__ __launch_bounds__(ST_BLOCK) void k_stage_copy(StageCopies c) {
         d[i] = s[i];
 }
 
-// one replica of a batch: its count, energy and buffer counts, then its particles
+// one replica of a batch: its count, energy and buffer counts, then its particles from lo on
 __global__ __launch_bounds__(ST_BLOCK) void k_stage_replica(StageReplica a) {
     const int n = a.ntot[a.r], off = a.off[a.r];
     const int t = blockIdx.x * ST_BLOCK + threadIdx.x;
     if (t == 0) { a.o_n[0] = n; a.o_ener[0] = a.gener[a.r]; }
     if (t < a.nbuf) a.o_nat[t] = a.nat[t];
-    for (int i = t; i < n; i += gridDim.x * ST_BLOCK) {
-        const double4 p = a.pos[off + i];
+    for (int i = t; i < min(n - a.lo, a.max); i += gridDim.x * ST_BLOCK) {
+        const int s = off + a.lo + i;
+        const double4 p = a.pos[s];
         a.o_x[i] = p.x; a.o_y[i] = p.y; a.o_z[i] = p.z;
-        a.o_ty[i] = a.typei[off + i];
-        a.o_ib[i] = a.ibuffer[off + i];
+        a.o_ty[i] = a.typei[s];
+        a.o_ib[i] = a.ibuffer[s];
     }
 }
 
@@ -86,8 +87,8 @@ hipError_t launch_stage_copy(const StageCopies &c, hipStream_t s) {
     hipLaunchKernelGGL(k_stage_copy, g, dim3(ST_BLOCK), 0, s, c);
     return hipGetLastError();
 }
-hipError_t launch_stage_replica(const StageReplica &a, int cap, hipStream_t s) {
-    hipLaunchKernelGGL(k_stage_replica, st_grid(cap > a.nbuf ? cap : a.nbuf), dim3(ST_BLOCK), 0, s, a);
+hipError_t launch_stage_replica(const StageReplica &a, hipStream_t s) {
+    hipLaunchKernelGGL(k_stage_replica, st_grid(a.max > a.nbuf ? a.max : a.nbuf), dim3(ST_BLOCK), 0, s, a);
     return hipGetLastError();
 }
 
