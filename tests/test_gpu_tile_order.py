@@ -128,6 +128,38 @@ def test_energies_lose_nothing_to_the_order(analytic, tpb, monkeypatch):
     assert err <= 6.0 + abs(total) / np.sqrt(sq)
 
 
-def test_items_of_several_columns(monkeypatch):
-    s = plain(seed=6, n_per_type=6100)
+def _tiles(n, runs=2):
+    """Tiles of 64 slots and tiles per column group of n particles, as the library has them."""
+    lib = abi.load_library()
+    tiles = lib._ZN6bromoc10tile_countEiii(n, 1, runs)
+    return tiles, lib._ZN6bromoc8tile_runEi(tiles)
+
+
+def _two_types(a, b):
+    n = a + b
+    s = plain(seed=a, n_per_type=(n + 1) // 2, box=8.5 * n ** (1.0 / 3.0)).copy()
+    s.ntot = s.capacity = n
+    s.x, s.y, s.z = s.x[:n].copy(), s.y[:n].copy(), s.z[:n].copy()
+    s.typei = np.random.default_rng(n).permutation([1] * a + [2] * b).astype(np.int32)
+    return s
+
+
+@pytest.mark.parametrize("a,b,run,left", [(8160, 8160, 2, 0), (8193, 8190, 2, 1), (11600, 11500, 4, 2),
+                                          (16210, 16150, 8, 3)])
+def test_items_of_several_columns(a, b, run, left, monkeypatch):
+    """Column groups of 2, 4 and 8 tiles, the last one whole or partial."""
+    tiles, r = _tiles(a + b)
+    assert r == run and tiles % run == left
+    _check(_two_types(a, b), 17, monkeypatch)
+
+
+def test_several_columns_with_reaction_field_and_steps(monkeypatch):
+    a, b = 8193, 8190
+    tiles, r = _tiles(a + b)
+    assert r == 2 and tiles % 2 == 1
+    s = configs.with_rfpar(_two_types(a, b), seed=3, shape=(45, 45, 45), dcel=5.0)
     _check(s, 17, monkeypatch)
+    g, o = Engine(s), Oracle(s)
+    g.step(2, abi.NOISE_PHILOX, seed=4, counter0=1)
+    o.step(2, abi.NOISE_PHILOX, seed=4, counter0=1)
+    assert float(np.max(np.abs(g.positions()[0] - o.positions()[0]))) <= 1e-9
