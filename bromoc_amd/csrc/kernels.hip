@@ -590,14 +590,18 @@ __global__ __launch_bounds__(BLOCK) void k_step_wave(StepParams P) {
 // writes no energies (the step loop) the block computes its site target's CG-DNA list terms
 // itself (dna_site_terms); otherwise the site targets read them from k_dna (fdna).  The pair
 // loop is pair_sums' with one target and the block's registers in mind (five wavefronts a
-// SIMD): what the end needs is parked in LDS.
+// SIMD; three with analytic pairs, which spill 47 to 110 registers at four and none at three:
+// 2500 particles with DNA and some analytic pair types 41 -> 32 us a step, 36 with a branch a
+// pair before, 40 with two wavefronts): what the end needs is parked in LDS.  DYNAMICS3 looks for
+// an ion's nearest site among the pairs in range as they are worked off (in the pair loop 31 us at
+// 2500 particles, 28.5 here).
 //
 // A step of a small system is one chain of loads behind the launch (5.0 us a step with two
 // ions): 400 ions 7.3 us, 2300 with DNA 22.8 -> 22.0 us, of that 10 us without pair loop and
 // list terms, mostly the rate at which blocks start.
 template <int FEAT, int NW>
 __global__ __launch_bounds__(NW * WAVE)
-__attribute__((amdgpu_waves_per_eu((FEAT & F_TAB) ? 5 : 4)))
+__attribute__((amdgpu_waves_per_eu((FEAT & F_TAB) ? 5 : 3)))
 void k_step(StepParams P) {
     constexpr int NB = NW * WAVE;   // threads of the block
     constexpr bool TAB = (FEAT & F_TAB) != 0;
@@ -789,14 +793,6 @@ void k_step(StepParams P) {
                             }
                         }
                         m |= near ? 1u << (k0 + u) : 0u;
-                        if constexpr ((FEAT & F_PROX) != 0) {
-                            const DevPair &pr = s_row[t2j];
-                            if (near && !tsite && j < ns && (TAB || (pr.flags & PF_EFPOT)) &&
-                                !(d2 < pr.dm2lo)) {
-                                const double dd = sqrt(d2) - pr.dmi;
-                                if (dd < pxd || (dd == pxd && j < pxj)) { pxd = dd; pxj = j; }
-                            }
-                        }
                         fx = fma(f, dx, fx);
                         fy = fma(f, dy, fy);
                         fz = fma(f, dz, fz);
@@ -818,6 +814,12 @@ void k_step(StepParams P) {
                         double y;
                         f = pair_table(row, P.ep, P.ires, d2, rsqrt_s26(d2), y);
                         if constexpr (EN) et += ce ? y : 0.0;
+                        if constexpr ((FEAT & F_PROX) != 0) {
+                            if (!tsite && j < ns && !(d2 < row.dm2lo)) {
+                                const double dd = sqrt(d2) - row.dmi;
+                                if (dd < pxd || (dd == pxd && j < pxj)) { pxd = dd; pxj = j; }
+                            }
+                        }
                     } else {
                         double q0 = 0.0, q1 = 0.0, q2 = 0.0;
                         f = pair_analytic(row, P, d2, q0, q1, q2);
