@@ -472,7 +472,7 @@ StepParams params_for(bromoc_ctx *c) {
 // Tile-mode buffers for the context's capacity at ttpl targets per lane (kept; grown when
 // a larger shape needs more).  Fails with BROMOC_E_CAPACITY when they would pass
 // TILE_MAX_BYTES.
-constexpr size_t TILE_MAX_BYTES = size_t(3) << 30;
+constexpr size_t TILE_MAX_BYTES = (size_t(3) << 30) + (size_t(32) << 20);   // the runs' tiles: some MiB
 int ensure_tiles(bromoc_ctx *c, int ttpl) {
     const size_t np = tile_part_doubles(c->cap, ttpl, c->truns, c->base.rfon);
     const size_t ne = tile_ener_doubles(c->cap, ttpl, c->truns);
@@ -646,15 +646,20 @@ int bromoc_create(const bromoc_system *s, int device, bromoc_ctx **out) {
     // tile mode's order has empty slots at the end of each run: at most a tile less one each
     for (int b = 0; b < 2; b++) ACHK(dalloc(c, &c->spos[b], (size_t)cap + TILE_MAX_RUNS * 256));
     {
-        // runs: the fixed ions, the sites of each type, the moving ions of each type
-        std::vector<char> seen(2 * MAX_LDS_TYPES, 0);
-        auto run_of = [&](int key) {
-            c->truns += seen[key] ? 0 : 1;
-            seen[key] = 1;
+        // runs: the fixed ions, the sites and the moving ions of each type; an ion may change
+        // its type later (bromoc_set_positions)
+        std::vector<char> seen(TILE_MAX_RUNS, 0);
+        auto run_of = [&](int cls, int t2v) {
+            char &k = seen[cls * MAX_LDS_TYPES + t2v];
+            c->truns += k ? 0 : 1;
+            k = 1;
         };
-        c->truns = s->nfix > 0 ? 1 : 0;
-        for (int i = 0; i < ns; i++) run_of(s->typtyp[i]);
-        for (int t = s->nold + 1; t <= s->ntype; t++) run_of(MAX_LDS_TYPES + s->nwtype[t]);
+        c->truns = 0;
+        for (int i = 0; i < ns; i++) run_of(1, s->typtyp[i]);
+        for (int t = s->nold + 1; t <= s->ntype; t++) {
+            if (s->nfix > 0) run_of(0, s->nwtype[t]);
+            run_of(2, s->nwtype[t]);
+        }
         c->truns = std::max(c->truns, 1);
     }
     ACHK(dalloc(c, &c->sb.keys, cap));

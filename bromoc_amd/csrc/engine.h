@@ -264,7 +264,7 @@ constexpr int TPB_TILE = 16;
 // items wanted of a grouping (tile_run): four rounds of the chip's 4,096 resident wavefronts
 constexpr int TILE_MIN_ITEMS = 16384;
 int tile_run(int n);               // tiles per column group of n tiles
-// tiles that hold n particles in `runs` runs (fixed ions, sites and ions of each type), each beginning a tile (an
+// tiles that hold n particles in `runs` runs (a class and type each), each beginning a tile (an
 // upper bound: the runs' sizes are known on the device only)
 int tile_count(int n, int ttpl, int runs);
 int tile_items(int n);
@@ -301,7 +301,7 @@ struct SortBufs {
 size_t sort_hist_ints(int n);
 hipError_t sort_partners(const SortBufs &b, const double4 *pos, int n, double4 *spos0,
                          double4 *spos1, hipStream_t s);
-// tile mode: after sort_partners, spos regrouped stably (fixed ions, sites by type, moving ions by type), each run
+// tile mode: after sort_partners, spos regrouped stably by class and type, each run
 // from a multiple of tt slots on, over nslot slots (torder, trank)
 hipError_t sort_tiles(const SortBufs &b, const double4 *pos, int n, int tt, int nslot,
                       double4 *spos0, double4 *spos1, hipStream_t s);
@@ -332,7 +332,7 @@ hipError_t launch_tiles(const StepParams &p, hipStream_t s, int which = 3);
 // reaction field: rf != 0)
 size_t tile_part_doubles(int cap, int ttpl, int runs, int rf);
 size_t tile_ener_doubles(int cap, int ttpl, int runs);
-constexpr int TILE_MAX_RUNS = 2 * MAX_LDS_TYPES;   // fixed ions (0), sites by type, ions by type
+constexpr int TILE_MAX_RUNS = 3 * MAX_LDS_TYPES;   // fixed ions, sites, moving ions by type
 hipError_t launch_advance(int64_t *ctr, int64_t by, hipStream_t s);
 hipError_t launch_philox_fill(const int64_t *ctl, uint64_t stream, int nrows, int ntot,
                               int64_t stride, double *out, hipStream_t s);

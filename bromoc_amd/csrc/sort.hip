@@ -410,15 +410,16 @@ hipError_t sort_partners(const SortBufs &b, const double4 *pos, int n, double4 *
     return hipGetLastError();
 }
 
-// key of slot k of the spatial order in the tile order: fixed ions 0, then the sites by atnam2
-// type, then the moving ions by theirs.  The class is part of the key: a site and an ion may be
+// key of slot k of the spatial order in the tile order: the fixed ions by atnam2 type, then the
+// sites, then the moving ions by theirs.  The class is part of the key: a site and an ion may be
 // of one atnam2 type, and a tile holds one class.
 __global__ void k_type_keys(const double4 *__restrict__ spos, int n, SortGeom g, uint32_t *keys) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const double w = spos[k].w;
     const int i = __double2hiint(w), t = __double2loint(w);
-    keys[k] = i < g.nsites ? (uint32_t)t : i < g.nsites + g.nfix ? 0u : (uint32_t)(MAX_LDS_TYPES + t);
+    const int cls = i < g.nsites ? 1 : i < g.nsites + g.nfix ? 0 : 2;
+    keys[k] = (uint32_t)(cls * MAX_LDS_TYPES + t);
 }
 
 // spos over the padded slots: run t of the tile order (key t, its first particle at hist[t * nb],
@@ -451,8 +452,8 @@ __global__ void k_tile_gather(const double4 *__restrict__ pos, const int32_t *__
 }
 
 // The tile order: the spatial order regrouped stably by class and type (less than
-// MAX_LDS_TYPES of them), so that a tile's particles are of one class and type (fixed ions: of
-// any) and near each other.  One more radix pass over the sorted slots; order, rank and cell_start stay those of the
+// MAX_LDS_TYPES of them), so that a tile's particles are of one class and type and near each
+// other.  One more radix pass over the sorted slots; order, rank and cell_start stay those of the
 // spatial order.
 hipError_t sort_tiles(const SortBufs &b, const double4 *pos, int n, int tt, int nslot,
                       double4 *spos0, double4 *spos1, hipStream_t s) {

@@ -81,6 +81,23 @@ def test_site_and_ion_of_one_type(rf, nfix, tpb, monkeypatch):
     assert float(np.max(np.abs(g.positions()[0] - o.positions()[0]))) <= 1e-9
 
 
+@pytest.mark.parametrize("tpb", [17, 18, 20])
+@pytest.mark.parametrize("counts,nfix", [((64, 64), 0), ((65, 127), 0), ((300, 217), 70)])
+def test_ions_on_zero_cells(counts, nfix, tpb, monkeypatch):
+    """Ions inside the reaction-field grid with srfe = 0 beside ions with a value: whether a
+    pair counts depends on their order, so the tiles take the reaction field in a masked sweep
+    of its own.  A wall of zeros leaves whole tiles without a value."""
+    a, b = counts
+    n = a + b
+    s = plain(seed=n, n_per_type=(n + 1) // 2).copy()
+    s.ntot = s.capacity = n
+    s.x, s.y, s.z = s.x[:n].copy(), s.y[:n].copy(), s.z[:n].copy()
+    s.typei = np.random.default_rng(n).permutation([1] * a + [2] * b).astype(np.int32)
+    s = configs.with_rfpar(with_fixed(s, nfix), seed=3, shape=(45, 45, 45), dcel=1.2, zero_frac=0.1,
+                           wall_radius=14.0)
+    _check(s, tpb, monkeypatch)
+
+
 @pytest.mark.parametrize("tpb", [17, 18])
 def test_near_and_far_clusters(tpb, monkeypatch):
     """Two dense clusters further apart than the tables reach: pairs in range at most steps
