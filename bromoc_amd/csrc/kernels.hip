@@ -220,9 +220,10 @@ __device__ inline double dna_site_finish(const StepParams &P, int i, int c,
 }
 
 // The far form of a pair type: r^-6, r^-12 and 1/r factors, range^2 (< 0: none).  A table pair's
-// tail, or LJ 4 eps (s^12 - s^6) and the Coulomb term.
+// tail, or LJ 4 eps (s^12 - s^6) and the Coulomb term.  With table pairs only (tab) the second is
+// six times the first instead, the force's factor.
 __device__ __forceinline__ double4 pair_far(const StepParams &P, bool tab, const DevPair &d) {
-    if (tab || (d.flags & PF_EFPOT)) return make_double4(d.sc3, 0.0, d.fct, d.dm2hi);
+    if (tab || (d.flags & PF_EFPOT)) return make_double4(d.sc3, tab ? 6.0 * d.sc3 : 0.0, d.fct, d.dm2hi);
     const double s6 = (d.flags & PF_LJ) ? pow3(d.sgp2) : 0.0;
     return make_double4(-d.epp4 * s6, d.epp4 * (s6 * s6), (d.flags & PF_CHR) ? d.fct : 0.0,
                         (d.flags & PF_SRPMF) ? P.rth : -1.0);
@@ -442,11 +443,12 @@ __device__ __forceinline__ void pair_sums(const StepParams &P, const DevPair *s_
                         recip_pair(d2, ri, i2);
                     }
                     const double i6 = i2 * i2 * i2, c = fa.x * i6, q = fa.z * ri;
-                    double f = 6.0 * c + q;
-                    double b = 0.0;
-                    if constexpr (!TAB) {
+                    double f, b = 0.0;
+                    if constexpr (TAB) {
+                        f = fma(fa.y, i6, q);
+                    } else {
                         b = fa.y * (i6 * i6);
-                        f = fma(12.0, b, f);
+                        f = fma(12.0, b, 6.0 * c + q);
                     }
                     f = on && !near ? f * i2 : 0.0;
                     if constexpr (EN) {
@@ -606,8 +608,7 @@ void k_step(StepParams P) {
     constexpr int NB = NW * WAVE;   // threads of the block
     constexpr bool TAB = (FEAT & F_TAB) != 0;
     __shared__ DevPair s_row[MAX_LDS_TYPES];   // pair parameters by partner type
-    // by partner type: the far form's r^-6, r^-12 and 1/r factors, range^2 (< 0: none)
-    __shared__ double4 s_far[MAX_LDS_TYPES];
+    __shared__ double4 s_far[MAX_LDS_TYPES];   // its far form (pair_far)
     __shared__ double s_red[NW][7];
     __shared__ double s_mv[6];   // Gaussians and factors of the update
 
@@ -673,14 +674,7 @@ void k_step(StepParams P) {
         for (int k = tid; k < nt1; k += NB) {
             const DevPair d = P.rows[row + k];
             s_row[k] = d;
-            if (TAB || (d.flags & PF_EFPOT)) {
-                s_far[k] = make_double4(d.sc3, 0.0, d.fct, d.dm2hi);
-            } else {   // LJ 4 eps (s^12 - s^6) and the Coulomb term
-                const double s6 = (d.flags & PF_LJ) ? pow3(d.sgp2) : 0.0;
-                s_far[k] = make_double4(-d.epp4 * s6, d.epp4 * (s6 * s6),
-                                           (d.flags & PF_CHR) ? d.fct : 0.0,
-                                           (d.flags & PF_SRPMF) ? P.rth : -1.0);
-            }
+            s_far[k] = pair_far(P, TAB, d);
         }
     }
     // the grid corners of this wavefront's target: static field, trilinear repulsion map
@@ -774,11 +768,12 @@ void k_step(StepParams P) {
                             recip_pair(d2, ri, i2);
                         }
                         const double i6 = i2 * i2 * i2, c = fa.x * i6, q = fa.z * ri;
-                        double f = 6.0 * c + q;
-                        double b = 0.0;
-                        if constexpr (!TAB) {
+                        double f, b = 0.0;
+                        if constexpr (TAB) {
+                            f = fma(fa.y, i6, q);
+                        } else {
                             b = fa.y * (i6 * i6);
-                            f = fma(12.0, b, f);
+                            f = fma(12.0, b, 6.0 * c + q);
                         }
                         f = on && !near ? f * i2 : 0.0;
                         if constexpr (EN) {
