@@ -2358,7 +2358,7 @@ struct AdjRun {
 
     StepParams step_params(int s) {
         StepParams p = params_for(c);
-        // one fixed launch shape (two targets per workgroup), not the autotuner's timed
+        // one fixed launch shape (k_step_wave, a target a wavefront), not the autotuner's timed
         // pick: every pass, and every context of the same system, replays the trajectory
         // bitwise
         p.tpb = 2;

@@ -21,15 +21,14 @@ namespace bromoc {
 // only at site 1 (j.eq.1) and later sites replace it only when strictly smaller, so when
 // site 1 is outside its table range the record stays zero unless some site gives a
 // negative dist - dmi.
-template <int T, int NW>
-__device__ inline void prox_record(const StepParams &P, int i, const double4 &pa, int a,
-                                   const double (*s_pxd)[T], const int (*s_pxj)[T],
-                                   const DevPair *row, double dids[5]) {
+template <int NW>
+__device__ inline void prox_record(const StepParams &P, int i, const double4 &pa, const double *s_pxd,
+                                   const int *s_pxj, const DevPair *row, double dids[5]) {
     double d = INFINITY;
     int jj = 0x7fffffff;
     for (int q = 0; q < NW; q++) {
-        const double od = s_pxd[q][a];
-        const int oj = s_pxj[q][a];
+        const double od = s_pxd[q];
+        const int oj = s_pxj[q];
         if (od < d || (od == d && oj < jj)) { d = od; jj = oj; }
     }
     if (jj == 0x7fffffff) return;
@@ -592,7 +591,7 @@ __global__ __launch_bounds__(BLOCK) void k_step_wave(StepParams P) {
 // writes no energies (the step loop) the block computes its site target's CG-DNA list terms
 // itself (dna_site_terms); otherwise the site targets read them from k_dna (fdna).  The pair
 // loop is pair_sums' with one target and the block's registers in mind (five wavefronts a
-// SIMD; three with analytic pairs, which spill 47 to 110 registers at four and none at three:
+// SIMD; three with analytic pairs, which spill 47 to 110 registers at four and 0 to 18 at three:
 // 2500 particles with DNA and some analytic pair types 41 -> 32 us a step, 36 with a branch a
 // pair before, 40 with two wavefronts): what the end needs is parked in LDS.  DYNAMICS3 looks for
 // an ion's nearest site among the pairs in range as they are worked off (in the pair loop 31 us at
@@ -644,8 +643,7 @@ void k_step(StepParams P) {
     double4 p_me = make_double4(0.0, 0.0, 0.0, 0.0);
     double g_me[3] = {0.0, 0.0, 0.0};
     if (mine) {
-        const int w = wbase;
-        i_me = w < ns ? w : w + nf;
+        i_me = wbase < ns ? wbase : wbase + nf;
         site_me = i_me < ns;
         p_me = P.pos[i_me];
         free_me = !site_me || ((FEAT & F_DNA) && P.stfree[i_me] != 0);
@@ -659,23 +657,16 @@ void k_step(StepParams P) {
         }
     }
 
-    int ti;
-    bool tsite;
-    double tx, ty, tz;
-    {
-        const int w = wbase;
-            const int i = w < ns ? w : w + nf;
-        ti = i;
-        tsite = i < ns;
-        const double4 pa = P.pos[i];
-        tx = pa.x; ty = pa.y; tz = pa.z;
-        // pair rows of this block's targets
-        const int row = __double2loint(pa.w) * nt1;
-        for (int k = tid; k < nt1; k += NB) {
-            const DevPair d = P.rows[row + k];
-            s_row[k] = d;
-            s_far[k] = pair_far(P, TAB, d);
-        }
+    // the block's target and its pair rows
+    const int ti = wbase < ns ? wbase : wbase + nf;
+    const bool tsite = ti < ns;
+    const double4 pa = P.pos[ti];
+    const double tx = pa.x, ty = pa.y, tz = pa.z;
+    const int row0 = __double2loint(pa.w) * nt1;
+    for (int k = tid; k < nt1; k += NB) {
+        const DevPair d = P.rows[row0 + k];
+        s_row[k] = d;
+        s_far[k] = pair_far(P, TAB, d);
     }
     // the grid corners of this wavefront's target: static field, trilinear repulsion map
     float ph_x = 0.0f;
@@ -722,13 +713,11 @@ void k_step(StepParams P) {
     }
     __syncthreads();
 
-    double fx, fy, fz, et, eel, evd, esr;
-    fx = fy = fz = et = eel = evd = esr = 0.0;
+    double fx = 0.0, fy = 0.0, fz = 0.0, et = 0.0, eel = 0.0, evd = 0.0, esr = 0.0;
     // PROXDIFF: per target ion, the tabulated site partner within its table range of least
     // dist - dmi, ties to the lower site index (energy.mono.f90:603-620 in site order)
-    double pxd;
-    int pxj;
-    { pxd = INFINITY; pxj = 0x7fffffff; }
+    double pxd = INFINITY;
+    int pxj = 0x7fffffff;
 
     // ---- pair loop (energy.mono.f90:117-194, 584-687), compiled twice: with the energy
     // sums, and without them for the steps that write no energies
@@ -736,8 +725,7 @@ void k_step(StepParams P) {
     auto pair_loop = [&](auto en) {
         constexpr bool EN = decltype(en)::value;
         for (int base = tid; base < ntot; base += 32 * NB) {
-            uint32_t m;
-            m = 0u;
+            uint32_t m = 0u;
             const int cnt = min(32, (ntot - base + NB - 1) / NB);
 #pragma unroll 1
             for (int k0 = 0; k0 < cnt; k0 += PU) {
@@ -754,80 +742,76 @@ void k_step(StepParams P) {
                     const bool jok = base + (k0 + u) * NB < ntot;
                     const int t2j = __double2loint(pj.w);
                     const int j = __double2hiint(pj.w);
-                    {
-                        const bool on = jok && j != ti && !(tsite && j < ns);
-                        const double4 fa = s_far[t2j];
-                        const double dx = tx - pj.x, dy = ty - pj.y, dz = tz - pj.z;
-                        const double d2 = on ? pair_d2(dx, dy, dz) : 1e30;
-                        const bool near = on && d2 <= fa.w;
-                        double ri, i2;
-                        if constexpr (TAB) {
-                            ri = rsqrt_s26(d2);
-                            i2 = ri * ri;
-                        } else {
-                            recip_pair(d2, ri, i2);
-                        }
-                        const double i6 = i2 * i2 * i2, c = fa.x * i6, q = fa.z * ri;
-                        double f, b = 0.0;
-                        if constexpr (TAB) {
-                            f = fma(fa.y, i6, q);
-                        } else {
-                            b = fa.y * (i6 * i6);
-                            f = fma(12.0, b, 6.0 * c + q);
-                        }
-                        f = on && !near ? f * i2 : 0.0;
-                        if constexpr (EN) {
-                            // a pair's energy is counted once: by the site of a site-ion pair,
-                            // by the higher-index ion of an ion-ion pair
-                            const bool ce = on && !near && (tsite || (j >= ns && j < ti));
-                            const int fl = TAB ? (int)PF_EFPOT : s_row[t2j].flags;
-                            et += ce && (fl & PF_EFPOT) ? c + q : 0.0;
-                            if constexpr (!TAB) {
-                                eel += ce && (fl & (PF_EFPOT | PF_CHR)) == PF_CHR ? q : 0.0;
-                                evd += ce && (fl & (PF_EFPOT | PF_LJ)) == PF_LJ ? b + c : 0.0;
-                            }
-                        }
-                        m |= near ? 1u << (k0 + u) : 0u;
-                        fx = fma(f, dx, fx);
-                        fy = fma(f, dy, fy);
-                        fz = fma(f, dz, fz);
-                    }
-                }
-            }
-            {
-                while (m) {   // the pairs in range
-                    const int k = __ffs(m) - 1;
-                    m &= m - 1u;
-                    const double4 pj = P.spos[base + k * NB];
-                    const int j = __double2hiint(pj.w);
-                    const DevPair &row = s_row[__double2loint(pj.w)];
+                    const bool on = jok && j != ti && !(tsite && j < ns);
+                    const double4 fa = s_far[t2j];
                     const double dx = tx - pj.x, dy = ty - pj.y, dz = tz - pj.z;
-                    const double d2 = pair_d2(dx, dy, dz);
-                    const bool ce = tsite || (j >= ns && j < ti);
-                    double f;
-                    if (TAB || (row.flags & PF_EFPOT)) {
-                        double y;
-                        f = pair_table(row, P.ep, P.ires, d2, rsqrt_s26(d2), y);
-                        if constexpr (EN) et += ce ? y : 0.0;
-                        if constexpr ((FEAT & F_PROX) != 0) {
-                            if (!tsite && j < ns && !(d2 < row.dm2lo)) {
-                                const double dd = sqrt(d2) - row.dmi;
-                                if (dd < pxd || (dd == pxd && j < pxj)) { pxd = dd; pxj = j; }
-                            }
-                        }
+                    const double d2 = on ? pair_d2(dx, dy, dz) : 1e30;
+                    const bool near = on && d2 <= fa.w;
+                    double ri, i2;
+                    if constexpr (TAB) {
+                        ri = rsqrt_s26(d2);
+                        i2 = ri * ri;
                     } else {
-                        double q0 = 0.0, q1 = 0.0, q2 = 0.0;
-                        f = pair_analytic(row, P, d2, q0, q1, q2);
-                        if constexpr (EN) {
-                            eel += ce ? q0 : 0.0;
-                            evd += ce ? q1 : 0.0;
-                            esr += ce ? q2 : 0.0;
+                        recip_pair(d2, ri, i2);
+                    }
+                    const double i6 = i2 * i2 * i2, c = fa.x * i6, q = fa.z * ri;
+                    double f, b = 0.0;
+                    if constexpr (TAB) {
+                        f = fma(fa.y, i6, q);
+                    } else {
+                        b = fa.y * (i6 * i6);
+                        f = fma(12.0, b, 6.0 * c + q);
+                    }
+                    f = on && !near ? f * i2 : 0.0;
+                    if constexpr (EN) {
+                        // a pair's energy is counted once: by the site of a site-ion pair,
+                        // by the higher-index ion of an ion-ion pair
+                        const bool ce = on && !near && (tsite || (j >= ns && j < ti));
+                        const int fl = TAB ? (int)PF_EFPOT : s_row[t2j].flags;
+                        et += ce && (fl & PF_EFPOT) ? c + q : 0.0;
+                        if constexpr (!TAB) {
+                            eel += ce && (fl & (PF_EFPOT | PF_CHR)) == PF_CHR ? q : 0.0;
+                            evd += ce && (fl & (PF_EFPOT | PF_LJ)) == PF_LJ ? b + c : 0.0;
                         }
                     }
+                    m |= near ? 1u << (k0 + u) : 0u;
                     fx = fma(f, dx, fx);
                     fy = fma(f, dy, fy);
                     fz = fma(f, dz, fz);
                 }
+            }
+            while (m) {   // the pairs in range
+                const int k = __ffs(m) - 1;
+                m &= m - 1u;
+                const double4 pj = P.spos[base + k * NB];
+                const int j = __double2hiint(pj.w);
+                const DevPair &row = s_row[__double2loint(pj.w)];
+                const double dx = tx - pj.x, dy = ty - pj.y, dz = tz - pj.z;
+                const double d2 = pair_d2(dx, dy, dz);
+                const bool ce = tsite || (j >= ns && j < ti);
+                double f;
+                if (TAB || (row.flags & PF_EFPOT)) {
+                    double y;
+                    f = pair_table(row, P.ep, P.ires, d2, rsqrt_s26(d2), y);
+                    if constexpr (EN) et += ce ? y : 0.0;
+                    if constexpr ((FEAT & F_PROX) != 0) {
+                        if (!tsite && j < ns && !(d2 < row.dm2lo)) {
+                            const double dd = sqrt(d2) - row.dmi;
+                            if (dd < pxd || (dd == pxd && j < pxj)) { pxd = dd; pxj = j; }
+                        }
+                    }
+                } else {
+                    double q0 = 0.0, q1 = 0.0, q2 = 0.0;
+                    f = pair_analytic(row, P, d2, q0, q1, q2);
+                    if constexpr (EN) {
+                        eel += ce ? q0 : 0.0;
+                        evd += ce ? q1 : 0.0;
+                        esr += ce ? q2 : 0.0;
+                    }
+                }
+                fx = fma(f, dx, fx);
+                fy = fma(f, dy, fy);
+                fz = fma(f, dz, fz);
             }
         }
     };
@@ -835,20 +819,16 @@ void k_step(StepParams P) {
         if (P.write_energy) pair_loop(std::true_type{});
         else pair_loop(std::false_type{});
     }
-    __shared__ double s_pxd[(FEAT & F_PROX) ? NW : 1][1];
-    __shared__ int s_pxj[(FEAT & F_PROX) ? NW : 1][1];
+    __shared__ double s_pxd[(FEAT & F_PROX) ? NW : 1];
+    __shared__ int s_pxj[(FEAT & F_PROX) ? NW : 1];
     if constexpr ((FEAT & F_PROX) != 0) {
-        {
-            double d = pxd;
-            int jj = pxj;
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const double od = __shfl_xor(d, off, WAVE);
-                const int oj = __shfl_xor(jj, off, WAVE);
-                if (od < d || (od == d && oj < jj)) { d = od; jj = oj; }
-            }
-            if (lane == 0) { s_pxd[wv][0] = d; s_pxj[wv][0] = jj; }
+        for (int off = 32; off > 0; off >>= 1) {
+            const double od = __shfl_xor(pxd, off, WAVE);
+            const int oj = __shfl_xor(pxj, off, WAVE);
+            if (od < pxd || (od == pxd && oj < pxj)) { pxd = od; pxj = oj; }
         }
+        if (lane == 0) { s_pxd[wv] = pxd; s_pxj[wv] = pxj; }
     }
 
     // forces that other kernels computed, before the sums
@@ -974,7 +954,7 @@ void k_step(StepParams P) {
         }
         double dids[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
         if constexpr ((FEAT & F_PROX) != 0) {
-            if (!site_me) prox_record<1, NW>(P, i, p_me, 0, s_pxd, s_pxj, s_row, dids);
+            if (!site_me) prox_record<NW>(P, i, p_me, s_pxd, s_pxj, s_row, dids);
         }
         const double g[3] = {s_mv[0], s_mv[1], s_mv[2]};
         const MoveFac m = {s_mv[3], s_mv[4], s_mv[5]};
