@@ -5,7 +5,7 @@
 // has its own static field and GCMC buffers.  One BD step of all replicas is one launch of
 // k_batch_step: its wavefronts take (replica, slot) work items -- a fixed table ordered by
 // replica size, largest first; a slot beyond the replica's present count is passed over --
-// from a device queue (or one item each in the non-persistent shape), gather the ion's pair
+// one each (from a device queue where BROMOC_BATCH_BLOCKS asks for it), gather the ion's pair
 // forces over its own replica's particles (all pairs, as energy.mono.f90:117-194), its grid
 // corners, and apply DYNAMICS0/1/2.  k_batch_noise draws the Gaussians of several steps at
 // once.  k_batch_gcmc runs

@@ -2,8 +2,8 @@
 reference routines and closed forms in test_oracle_analytic.py): Coulomb, 12-6 LJ and SRPMF
 pair types without EFPOT tables (energy.mono.f90:135-178,623-668; interact.f90:182-204,
 365-404), all-analytic and mixed with tabulated types, ion-ion and site-ion, through every
-launch shape of the step kernels (BROMOC_TPB 1, 2, 4 targets per block; 8, one target per
-wavefront), in BD trajectories (5 steps launched directly, 40 steps replayed from captured
+launch shape of the step kernels (BROMOC_TPB 1: a block per target; 2, 4: one, two targets
+a wavefront; 8: a wavefront per target, partners through LDS), in BD trajectories (5 steps launched directly, 40 steps replayed from captured
 graphs), in INTERACT and GRAND, and in replica batches (the batch step kernel's analytic
 path and its device GRAND).
 

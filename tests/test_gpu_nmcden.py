@@ -1,7 +1,7 @@
 """Per-species repulsion maps (NMCDEN: vdwgd1trln.f90:61-80, vdwgd1spln.f90:61-80,
 vdwgd0trln.f90:56-75, vdwgd0spln.f90:58-77) on the HIP path against the C oracle, through
-every launch shape of the step kernels (BROMOC_TPB 1, 2, 4 targets per block and the
-one-target-per-wavefront kernel, 8).
+every launch shape of the step kernels (BROMOC_TPB 1: a block per target; 2, 4: one, two
+targets a wavefront; 8: a wavefront per target, partners through LDS).
 
 Bar as the other parity tests: energies and norm-wise forces 1e-10 relative, positions
 after BD steps 1e-9 A (1e-8 after 40 graph-replayed steps), INTERACT 1e-10 relative.
