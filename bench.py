@@ -35,10 +35,11 @@ FP64_PEAK_TFLOPS = 78.6
 # the same counters read for a 256 MiB device copy (bench.py --copy-probe 256): FETCH_SIZE
 # x 2.0, WRITE_SIZE x 1.0.  The counters cannot be read from inside this process; a shape
 # without a measurement reports null.
-TRAFFIC_KIB = {("translocation", 18): (192662.1, 667574.8), ("pore_dna", 1): (4327.2, 1389.2)}
+TRAFFIC_KIB = {("translocation", 18): (192662.1, 667574.8), ("translocation", 20): (410465.2, 740473.4),
+               ("pore_dna", 1): (4327.2, 1389.2)}
 # L2 hit rate of the same launches, TCC_HIT_sum / (TCC_HIT_sum + TCC_MISS_sum) from the
 # WRITE_SIZE run's two L2 counters
-L2_HIT = {("translocation", 18): 0.858, ("pore_dna", 1): 0.925}
+L2_HIT = {("translocation", 18): 0.858, ("translocation", 20): 0.764, ("pore_dna", 1): 0.925}
 TRAFFIC_SCALE = (2.0, 1.0)
 # FP64 operations per pair evaluation: a table pair ~34 (r^2 8, sqrt 1, index 2, U 4, F/r 3,
 # energy 1, force update on both particles ~15); the reaction-field cross term of an ion

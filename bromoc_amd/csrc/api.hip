@@ -1202,10 +1202,9 @@ static hipError_t enqueue_step(bromoc_ctx *c, const StepParams &p, hipEvent_t t0
 // with 1, 2 or 4 targets per lane (17, 18, 20) -- chosen by timing ENERGY-only launches
 // (warnings go to a scratch counter) on the ctx's stream: the reaction-field kernels the shape
 // needs, the CG-DNA kernel and its pair kernels.  A first round of two launches a shape drops
-// those that take three times the best, sixty-fold losers among them (timed to the end like
-// the others they were most of the tuning: 25 -> 5.3 ms for 1531 analytic ions, 8.8 -> 4.0 for
-// 2300 particles with DNA, 0.81 -> 0.35 s for 56,000).  The environment variable BROMOC_TPB
-// forces a value.
+// those that take twice the best, sixty-fold losers among them (timed to the end like the others
+// they were most of the tuning: 25 -> 5.8 ms for 1531 analytic ions, 8.8 -> 4.2 for 2300 particles
+// with DNA, 0.81 -> 0.30 s for 56,000).  The environment variable BROMOC_TPB forces a value.
 static int autotune(bromoc_ctx *c) {
     if (c->tpb > 0) return BROMOC_OK;
     if (const char *env = std::getenv("BROMOC_TPB")) {
@@ -1235,12 +1234,12 @@ static int autotune(bromoc_ctx *c) {
     hipEvent_t e0, e1;
     HIPCHK(c, hipEventCreate(&e0));
     HIPCHK(c, hipEventCreate(&e1));
-    // then two interleaved rounds of five launches per shape left; each keeps its best round
+    // then three interleaved rounds of five launches per shape left; each keeps its best round
     // (shapes within a few per cent of each other are told apart reliably this way)
     double bt = 1e300;
-    for (int round = 0; round < 3; round++) {
+    for (int round = 0; round < 4; round++) {
         const int reps = round == 0 ? 2 : 5;
-        const double limit = 3.0 * bt;
+        const double limit = 2.0 * bt;
         for (int q = 0; q < nc; q++) {
             if (round > 0 && best[q] > limit) continue;
             c->tpb = cand[q];

@@ -59,7 +59,7 @@ def test_analytic_pairs(n, tpb, monkeypatch):
 
 def test_tuning_drops_losers():
     """Analytic ions, where the slowest shape takes sixty times the fastest: the tuning takes
-    the time of 340 steps when slow shapes are dropped after a first round, of 1600 when every
+    the time of 330 to 400 steps when slow shapes are dropped after a first round, of 1600 when every
     shape is timed to the end."""
     n = 1531
     s = configs.with_analytic(_first(_ions(n), n), seed=n)
