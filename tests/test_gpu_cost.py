@@ -1,7 +1,7 @@
 """Options cost about what their work does: times of steps against those of the same system
 without the option, in one launch shape, so that a variant that spills its registers or takes
 a general path for ordinary pairs is seen.  Bounds lie between the ratio a sound variant shows
-and that of one with such a fault (in the comments), some 15 % from either.
+and that of one with such a fault (in the comments), 7 % or more from either.
 """
 import time
 
@@ -46,14 +46,14 @@ def test_analytic_pair_types_beside_tables(monkeypatch):
     a = _times(s, 1, monkeypatch)[0]
     b = _times(configs.with_analytic(s, types=[1, 4, 9], seed=3), 1, monkeypatch)[0]
     print(f"tables {1e6 * a:.1f} us, some analytic {1e6 * b:.1f} us: {b / a:.2f}")
-    assert b <= 1.55 * a           # 1.38; 1.72 with 80 spilled registers
+    assert b <= 1.6 * a            # 1.38; 1.72 with 80 spilled registers
 
 
 def test_reaction_field_with_zero_cells(monkeypatch):
     a = _times(_rf(_ions()), 17, monkeypatch)[0]
     b = _times(_rf(_ions(), zero_frac=0.05, wall_radius=60.0), 17, monkeypatch)[0]
     print(f"smooth {1e6 * a:.1f} us, zero cells {1e6 * b:.1f} us: {b / a:.2f}")
-    assert b <= 1.57 * a           # 1.39; 1.75 with the pair forces in the masked sweep
+    assert b <= 1.6 * a            # 1.39; 1.75 with the pair forces in the masked sweep
 
 
 @pytest.mark.parametrize("nfix", [0, 4000])
@@ -68,4 +68,4 @@ def test_fixed_ions(monkeypatch):
     a = _times(_ions(), 17, monkeypatch)[0]
     b = _times(with_fixed(_ions(), 4000), 17, monkeypatch)[0]
     print(f"none fixed {1e6 * a:.1f} us, a third {1e6 * b:.1f} us: {b / a:.2f}")
-    assert b <= 1.1 * a            # 0.96; 1.20 with the pair forces in the masked sweep
+    assert b <= 1.13 * a           # 0.96; 1.20 with the pair forces in the masked sweep
